@@ -44,7 +44,9 @@ extern "C" {
  * reference's multi-block and last-table kernels,
  * X-TED_GPU/parallel_X_TED.cu:883-1131); 33, 34, 35 = tables of at most 16,
  * 32 or 64 columns, four, two or one to a wave (the role of the reference's
- * single-thread tasks, X-TED_GPU/parallel_X_TED.cu:382). */
+ * single-thread tasks, X-TED_GPU/parallel_X_TED.cu:382); 36, 37, 38 = on-chip
+ * tables of deep column keyroots, 4, 8 or 16 waves of 8 columns per lane that
+ * share their slot rows (never forced). */
 #define XTED_CLASS_AUTO (-1)
 #define XTED_CLASS_LANE 0
 

@@ -108,16 +108,16 @@ struct PoolView {
   const TreeMeta* trees;
 };
 
-// A table task: pair id (24 bits) | x keyroot node (20 bits) | y keyroot node (20 bits).
-// Trees in a pool are limited to 2^20 nodes and a batch to 2^24 pairs.
-constexpr int kTaskNodeBits = 20;
+// A table task: pair id (24 bits) | x keyroot node (20 bits) | 1 when the rows
+// are x's nodes | y keyroot node (19 bits). Trees of a pool have at most
+// 32,767 nodes and a batch at most 2^24 pairs.
 constexpr int kTaskPairBits = 24;
-XTED_HD inline uint64_t task_pack(uint32_t pair, uint32_t i0, uint32_t j0) {
-  return ((uint64_t)pair << 40) | ((uint64_t)i0 << 20) | (uint64_t)j0;
+XTED_HD inline uint64_t task_pack(uint32_t pair, uint32_t i0, uint32_t j0, bool rows_x) {
+  return ((uint64_t)pair << 40) | ((uint64_t)i0 << 20) | ((uint64_t)rows_x << 19) | (uint64_t)j0;
 }
 XTED_HD inline uint32_t task_pair(uint64_t t) { return (uint32_t)(t >> 40); }
 XTED_HD inline uint32_t task_i0(uint64_t t) { return (uint32_t)(t >> 20) & 0xFFFFFu; }
-XTED_HD inline uint32_t task_j0(uint64_t t) { return (uint32_t)t & 0xFFFFFu; }
+XTED_HD inline uint32_t task_j0(uint64_t t) { return (uint32_t)t & 0x7FFFFu; }
 
 // ---- granularity classes ----------------------------------------------------
 // Class 0: leaf (a table whose short side is one node, a leaf keyroot),
@@ -130,6 +130,9 @@ XTED_HD inline uint32_t task_j0(uint64_t t) { return (uint32_t)t & 0xFFFFFu; }
 //   chained per row through device memory, class = 27 + k.
 // Classes 33..35: tiny tables of at most 16, 32 or 64 columns, one per 16-,
 //   32- or 64-lane segment of a wave (four, two or one to a wave).
+// Classes 36..38: on-chip tables of deep column keyroots, whose waves' imports
+//   do not fit LDS beside the slot rows: slot rows shared by 4, 8 or 16 waves,
+//   with a barrier per row.
 constexpr int kClassLane = 0;  // the leaf class
 constexpr int kNumRowClasses = 25;
 constexpr int kClassXL = 26;
@@ -137,8 +140,13 @@ constexpr int kFirstXLClass = 27;
 constexpr int kNumXLForms = 6;
 constexpr int kClassTiny = kFirstXLClass + kNumXLForms;  // 33: the first tiny form
 constexpr int kNumTinyForms = 3;
-constexpr int kNumClasses = kClassTiny + kNumTinyForms;  // 36
-XTED_HD inline bool is_tiny(int cls) { return cls >= kClassTiny && cls < kNumClasses; }
+constexpr int kClassShared = kClassTiny + kNumTinyForms;  // 36: the first shared-slot form
+constexpr int kNumSharedForms = 3;
+constexpr int kNumClasses = kClassShared + kNumSharedForms;  // 39
+XTED_HD inline bool is_tiny(int cls) { return cls >= kClassTiny && cls < kClassShared; }
+XTED_HD inline bool is_shared(int cls) { return cls >= kClassShared && cls < kNumClasses; }
+// Shared-slot form k: 4, 8 or 16 waves of 8 columns per lane.
+XTED_HD inline int shared_cols(int k) { return 64 * 8 * (4 << k); }
 // Lanes per table (and most columns) of tiny form k.
 XTED_HD inline int tiny_seg(int k) { return 16 << k; }
 // Slot bytes of one table of tiny form k: 32 KiB per workgroup of 256 lanes.
@@ -224,7 +232,32 @@ struct ClassRule {
   // blocks, 1: 2048, 2: 1024, ...): narrower blocks put more workgroups on
   // one table.
   int32_t xl_first = 0;
+  // Tables of at least tall_rows rows and more than kTallCols columns take at
+  // most tall_cpl columns per lane (set_tall).
+  int32_t tall_rows = 1 << 30;
+  int32_t tall_cpl = 16;
 };
+// A row of up to 256 columns takes one wave about as long as several
+// (a 120-node pair's root table 0.21 us a row either way).
+constexpr int32_t kTallCols = 256;
+
+// How tall tables are split, by the interior cells of the whole plan. A plan
+// of few cells waits for its largest tables, one after another along the
+// levels, and a row of a table takes the less the fewer columns a lane holds
+// (1000 columns: 0.38 us with 16, 0.32 with 8, 0.24 with 4, 0.21 with 2); a
+// plan of many fills the device, and more waves per table only add their rows'
+// fixed instructions. Measured, ms, without the rule and with tall_rows 64 and
+// 4 or 2 columns: a deep 1000-node pair (2.6e8 cells) 11.3, 8.4, 7.7; 128
+// pairs of 100-600 nodes (9.6e8) 23.5, 20.8, 20.2; 1024 pairs of 100-1000
+// nodes under a cost model (3.7e10) 67, 55, 61; 4096 such pairs with unit costs
+// (1.4e11) 93, 111, 143.
+constexpr int64_t kTall2Cells = 4000000000ll;
+constexpr int64_t kTall4Cells = 80000000000ll;
+XTED_HD inline void set_tall(ClassRule& rule, int64_t cells) {
+  if (cells > kTall4Cells) return;
+  rule.tall_rows = 64;
+  rule.tall_cpl = cells <= kTall2Cells ? 2 : 4;
+}
 
 XTED_HD inline int ilog2_ceil(int v) {
   int r = 0;
@@ -240,19 +273,59 @@ XTED_HD inline int64_t xl_lds_need(int kd_r, int kd_c, int leaves_c, int bw) {
   return (int64_t)(kd_r > 1 ? kd_r : 1) * (own + 3 + kd_c) * 2;
 }
 
-// Class of table (a x b): lds_need is the slot storage of its oriented
-// on-chip form; kd_r / kd_c / leaves_c (row keyroot height, column keyroot
-// height and leaves) size the column-blocked forms. Single-row tables are
+// On-chip row scan of w waves: entries of the ring between two waves, and the
+// LDS bytes of a table whose row keyroot has nesting height slots (at least 1)
+// and whose column keyroot has leaves_c leaves and nesting height kd_c: one
+// uint16 row per slot with every far column (the leaves but the last), and
+// per wave the boundary entry, a sink and, with several waves, the kd_c + 1
+// values imported from earlier blocks; and w + 1 rings of a carry, the
+// imports and a trash word per entry, and w + 2 progress words.
+constexpr int kEdgeRows = 8;
+XTED_HD inline int64_t scan_lds_need(int slots, int leaves_c, int kd_c, int w) {
+  if (w == 1) return (int64_t)slots * (leaves_c + 1) * 2;
+  return (int64_t)slots * (leaves_c - 1 + w * (kd_c + 3)) * 2 +
+         (int64_t)(w + 1) * kEdgeRows * (kd_c + 3) * 4 + 8 * (w + 2);
+}
+
+// Class of table (a x b): kd_r / kd_c / leaves_c (row keyroot height, column
+// keyroot height and leaves) of its oriented form size its LDS storage. Single-row tables are
 // the leaf class when leaf_form is set. *need receives the slot bytes of the
 // chosen form.
-XTED_HD inline int table_class(int a, int b, int64_t lds_need, int kd_r, int kd_c, int leaves_c,
-                               bool leaf_form, const ClassRule& rule, int64_t* need) {
+XTED_HD inline int table_class(int a, int b, int kd_r, int kd_c, int leaves_c, bool leaf_form,
+                               const ClassRule& rule, int64_t* need) {
   const int rows = a <= b ? a : b;
   const int cols = a <= b ? b : a;
+  const int slots = kd_r > 1 ? kd_r : 1;
+  const int64_t lds_need = scan_lds_need(slots, leaves_c, kd_c, 1);
   *need = lds_need;
   if (rows == 1 && leaf_form) return kClassLane;
+  for (int k = 0; k < kNumTinyForms; ++k)
+    if ((rule.tiny >> k & 1) && cols <= tiny_seg(k) && lds_need <= tiny_max_lds(k))
+      return kClassTiny + k;
   const int cpl_cap = rule.max_cpl < 8 ? rule.max_cpl : 8;
-  if (cols > 64 * cpl_cap * kMaxRowWaves || lds_need > rule.lds_max) {
+  int wi = 0;
+  while (wi < 4 && lds_need > (int64_t)rule.lds_per_wave * (1 << wi)) ++wi;
+  while (wi < 4 && cols > 64 * rule.max_cpl * (1 << wi)) ++wi;
+  if (rows >= rule.tall_rows && cols > kTallCols) {
+    while (wi < 4 && cols > 64 * rule.tall_cpl * (1 << wi)) ++wi;
+  }
+  if (cols >= rule.wide_cols) {
+    while (wi < 4 && (1 << wi) < rule.min_waves) ++wi;
+  }
+  // More waves hold more imports: no more than fit (up to 16 columns a lane).
+  while (wi > 0 && scan_lds_need(slots, leaves_c, kd_c, 1 << wi) > rule.lds_max &&
+         cols <= 64 * 16 * (1 << (wi - 1)))
+    --wi;
+  *need = scan_lds_need(slots, leaves_c, kd_c, 1 << wi);
+  if (*need > rule.lds_max && lds_need <= rule.lds_max) {
+    for (int k = 0; k < kNumSharedForms; ++k) {
+      if (cols <= shared_cols(k)) {
+        *need = lds_need;
+        return kClassShared + k;
+      }
+    }
+  }
+  if (cols > 64 * cpl_cap * kMaxRowWaves || *need > rule.lds_max) {
     if (kd_c + 1 > kMaxImports) return kClassXL;
     // Short tables take the forms one workgroup sweeps.
     for (int k = rows <= rule.xl_seq_rows ? kFirstSeqXLForm : rule.xl_first; k < kNumXLForms;
@@ -264,15 +337,6 @@ XTED_HD inline int table_class(int a, int b, int64_t lds_need, int kd_r, int kd_
       }
     }
     return kClassXL;
-  }
-  for (int k = 0; k < kNumTinyForms; ++k)
-    if ((rule.tiny >> k & 1) && cols <= tiny_seg(k) && lds_need <= tiny_max_lds(k))
-      return kClassTiny + k;
-  int wi = 0;
-  while (wi < 4 && lds_need > (int64_t)rule.lds_per_wave * (1 << wi)) ++wi;
-  while (wi < 4 && cols > 64 * rule.max_cpl * (1 << wi)) ++wi;
-  if (cols >= rule.wide_cols) {
-    while (wi < 4 && (1 << wi) < rule.min_waves) ++wi;
   }
   int w = 1 << wi;
   int c = (cols + 64 * w - 1) / (64 * w);

@@ -91,7 +91,7 @@ void DevBuf::release() {
 // The no-allocation batch path's buffers, one array per device (each device
 // holds its own copy). Host code reaches it only through the address
 // hipGetSymbolAddress returns for the current device (Context::init).
-static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
+static __device__ __align__(256) unsigned char scratch[kNoAllocArray];
 
 Context::Context(int device) : device_(device) {}
 
@@ -597,9 +597,11 @@ int Context::plan(Group& g, int32_t npairs, const int32_t* xs, const int32_t* ys
   // SIMD): under a cost model a table gets more waves instead (the 4096-pair
   // batch under a cost model ran 125.5 ms against 131.3 with up to 16).
   if (cost_alphabet_ > 0) pa.rule.max_cpl = std::min(pa.rule.max_cpl, kMaxCostCpl);
+  if (g.maxn <= kMaxOnChipCols) set_tall(pa.rule, st.cells);
   pa.rule_tail = ClassRule{lds_limit, 1, 1 << 30, lds_limit, 16, rule.xl_seq_rows};
   pa.rule_tail.xl_first = rule.xl_first;
   pa.rule_tail.tiny = rule.tiny;
+  if (g.maxn <= kMaxOnChipCols) set_tall(pa.rule_tail, st.cells);
   pa.tail_level = g.tail_lv.as<uint8_t>();
   pa.force_class = force_class;
   pa.bands = size_bands;
@@ -738,7 +740,7 @@ int Context::launch_levels(Group* const* gs, int ng, std::vector<ProfLaunch>* pr
   // 101 ms per batch; among the rest, class order measured about 1% faster
   // than ordering by cells.)
   auto latency_bound = [](const Launch& l) {
-    return l.heavy || (l.cls >= row_class(2, 0) && l.cls <= kNumRowClasses);
+    return l.heavy || is_shared(l.cls) || (l.cls >= row_class(2, 0) && l.cls <= kNumRowClasses);
   };
   std::stable_sort(lv.begin(), lv.end(), [&](const Launch& x, const Launch& y) {
     return latency_bound(x) != latency_bound(y) ? latency_bound(x) : x.cls > y.cls;
@@ -837,8 +839,8 @@ int Context::finish_async(Group& g, int lane) {
   hipStream_t ls = lane_stream(lane);
   ST_TRY(reserve_pinned(g, g.npairs));
   if (!g.done_ev) HIP_TRY(hipEventCreateWithFlags(&g.done_ev, hipEventDisableTiming));
-  launch_gather_dist(g.pairs.as<PairMeta>(), g.td.as<td_t>(), g.npairs, g.dist.as<int32_t>(),
-                     ls);
+  launch_gather_dist(g.pairs.as<PairMeta>(), g.td.as<td_t>(), g.npairs,
+                     g.abort.as<int32_t>(), g.dist.as<int32_t>(), ls);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipMemcpyAsync(g.h_dist_pin, g.dist.p, sizeof(int32_t) * g.npairs,
                          hipMemcpyDeviceToHost, ls));
@@ -856,15 +858,17 @@ int Context::poll(Group& g, bool wait, int32_t* dist) {
   }
   HIP_TRY(e);
   std::copy(g.h_dist_pin, g.h_dist_pin + g.npairs, dist);
-  if (g.nxl > 0 && g.h_dist_pin[g.npairs]) return xl_timeout(g.h_dist_pin + g.npairs);
+  if (g.h_dist_pin[g.npairs]) return xl_timeout(g.h_dist_pin + g.npairs);
   return OK;
 }
 
-// The abort record of a column-blocked launch: {flag, claimed, ticket,
-// kind << 24 | row, word low, word high, epoch}.
+// The abort record of a group: {flag, claimed, ticket (or task), kind << 24 |
+// row, word low, word high, epoch}; kinds as below.
 int xl_timeout(const int32_t* rec) {
-  set_error("run_batch: a column-blocked table stopped waiting for its neighbour block (ticket " +
-            std::to_string(rec[2]) + ", " + ((rec[3] >> 24) ? "import" : "carry") + " of row " +
+  const char* const kinds[] = {"carry", "import", "wave"};
+  set_error("run_batch: a table stopped waiting for its neighbour block (ticket " +
+            std::to_string(rec[2]) + ", " + kinds[std::min(2, std::max(0, rec[3] >> 24))] +
+            " of row " +
             std::to_string(rec[3] & 0xFFFFFF) + ", read " + std::to_string((uint32_t)rec[5]) +
             ":" + std::to_string(rec[4]) + ", epoch " + std::to_string((uint32_t)rec[6]) + ")");
   return ERR_TIMEOUT;
@@ -923,7 +927,7 @@ std::vector<uint64_t> Context::graph_signature(const Group& g, int lane) const {
   s.push_back((uint64_t)g.npairs);
   s.push_back((uint64_t)g.nlevels);
   s.push_back((uint64_t)g.lines[g.npairs]);
-  for (const void* p : {g.pairs.p, g.td.p, g.tasks.p, g.descs.p, g.lines_d.p})
+  for (const void* p : {g.pairs.p, g.td.p, g.tasks.p, g.descs.p, g.lines_d.p, g.abort.p})
     s.push_back((uint64_t)(uintptr_t)p);
   const PoolView v = view();
   const uint64_t* pv = reinterpret_cast<const uint64_t*>(&v);
@@ -1025,8 +1029,8 @@ int Context::run_batch(int32_t npairs, const int32_t* xs, const int32_t* ys, int
     hipStream_t s = lane_stream(ng > 1 ? k : -1);
     gd[k].assign(g.npairs, 0);
     aborted[k].fill(0);
-    launch_gather_dist(g.pairs.as<PairMeta>(), g.td.as<td_t>(), g.npairs, g.dist.as<int32_t>(),
-                       s);
+    launch_gather_dist(g.pairs.as<PairMeta>(), g.td.as<td_t>(), g.npairs,
+                       g.abort.as<int32_t>(), g.dist.as<int32_t>(), s);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipMemcpyAsync(gd[k].data(), g.dist.p, sizeof(int32_t) * g.npairs,
                            hipMemcpyDeviceToHost, s));
@@ -1052,8 +1056,12 @@ int Context::run_batch(int32_t npairs, const int32_t* xs, const int32_t* ys, int
     }
   }
   for (int k = 0; k < ng; ++k) HIP_TRY(hipStreamSynchronize(lane_stream(ng > 1 ? k : -1)));
-  for (int k = 0; k < ng; ++k)
-    if (aborted[k][0]) return xl_timeout(aborted[k].data());
+  for (int k = 0; k < ng; ++k) {
+    if (gd[k][0] != kDistAborted) continue;
+    HIP_TRY(hipMemcpy(aborted[k].data(), batch_[k].abort.p, sizeof(int32_t) * kAbortInts,
+                      hipMemcpyDeviceToHost));
+    return xl_timeout(aborted[k].data());
+  }
   for (int k = 0; k < ng; ++k)
     for (size_t j = 0; j < idx[k].size(); ++j) dist[idx[k][j]] = gd[k][j];
 
@@ -1100,7 +1108,9 @@ int Context::run_batch(int32_t npairs, const int32_t* xs, const int32_t* ys, int
 
 // Bytes plan() carves for these pairs, every buffer rounded to 256 bytes as
 // the arena does (the column-blocked words, sized on the device, come on top).
-int64_t Context::noalloc_bytes(int32_t npairs, const int32_t* xs, const int32_t* ys) const {
+// classes: granularity classes the bucket counters are counted for.
+int64_t Context::noalloc_bytes(int32_t npairs, const int32_t* xs, const int32_t* ys,
+                               int32_t classes) const {
   auto r = [](int64_t b) { return (b + 255) & ~int64_t{255}; };
   int64_t td = 0, planned = 0;
   int32_t nlevels = 0;
@@ -1111,7 +1121,7 @@ int64_t Context::noalloc_bytes(int32_t npairs, const int32_t* xs, const int32_t*
     planned += (int64_t)(le ? a.K - a.K1 : a.K) * (le ? b.K - b.K1 : b.K);
     nlevels = std::max(nlevels, a.kdmax + b.kdmax + 1);
   }
-  const int64_t nb = (int64_t)nlevels * kNumClasses * kBands;
+  const int64_t nb = (int64_t)nlevels * classes * kBands;
   planned = std::max<int64_t>(planned, 1);
   return r(sizeof(PairMeta) * npairs) + r(nlevels) + 2 * r(8 * (int64_t)(npairs + 1)) +
          3 * r(8 * nb) + 2 * r(4 * nb) + r(32) + r(8 * planned) + r(64 * planned) +
@@ -1138,10 +1148,11 @@ int Context::run_batch_noalloc(int32_t npairs, const int32_t* xs, const int32_t*
       return ERR_NOT_FOUND;
     }
   }
-  const int64_t need = noalloc_bytes(npairs, xs, ys);
-  if (need > (int64_t)na_arena_.cap) {
+  const int64_t need = noalloc_bytes(npairs, xs, ys, kNoAllocClasses);
+  na_arena_.cap = kNoAllocBytes + (noalloc_bytes(npairs, xs, ys, kNumClasses) - need);
+  if (need > (int64_t)kNoAllocBytes) {
     set_error("batch_noalloc: the pairs need " + std::to_string(need) +
-              " bytes of device scratch; the array holds " + std::to_string(na_arena_.cap));
+              " bytes of device scratch; the array holds " + std::to_string(kNoAllocBytes));
     return ERR_TOO_LARGE;
   }
   HIP_TRY(hipSetDevice(device_));
@@ -1165,14 +1176,15 @@ int Context::run_batch_noalloc(int32_t npairs, const int32_t* xs, const int32_t*
   }
   hipStream_t s = lane_stream(-1);
   int32_t rec[kAbortInts] = {};
-  launch_gather_dist(na_.pairs.as<PairMeta>(), na_.td.as<td_t>(), npairs,
+  launch_gather_dist(na_.pairs.as<PairMeta>(), na_.td.as<td_t>(), npairs, na_.abort.as<int32_t>(),
                      na_.dist.as<int32_t>(), s);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipMemcpyAsync(dist, na_.dist.p, sizeof(int32_t) * npairs, hipMemcpyDeviceToHost, s));
-  if (na_.nxl > 0)
-    HIP_TRY(hipMemcpyAsync(rec, na_.abort.p, sizeof(rec), hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
-  if (rec[0]) return xl_timeout(rec);
+  if (dist[0] == kDistAborted) {
+    HIP_TRY(hipMemcpy(rec, na_.abort.p, sizeof(rec), hipMemcpyDeviceToHost));
+    return xl_timeout(rec);
+  }
   return OK;
 }
 

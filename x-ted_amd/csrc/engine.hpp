@@ -27,6 +27,12 @@ constexpr int kMaxLevelStreams = 4;
 // Device bytes of the fixed array the no-allocation batch path carves its
 // buffers from (one per device, held until the process ends).
 constexpr size_t kNoAllocBytes = size_t{64} << 20;
+// Which requests fit is decided with the plan's counters of the first
+// kNoAllocClasses granularity classes; the array holds those of the classes
+// after them on top (their share of the counters, which are less than all).
+constexpr int kNoAllocClasses = kClassShared;
+constexpr size_t kNoAllocArray =
+    kNoAllocBytes + kNoAllocBytes / kNoAllocClasses * (kNumClasses - kNoAllocClasses) + 8192;
 
 struct BatchStats {
   double plan_ms = 0;      // device plan build incl. the count read-back
@@ -190,7 +196,7 @@ class Context {
   // null per pair) receives the m x n tree-distance table.
   // run_batch without any device allocation: every buffer of the batch (plan,
   // TD arena, distances) is carved from the fixed device array of
-  // kNoAllocBytes this library holds per device (its address is looked up
+  // kNoAllocArray this library holds per device (its address is looked up
   // once, at init); launches go one by one (no graph is instantiated), the
   // distances are copied to the caller's memory directly. Pairs that do not
   // fit are refused with ERR_TOO_LARGE. Calls that overlap on one device
@@ -290,8 +296,9 @@ class Context {
   Group batch_[kMaxLevelStreams];  // the groups run_batch reuses
   Group na_;                        // run_batch_noalloc's group, bound to na_arena_
   std::vector<void*> retired_;      // see retire_list()
-  Arena na_arena_;                  // this device's fixed array (kNoAllocBytes)
-  int64_t noalloc_bytes(int32_t npairs, const int32_t* xs, const int32_t* ys) const;
+  Arena na_arena_;                  // this device's fixed array (kNoAllocArray)
+  int64_t noalloc_bytes(int32_t npairs, const int32_t* xs, const int32_t* ys,
+                        int32_t classes) const;
   // Whether the leaf lines of pair (x, y) are written in closed form (the
   // leaf kernel) rather than planned as tables: lane_enable, and under a
   // cost model both trees within the cost form's stack.

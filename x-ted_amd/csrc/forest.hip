@@ -31,35 +31,9 @@
 #include <utility>
 
 #include "kernels.hpp"
+#include "wave.hpp"
 
 namespace xted {
-
-constexpr int kBig = INT_MAX / 4;
-
-// DPP control codes (GFX9 encoding).
-#define DPP_ROW_SHR(n) (0x110 + (n))
-#define DPP_WAVE_SHR1 0x138
-#define DPP_ROW_BCAST15 0x142
-#define DPP_ROW_BCAST31 0x143
-
-// Inclusive prefix minimum over the 64 lanes of a wave (lane order). A lane
-// whose DPP source is out of range (or whose row the mask leaves out) reads
-// INT_MAX, the identity of min; with that identity as the "old" operand the
-// compiler fuses each move into its min (one v_min_i32 with a DPP source).
-__device__ __forceinline__ int wave_incl_min(int v) {
-  v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, DPP_ROW_SHR(1), 0xf, 0xf, false));
-  v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, DPP_ROW_SHR(2), 0xf, 0xf, false));
-  v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, DPP_ROW_SHR(4), 0xf, 0xf, false));
-  v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, DPP_ROW_SHR(8), 0xf, 0xf, false));
-  v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, DPP_ROW_BCAST15, 0xa, 0xf, false));
-  v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, DPP_ROW_BCAST31, 0xc, 0xf, false));
-  return v;
-}
-
-// Value of lane-1 (lane 0 receives `fill`).
-__device__ __forceinline__ int wave_shr1(int v, int fill) {
-  return __builtin_amdgcn_update_dpp(fill, v, DPP_WAVE_SHR1, 0xf, 0xf, false);
-}
 
 // ---------------------------------------------------------------------------
 // Leaf-keyroot lines in closed form. A line is a leaf keyroot v of one tree R
@@ -307,10 +281,6 @@ __global__ __launch_bounds__(64) void leaf_cost_kernel(LeafArgs A, int64_t ntile
   }
 }
 
-// A grid's threads (gridDim.x * blockDim.x) must stay below 2^32: launches
-// over more work items than kGridThreads / threads-per-group go in pieces.
-constexpr int64_t kGridThreads = int64_t{1} << 31;
-
 void launch_leaf(const LeafArgs& a, int64_t ntiles, hipStream_t s) {
   if (a.costs) {
     constexpr int64_t kChunk = kGridThreads / 64;
@@ -335,17 +305,6 @@ void launch_leaf(const LeafArgs& a, int64_t ntiles, hipStream_t s) {
 // reads with one coalesced E-int load per lane, and the row scan is G
 // chained wave scans over groups.
 // ---------------------------------------------------------------------------
-// Words of a TD row group: 2, 4 or 8 entries of 16 bits (td_t), two to a
-// 32-bit word, at any even byte address (the target's unaligned-access mode
-// lets one dwordx2 / dwordx4 load read them).
-typedef uint32_t u32x4a2 __attribute__((ext_vector_type(4), aligned(2)));
-typedef uint32_t u32x2a2 __attribute__((ext_vector_type(2), aligned(2)));
-typedef uint32_t u32x1a2 __attribute__((aligned(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-// Word 3 of a raw buffer resource on CDNA (32-bit data format, no swizzle).
-constexpr int32_t kBufferWord3 = 0x00020000;
-
 // ---------------------------------------------------------------------------
 // Column-blocked form (kXL). A table too wide or too LDS-hungry for one
 // workgroup is cut into blocks of BW = 64*W*C columns (t ranges), one
@@ -1503,8 +1462,8 @@ void launch_xl_zero(unsigned long long* p, int64_t n, hipStream_t s) {
 // ---------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------
-template <int W, int C>
-static void launch_row(const DPArgs& a, int lds_bytes, hipStream_t s) {
+template <int W>
+static void launch_shared(const DPArgs& a, int lds_bytes, hipStream_t s) {
   // One table per workgroup: a long task list goes in pieces.
   constexpr int64_t kChunk = kGridThreads / (64 * W);
   for (int64_t off = 0; off < a.ntasks; off += kChunk) {
@@ -1513,22 +1472,11 @@ static void launch_row(const DPArgs& a, int lds_bytes, hipStream_t s) {
     c.descs = a.descs + off;
     c.ntasks = std::min(kChunk, a.ntasks - off);
     if (a.costs)
-      hipLaunchKernelGGL((rowscan_kernel<W, C, false, true>), dim3((unsigned)c.ntasks),
+      hipLaunchKernelGGL((rowscan_kernel<W, 8, false, true>), dim3((unsigned)c.ntasks),
                          dim3(64 * W), (size_t)lds_bytes, s, c);
     else
-      hipLaunchKernelGGL((rowscan_kernel<W, C, false, false>), dim3((unsigned)c.ntasks),
+      hipLaunchKernelGGL((rowscan_kernel<W, 8, false, false>), dim3((unsigned)c.ntasks),
                          dim3(64 * W), (size_t)lds_bytes, s, c);
-  }
-}
-
-template <int W>
-static void launch_row_c(int ci, const DPArgs& a, int lds, hipStream_t s) {
-  switch (ci) {
-    case 0: launch_row<W, 1>(a, lds, s); break;
-    case 1: launch_row<W, 2>(a, lds, s); break;
-    case 2: launch_row<W, 4>(a, lds, s); break;
-    case 3: launch_row<W, 8>(a, lds, s); break;
-    default: launch_row<W, 16>(a, lds, s); break;
   }
 }
 
@@ -1561,22 +1509,12 @@ static hipError_t allow_lds(int limit) {
   return hipFuncSetAttribute(reinterpret_cast<const void*>(&rowscan_kernel<W, C, kXL, true>),
                              hipFuncAttributeMaxDynamicSharedMemorySize, limit);
 }
-template <int W>
-static hipError_t allow_lds_c(int limit) {
-  hipError_t e;
-  if ((e = allow_lds<W, 1>(limit)) != hipSuccess) return e;
-  if ((e = allow_lds<W, 2>(limit)) != hipSuccess) return e;
-  if ((e = allow_lds<W, 4>(limit)) != hipSuccess) return e;
-  if ((e = allow_lds<W, 8>(limit)) != hipSuccess) return e;
-  return allow_lds<W, 16>(limit);
-}
 hipError_t forest_init_attributes(int limit) {
-  hipError_t e;
-  if ((e = allow_lds_c<1>(limit)) != hipSuccess) return e;
-  if ((e = allow_lds_c<2>(limit)) != hipSuccess) return e;
-  if ((e = allow_lds_c<4>(limit)) != hipSuccess) return e;
-  if ((e = allow_lds_c<8>(limit)) != hipSuccess) return e;
-  if ((e = allow_lds_c<16>(limit)) != hipSuccess) return e;
+  hipError_t e = scan_init_attributes(limit);
+  if (e != hipSuccess) return e;
+  if ((e = allow_lds<4, 8>(limit)) != hipSuccess) return e;
+  if ((e = allow_lds<8, 8>(limit)) != hipSuccess) return e;
+  if ((e = allow_lds<16, 8>(limit)) != hipSuccess) return e;
   // column-blocked forms (xl_waves / xl_cpl)
   if ((e = allow_lds<8, 8, true>(limit)) != hipSuccess) return e;
   if ((e = allow_lds<8, 4, true>(limit)) != hipSuccess) return e;
@@ -1594,15 +1532,14 @@ bool launch_forest(int cls, const DPArgs& a, int lds_bytes, hipStream_t s) {
     return true;
   }
   if (cls >= 1 && cls <= kNumRowClasses) {
-    const int wi = (cls - 1) / 5, ci = (cls - 1) % 5;
-    switch (wi) {
-      case 0: launch_row_c<1>(ci, a, lds_bytes, s); break;
-      case 1: launch_row_c<2>(ci, a, lds_bytes, s); break;
-      case 2: launch_row_c<4>(ci, a, lds_bytes, s); break;
-      case 3: launch_row_c<8>(ci, a, lds_bytes, s); break;
-      default: launch_row_c<16>(ci, a, lds_bytes, s); break;
-    }
+    launch_scan((cls - 1) / 5, (cls - 1) % 5, a, lds_bytes, s);
     return true;
+  }
+  switch (cls - kClassShared) {
+    case 0: launch_shared<4>(a, lds_bytes, s); return true;
+    case 1: launch_shared<8>(a, lds_bytes, s); return true;
+    case 2: launch_shared<16>(a, lds_bytes, s); return true;
+    default: break;
   }
   switch (cls - kFirstXLClass) {  // must match xl_waves / xl_cpl
     case 0: launch_xl<8, 8>(a, lds_bytes, s); return true;

@@ -89,8 +89,9 @@ inline int64_t plan_blocks(int32_t Kx, int32_t Ky, int32_t chunk) {
   return (Ky + lper - 1) / lper;
 }
 void launch_plan(const PlanArgs& a, int64_t nblocks, hipStream_t s);
-void launch_gather_dist(const PairMeta* pairs, const td_t* td, int32_t npairs, int32_t* dist,
-                        hipStream_t s);
+constexpr int32_t kDistAborted = INT32_MIN;  // what a gather writes for a group that gave up
+void launch_gather_dist(const PairMeta* pairs, const td_t* td, int32_t npairs,
+                        const int32_t* abort_flag, int32_t* dist, hipStream_t s);
 // dst[i] = src[i] for i < n: a table of the arena widened to the int32 a
 // caller receives.
 void launch_widen_td(const td_t* src, int32_t* dst, int64_t n, hipStream_t s);
@@ -140,6 +141,10 @@ void launch_leaf(const LeafArgs& a, int64_t ntiles, hipStream_t s);
 // Ints of a group's column-blocked record (DPArgs::xl_abort).
 constexpr int kAbortInts = 16;
 
+// A grid's threads (gridDim.x * blockDim.x) must stay below 2^32: launches
+// over more work items than kGridThreads / threads-per-group go in pieces.
+constexpr int64_t kGridThreads = int64_t{1} << 31;
+
 // Entries of padding the TD arena keeps before and after every table, so
 // the row-scan kernels can issue whole-group loads without bounds branches
 // (a group of 8 entries starts at most 7 before column c0 or at c0 itself).
@@ -183,6 +188,9 @@ void launch_xl_layout(const XLLayoutArgs& a, hipStream_t s);
 void launch_xl_zero(unsigned long long* p, int64_t n, hipStream_t s);
 // Lets every row-scan kernel request up to lds_limit bytes of dynamic LDS.
 hipError_t forest_init_attributes(int lds_limit);
+hipError_t scan_init_attributes(int lds_limit);
+// On-chip row scan of W = 2^wi waves and C = 2^ci columns per lane (scan.hip).
+void launch_scan(int wi, int ci, const DPArgs& a, int lds_bytes, hipStream_t s);
 // Launches the row-scan kernel of class `cls` over a.tasks[0..ntasks).
 // Returns false when the class has no kernel (the leaf class runs as one
 // launch_leaf, class kClassXL has none). Column-blocked classes launch

@@ -41,15 +41,14 @@ __device__ __forceinline__ void classify(const PlanArgs& A, const TreeMeta& tx,
   const int32_t kdx = A.pool.skd[kx], kdy = A.pool.skd[ly];
   const int32_t level = kdx + kdy + loff;
   const ClassRule& rule = A.tail_level[level] ? A.rule_tail : A.rule;
-  // Slot storage of the oriented table: one uint16 row per nesting level of
-  // the row keyroot (at least one: the kernels read slot 0 unconditionally),
-  // each as long as the column keyroot's leaf count plus one sink entry.
+  // One slot row per nesting level of the row keyroot (at least one: the
+  // kernels read slot 0 unconditionally).
   const int32_t slots = max(a <= b ? kdx : kdy, 1);
   const int32_t leaves_c = a <= b ? A.pool.sleaf[ly] : A.pool.sleaf[kx];
-  int64_t need = (int64_t)slots * (leaves_c + 1) * 2;
+  int64_t need = 0;
   // With the leaf kernel off, single-row tables take the row-scan forms.
-  int cls = table_class(a, b, need, a <= b ? kdx : kdy, a <= b ? kdy : kdx, leaves_c,
-                        leaf_form, rule, &need);
+  int cls = table_class(a, b, a <= b ? kdx : kdy, a <= b ? kdy : kdx, leaves_c, leaf_form, rule,
+                        &need);
   // A forced column-blocked form takes every multi-row table it can hold.
   if (A.force_class >= kFirstXLClass && A.force_class < kFirstXLClass + kNumXLForms && cls >= 1 &&
       cls != kClassXL) {
@@ -66,18 +65,18 @@ __device__ __forceinline__ void classify(const PlanArgs& A, const TreeMeta& tx,
   if (is_tiny(A.force_class) && cls >= 1 && (cls <= kNumRowClasses || is_tiny(cls))) {
     const int k = A.force_class - kClassTiny;
     const int cols = a <= b ? b : a;
-    const int64_t row_need = (int64_t)slots * (leaves_c + 1) * 2;
+    const int64_t row_need = scan_lds_need(slots, leaves_c, 0, 1);
     if (cols <= tiny_seg(k) && row_need <= tiny_max_lds(k)) {
       cls = A.force_class;
       need = row_need;
     }
   }
   if (A.force_class >= 1 && A.force_class <= kNumRowClasses && cls >= 1 &&
-      (cls <= kNumRowClasses || is_tiny(cls))) {
+      (cls <= kNumRowClasses || is_tiny(cls) || is_shared(cls))) {
     const int wi = (A.force_class - 1) / 5, ci = (A.force_class - 1) % 5;
     const int cols = a <= b ? b : a;
-    const int64_t row_need = (int64_t)slots * (leaves_c + 1) * 2;
-    if ((cls < kClassXL || is_tiny(cls)) && cols <= 64 * (1 << wi) * (1 << ci) &&
+    const int64_t row_need = scan_lds_need(slots, leaves_c, a <= b ? kdy : kdx, 1 << wi);
+    if ((cls < kClassXL || is_tiny(cls) || is_shared(cls)) && cols <= 64 * (1 << wi) * (1 << ci) &&
         row_need <= A.rule.lds_max) {
       cls = A.force_class;
       need = row_need;
@@ -338,8 +337,9 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs A) {
     sweep([&](bool active, int bucket, int, uint32_t i0, uint32_t j0, unsigned long long) {
       const unsigned long long pos = wave_reserve(A, T, bucket, active);
       if (active) {
-        A.tasks[pos] = task_pack((uint32_t)ch.p, i0, j0);
-        A.descs[pos] = make_desc(A, pm, tx, ty, (int32_t)i0, (int32_t)j0);
+        const TaskDesc d = make_desc(A, pm, tx, ty, (int32_t)i0, (int32_t)j0);
+        A.descs[pos] = d;
+        A.tasks[pos] = task_pack((uint32_t)ch.p, i0, j0, d.base_rx < 0);
       }
     });
   }
@@ -392,18 +392,19 @@ void launch_plan(const PlanArgs& a, int64_t nblocks, hipStream_t s) {
     hipLaunchKernelGGL(plan_kernel<true>, dim3((unsigned)nblocks), dim3(kPlanThreads), 0, s, a);
 }
 
-// Distances TD[0][0] of every pair into dist[].
+// Distances TD[0][0] of every pair into dist[], or kDistAborted everywhere
+// when a wait of the group's kernels gave up.
 __global__ void gather_dist_kernel(const PairMeta* pairs, const td_t* td, int32_t npairs,
-                                   int32_t* dist) {
+                                   const int32_t* abort_flag, int32_t* dist) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < npairs) dist[i] = td[pairs[i].td_off];
+  if (i < npairs) dist[i] = abort_flag[0] ? kDistAborted : td[pairs[i].td_off];
 }
 
-void launch_gather_dist(const PairMeta* pairs, const td_t* td, int32_t npairs, int32_t* dist,
-                        hipStream_t s) {
+void launch_gather_dist(const PairMeta* pairs, const td_t* td, int32_t npairs,
+                        const int32_t* abort_flag, int32_t* dist, hipStream_t s) {
   if (npairs <= 0) return;
   hipLaunchKernelGGL(gather_dist_kernel, dim3((npairs + 255) / 256), dim3(256), 0, s, pairs, td,
-                     npairs, dist);
+                     npairs, abort_flag, dist);
 }
 
 __global__ __launch_bounds__(256) void widen_td_kernel(const td_t* __restrict__ src,
