@@ -151,9 +151,11 @@ XTED_HD inline int shared_cols(int k) { return 64 * 8 * (4 << k); }
 XTED_HD inline int tiny_seg(int k) { return 16 << k; }
 // Slot bytes of one table of tiny form k: 32 KiB per workgroup of 256 lanes.
 XTED_HD inline int64_t tiny_max_lds(int k) { return (int64_t)2048 << k; }
-// Column-blocked forms: waves and columns per lane of one block.
-XTED_HD inline int xl_waves(int k) { return k <= 1 ? 8 : k == 2 ? 4 : 2; }
-XTED_HD inline int xl_cpl(int k) { return k == 0 ? 8 : k <= 3 ? 4 : k == 4 ? 2 : 1; }
+// Column-blocked forms: waves and columns per lane of one block. The narrow
+// forms serve deep trees, whose slot rows leave little LDS: one wave's edges
+// take the least.
+XTED_HD inline int xl_waves(int k) { return k <= 1 ? 8 : k == 2 ? 4 : 1; }
+XTED_HD inline int xl_cpl(int k) { return k == 0 || k == 3 ? 8 : k == 5 ? 2 : 4; }
 XTED_HD inline int xl_bw(int k) { return 64 * xl_waves(k) * xl_cpl(k); }  // 4096 .. 128
 // Column-blocked tables with at most this many rows are swept block after
 // block by one workgroup (forms of at most 1024 columns), with no waits
@@ -197,6 +199,10 @@ XTED_HD inline int size_band(int cls, int rows, int64_t lds, int mode, int light
 XTED_HD inline int bucket_of(int level, int cls, int band) {
   return (level * kNumClasses + cls) * kBands + band;
 }
+
+// Words of a column-blocked table are laid out in whole 128-byte L2 lines.
+constexpr int32_t kXLLineWords = 16;
+XTED_HD inline int32_t xl_pad(int32_t w) { return (w + kXLLineWords - 1) & ~(kXLLineWords - 1); }
 
 // Saved-row slots are uint16 (F <= |subtree x| + |subtree y| < 65536).
 // LDS budget for the slots of one table, per wave of its workgroup.
@@ -265,14 +271,6 @@ XTED_HD inline int ilog2_ceil(int v) {
   return r;
 }
 
-// Slot bytes of one block of a column-blocked table: one uint16 row per
-// nesting level of the row keyroot, each holding the block's own far columns
-// (at most min(leaves, bw)), the boundary entry, kd_c+1 imports and a sink.
-XTED_HD inline int64_t xl_lds_need(int kd_r, int kd_c, int leaves_c, int bw) {
-  const int own = leaves_c < bw ? leaves_c : bw;
-  return (int64_t)(kd_r > 1 ? kd_r : 1) * (own + 3 + kd_c) * 2;
-}
-
 // On-chip row scan of w waves: entries of the ring between two waves, and the
 // LDS bytes of a table whose row keyroot has nesting height slots (at least 1)
 // and whose column keyroot has leaves_c leaves and nesting height kd_c: one
@@ -285,6 +283,29 @@ XTED_HD inline int64_t scan_lds_need(int slots, int leaves_c, int kd_c, int w) {
   if (w == 1) return (int64_t)slots * (leaves_c + 1) * 2;
   return (int64_t)slots * (leaves_c - 1 + w * (kd_c + 3)) * 2 +
          (int64_t)(w + 1) * kEdgeRows * (kd_c + 3) * 4 + 8 * (w + 2);
+}
+
+// The same of one block of a column-blocked table, whose own far columns are
+// at most bw, with edges of shorter rings on the narrow forms.
+XTED_HD constexpr int xl_edge_rows(int cols_per_lane) { return cols_per_lane <= 8 ? 4 : 8; }
+XTED_HD inline int64_t xl_lds_need(int kd_r, int kd_c, int leaves_c, int k) {
+  const int w = xl_waves(k), bw = xl_bw(k);
+  const int own = leaves_c < bw ? leaves_c : bw;
+  return (int64_t)(kd_r > 1 ? kd_r : 1) * (own + w * (kd_c + 3)) * 2 +
+         (int64_t)(w + 1) * xl_edge_rows(w * xl_cpl(k)) * (kd_c + 3) * 4 + 8 * (w + 2);
+}
+// Which of these forms, from form k on, takes a table: the widest whose blocks
+// fit lds_max. A table the narrowest form's slot rows fit is never refused:
+// its edges, at most kXLEdgeBytes, come on top of lds_max (a workgroup may
+// have 160 KiB). -1: none. *need receives the form's bytes.
+constexpr int kXLEdgeBytes = 2 * 4 * (kMaxImports + 2) * 4 + 8 * 3;
+XTED_HD inline int xl_form(int kd_r, int kd_c, int leaves_c, int k, int lds_max, int64_t* need) {
+  if (kd_c + 1 > kMaxImports) return -1;
+  for (; k < kNumXLForms; ++k) {
+    *need = xl_lds_need(kd_r, kd_c, leaves_c, k);
+    if (*need <= lds_max + (k == kNumXLForms - 1 ? 8 * (kd_c + 3) * 4 + 24 : 0)) return k;
+  }
+  return -1;
 }
 
 // Class of table (a x b): kd_r / kd_c / leaves_c (row keyroot height, column
@@ -326,17 +347,11 @@ XTED_HD inline int table_class(int a, int b, int kd_r, int kd_c, int leaves_c, b
     }
   }
   if (cols > 64 * cpl_cap * kMaxRowWaves || *need > rule.lds_max) {
-    if (kd_c + 1 > kMaxImports) return kClassXL;
     // Short tables take the forms one workgroup sweeps.
-    for (int k = rows <= rule.xl_seq_rows ? kFirstSeqXLForm : rule.xl_first; k < kNumXLForms;
-         ++k) {
-      const int64_t n = xl_lds_need(kd_r, kd_c, leaves_c, xl_bw(k));
-      if (n <= rule.lds_max) {
-        *need = n;
-        return kFirstXLClass + k;
-      }
-    }
-    return kClassXL;
+    const int k = xl_form(kd_r, kd_c, leaves_c,
+                          rows <= rule.xl_seq_rows ? kFirstSeqXLForm : rule.xl_first,
+                          rule.lds_max, need);
+    return k < 0 ? kClassXL : kFirstXLClass + k;
   }
   int w = 1 << wi;
   int c = (cols + 64 * w - 1) / (64 * w);

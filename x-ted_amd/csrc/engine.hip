@@ -141,7 +141,8 @@ int Context::init() {
   HIP_TRY(hipEventCreateWithFlags(&plan_done_, hipEventDisableTiming));
   for (auto& ev : join_ev_) HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
   // Slot storage limit: what the device grants one workgroup, less the
-  // row-scan kernels' static LDS, capped at kLdsMaxTable.
+  // row-scan kernels' static LDS, capped at kLdsMaxTable (which leaves the
+  // column-blocked forms their kXLEdgeBytes).
   hipDeviceProp_t prop;
   HIP_TRY(hipGetDeviceProperties(&prop, device_));
   lds_limit = (int32_t)std::min<size_t>(kLdsMaxTable, prop.sharedMemPerBlock - 256);
@@ -862,15 +863,14 @@ int Context::poll(Group& g, bool wait, int32_t* dist) {
   return OK;
 }
 
-// The abort record of a group: {flag, claimed, ticket (or task), kind << 24 |
-// row, word low, word high, epoch}; kinds as below.
+// The abort record of a group: {flag, claimed, task, kind << 24 | row}; kinds
+// as below.
 int xl_timeout(const int32_t* rec) {
   const char* const kinds[] = {"carry", "import", "wave"};
-  set_error("run_batch: a table stopped waiting for its neighbour block (ticket " +
+  set_error("run_batch: a table stopped waiting for its neighbour block (task " +
             std::to_string(rec[2]) + ", " + kinds[std::min(2, std::max(0, rec[3] >> 24))] +
             " of row " +
-            std::to_string(rec[3] & 0xFFFFFF) + ", read " + std::to_string((uint32_t)rec[5]) +
-            ":" + std::to_string(rec[4]) + ", epoch " + std::to_string((uint32_t)rec[6]) + ")");
+            std::to_string(rec[3] & 0xFFFFFF) + ")");
   return ERR_TIMEOUT;
 }
 

@@ -162,7 +162,7 @@ struct DPArgs {
   unsigned long long* xl_words;  // cross-workgroup words of every such task
   const int64_t* xl_off;         // this launch's tasks' offsets into xl_words
   unsigned int* xl_ticket;       // (task, block) counter of this launch, zeroed
-  int32_t* xl_abort;             // [0] raised when a wait gives up, [1..6] what it waited for,
+  int32_t* xl_abort;             // [0] raised when a wait gives up, [1..3] what it waited for,
                                  // [8] stale prefetched reads, [9] throttle checks that waited
   uint32_t xl_epoch;             // tag of this launch's words (never 0)
   int32_t xl_nbmax;              // workgroups per task in the grid
@@ -186,11 +186,14 @@ struct XLLayoutArgs {
 };
 void launch_xl_layout(const XLLayoutArgs& a, hipStream_t s);
 void launch_xl_zero(unsigned long long* p, int64_t n, hipStream_t s);
-// Lets every row-scan kernel request up to lds_limit bytes of dynamic LDS.
+// Lets every row-scan kernel request up to lds_limit bytes of dynamic LDS,
+// the column-blocked ones kXLEdgeBytes more.
 hipError_t forest_init_attributes(int lds_limit);
 hipError_t scan_init_attributes(int lds_limit);
-// On-chip row scan of W = 2^wi waves and C = 2^ci columns per lane (scan.hip).
+// On-chip row scan of W = 2^wi waves and C = 2^ci columns per lane, and
+// column-blocked form k (scan.hip).
 void launch_scan(int wi, int ci, const DPArgs& a, int lds_bytes, hipStream_t s);
+void launch_xl(int form, const DPArgs& a, int lds_bytes, hipStream_t s);
 // Launches the row-scan kernel of class `cls` over a.tasks[0..ntasks).
 // Returns false when the class has no kernel (the leaf class runs as one
 // launch_leaf, class kClassXL has none). Column-blocked classes launch

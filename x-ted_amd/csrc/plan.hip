@@ -54,8 +54,8 @@ __device__ __forceinline__ void classify(const PlanArgs& A, const TreeMeta& tx,
       cls != kClassXL) {
     const int k = A.force_class - kFirstXLClass;
     const int32_t kd_c = a <= b ? kdy : kdx;
-    const int64_t n = xl_lds_need(a <= b ? kdx : kdy, kd_c, leaves_c, xl_bw(k));
-    if (kd_c + 1 <= kMaxImports && n <= A.rule.lds_max) {
+    int64_t n = 0;
+    if (xl_form(a <= b ? kdx : kdy, kd_c, leaves_c, k, A.rule.lds_max, &n) == k) {
       cls = A.force_class;
       need = n;
     }

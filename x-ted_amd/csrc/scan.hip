@@ -67,13 +67,6 @@ constexpr int32_t kRowTree = 1 << 28;
 constexpr int32_t kRowFull = 1 << 29;
 constexpr int32_t kRowSaved = 1 << 30;
 
-// Polls of a neighbour's progress before a wave gives up (never reached: the
-// waves of a workgroup are resident together and wait only on the wave before
-// or after them).
-constexpr int kEdgePolls = 1 << 24;
-constexpr int kSyncRows = 4;
-static_assert(kEdgeRows == 2 * kSyncRows, "a wave may fill one group while the next takes another");
-
 // Bytes of a TD buffer resource, from kTdPad entries before the table: more
 // than any table and its padding (32767^2 entries of 2 bytes), and as an
 // offset out of range whatever scalar offset (below it) is added.
@@ -84,25 +77,277 @@ __device__ __forceinline__ void lds_order() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 }
 
-template <int W, int C, bool kCost>
-__global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
+// ---------------------------------------------------------------------------
+// Column-blocked tables (kXL): a table too wide or too LDS-hungry for one
+// workgroup, cut into blocks of 64*W*C columns, one workgroup each. The edge
+// between two blocks goes through device memory: wave W + 1 of the block
+// before (edge_out) takes the last wave's edge entries from LDS and writes
+// them out, wave W of the block after (edge_in) reads them and fills its
+// block's first edge, so the other waves only ever see LDS. Per row a carry
+// word (nb - 1 runs, one per edge, padded to whole 128-byte L2 lines), per
+// saved row and edge a line-padded run of kds imports.
+//
+// Words are {epoch:32 | value:32}, written once per launch with atomic
+// exchanges (performed where every XCD sees the same line; each XCD has an L2
+// of its own), so nothing is cleared between launches and a word tells by
+// itself whether it is there. Carries are read a line (16 rows) at a time with
+// compare-exchanges against a value no word holds, which return the current
+// word; once a line is complete so are the imports of its rows, as a rule,
+// and these are read with plain loads, whose lines no XCD has read before. A
+// stale word all the same (its epoch is old) is read again atomically.
+// Workgroups take (table, block) from a ticket counter in start order, so a
+// block only waits on blocks that are already running. Waits are bounded:
+// after kXLWaitTicks of the 100 MHz wall clock a wave raises the abort flag
+// (recording what it waited for), every waiting wave then stops waiting, and
+// the call fails.
+// Tables with at most xl_seq_rows rows are swept block after block by one
+// workgroup; their words stay in its XCD and need no atomics.
+//
+// What bounds a row: the instructions of one wave, as on chip, with at most
+// two waves to a SIMD. Measured, us a row over the blocks of an 8000-node RRT
+// pair's root table, of 4096 / 2048 / 1024 / 512 columns: 0.45 / 0.32 / 0.29 /
+// 0.40 (on chip 16 waves of 8 columns 0.63). With a barrier per row and every
+// wave reading the words itself, a 20,000-node pair's pipelined blocks took
+// 138 ms against 34 here, its tables of at most 256 rows 42 against 29.
+// ---------------------------------------------------------------------------
+constexpr uint64_t kXLWaitTicks = 1000000000ull;  // 10 s at 100 MHz
+constexpr unsigned long long kXLNever = ~0ull;    // epoch 0xFFFFFFFF is never issued
+constexpr int kXLLineRows = kXLLineWords;         // carries read at a time: one line
+__device__ __forceinline__ unsigned long long xl_peek(const unsigned long long* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// (An idempotent or-with-0 would be turned back into a plain load.)
+__device__ __forceinline__ unsigned long long xl_load(unsigned long long* p) {
+  unsigned long long cur = kXLNever;
+  (void)__hip_atomic_compare_exchange_strong(p, &cur, kXLNever, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+  return cur;
+}
+__device__ __forceinline__ void xl_store(unsigned long long* p, uint32_t epoch, int32_t v,
+                                         bool local) {
+  const unsigned long long w = ((unsigned long long)epoch << 32) | (uint32_t)v;
+  if (local) __hip_atomic_store(p, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else (void)__hip_atomic_exchange(p, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// A bounded wait: true while it may go on. The wave that gives up records
+// what = kind << 24 | row (kinds: 0 a carry, 1 an import, 2 a neighbour wave)
+// in abort_flag[2..3]; others see the flag.
+struct Patience {
+  uint64_t t0 = 0;
+  bool gone = false;
+  __device__ __forceinline__ bool wait(int n, int32_t* abort_flag, int32_t ticket, int32_t what) {
+    if (gone) return false;
+    __builtin_amdgcn_s_sleep(1);
+    if ((n & 255) != 255) return true;
+    const uint64_t now = wall_clock64();
+    if (n < 256) t0 = now;  // this wait's first look at the clock
+    const bool raised = xl_peek(reinterpret_cast<unsigned long long*>(abort_flag)) & 0xFFFFFFFFu;
+    if (raised || now - t0 > kXLWaitTicks) {
+      if (!raised && atomicCAS(abort_flag + 1, 0, 1) == 0) {
+        abort_flag[2] = ticket;
+        abort_flag[3] = what;
+      }
+      (void)atomicExch(abort_flag, 1);
+      gone = true;
+    }
+    return !gone;
+  }
+};
+
+// What the edge waves need of a block: the table's rows, the first of its
+// words, its edges' byte offsets in LDS.
+struct XLEdge {
+  const NodeRec* rrecR;
+  const int32_t* lrankR;
+  int32_t r0, rmax, nrows, kds, nb, blk, ticket;
+  bool seq;
+  unsigned long long* words;
+  uint32_t edge;         // LDS byte offset of the edge to fill or empty
+  uint32_t entry_bytes;
+};
+// Flags of 64 rows (lane = row k0 + lane): bit 0 full, bit 1 saved, bit 2 the
+// row is in the table; and the saved row's index (leaf rank of r-1).
+__device__ __forceinline__ void xl_rows(const XLEdge& x, int32_t k0, int lane, int32_t& flags,
+                                        int32_t& rid) {
+  const int32_t rr = x.rmax - 1 - (k0 + lane);
+  const int32_t r = max(rr, x.r0);
+  NodeRec rc = x.rrecR[r];
+  int32_t onext = x.rrecR[max(r - 1, x.r0)].orl;
+  int32_t lr = x.lrankR[max(r - 1, x.r0)] - x.lrankR[x.r0];
+  asm volatile("" : "+v"(rc.orl), "+v"(rc.y), "+v"(onext), "+v"(lr));
+  const bool in = rr >= x.r0;
+  const bool saved = in & (r > x.r0) & (rc.y < 0);
+  const bool full = saved | (in & (rc.orl + 1 == x.rmax)) |
+                    (in & (r > x.r0) & (onext + 1 == x.rmax));
+  flags = (int32_t)full | ((int32_t)saved << 1) | ((int32_t)in << 2);
+  rid = lr;
+}
+
+// Wave W: fills the block's first edge from the words of the block before.
+template <int D, int kSync>
+__device__ __forceinline__ void edge_in(const DPArgs& A, const XLEdge& x, unsigned char* lds,
+                                        int lane) {
+  auto l32 = [&](uint32_t byte) -> int32_t& { return *reinterpret_cast<int32_t*>(lds + byte); };
+  unsigned long long* const prog = reinterpret_cast<unsigned long long*>(lds);
+  const int32_t cstride = xl_pad(x.nrows), kdsp = xl_pad(x.kds);
+  unsigned long long* const carries = x.words + (int64_t)(x.blk - 1) * cstride;
+  unsigned long long* const exps = x.words + (int64_t)(x.nb - 1) * cstride;
+  auto imp_word = [&](int32_t rid, int32_t d) {
+    return exps + ((int64_t)rid * x.nb + (x.blk - 1)) * kdsp + d;
+  };
+  Patience pat;
+  int32_t flags = 0, rid = 0, n_stale = 0, n_wait = 0, q = 0;
+  uint32_t qoff = 0;
+  const uint32_t edge_bytes = D * x.entry_bytes;
+  // The line of row k: lane l holds row k + l's carry word.
+  auto poll_line = [&](int32_t k) {
+    const int32_t row = min(k + (lane & (kXLLineRows - 1)), x.nrows - 1);
+    return x.seq ? xl_peek(carries + row) : xl_load(carries + row);
+  };
+  unsigned long long cw = poll_line(0);
+  for (int32_t k0 = 0; k0 < x.nrows; k0 += kXLLineRows) {
+    if ((k0 & 63) == 0) xl_rows(x, k0, lane, flags, rid);
+    if (__ballot((uint32_t)(cw >> 32) != A.xl_epoch)) {
+      ++n_wait;
+      for (int n = 0; __ballot((uint32_t)(cw >> 32) != A.xl_epoch); ++n) {
+        if (!pat.wait(n, A.xl_abort, x.ticket, k0)) break;
+        cw = poll_line(k0);
+      }
+    }
+    const int32_t carry = (int32_t)(uint32_t)cw;
+    // The first 64 imports of the line's saved rows, all in flight together.
+    unsigned long long iw[kXLLineRows];
+#pragma unroll
+    for (int i = 0; i < kXLLineRows; ++i) {
+      const int at = (k0 & 63) + i;
+      iw[i] = (unsigned long long)A.xl_epoch << 32;  // nothing to read: valid
+      if ((__builtin_amdgcn_readlane(flags, at) & 2) && lane < x.kds)
+        iw[i] = xl_peek(imp_word(__builtin_amdgcn_readlane(rid, at), lane));
+    }
+    if (k0 + kXLLineRows < x.nrows) cw = poll_line(k0 + kXLLineRows);
+#pragma unroll
+    for (int i = 0; i < kXLLineRows; ++i) {
+      const int32_t k = k0 + i;
+      if (i % kSync == 0) {
+        // The group's full rows find room once the first wave has taken
+        // enough of the entries before.
+        for (int n = 0;; ++n) {
+          const unsigned long long pa =
+              __hip_atomic_load(prog + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          if (__builtin_amdgcn_readfirstlane((int32_t)(uint32_t)(pa >> 32)) >= q - kSync) break;
+          if (!pat.wait(n, A.xl_abort, x.ticket, (2 << 24) | k)) break;
+        }
+        lds_order();
+      }
+      const int at = (k0 & 63) + i;
+      const int32_t fl = __builtin_amdgcn_readlane(flags, at);
+      if (fl & 1) {
+        if ((fl & 2) && __ballot((uint32_t)(iw[i] >> 32) != A.xl_epoch)) {
+          ++n_stale;
+          for (int n = 0; __ballot((uint32_t)(iw[i] >> 32) != A.xl_epoch); ++n) {
+            if ((uint32_t)(iw[i] >> 32) != A.xl_epoch)
+              iw[i] = xl_load(imp_word(__builtin_amdgcn_readlane(rid, at), lane));
+            if (!pat.wait(n, A.xl_abort, x.ticket, (1 << 24) | k)) break;
+          }
+        }
+        const uint32_t entry = x.edge + qoff;
+        l32(entry + 4 * min(1 + lane, x.kds + 1)) = (int32_t)(uint32_t)iw[i];
+        if (fl & 2) {
+          for (int32_t d0 = 64; d0 < x.kds; d0 += 64) {
+            const int32_t d = d0 + lane;
+            unsigned long long w = (unsigned long long)A.xl_epoch << 32;
+            if (d < x.kds) w = xl_peek(imp_word(__builtin_amdgcn_readlane(rid, at), d));
+            for (int n = 0; __ballot((uint32_t)(w >> 32) != A.xl_epoch); ++n) {
+              if ((uint32_t)(w >> 32) != A.xl_epoch)
+                w = xl_load(imp_word(__builtin_amdgcn_readlane(rid, at), d));
+              if (!pat.wait(n, A.xl_abort, x.ticket, (1 << 24) | k)) break;
+            }
+            l32(entry + 4 * min(1 + d, x.kds + 1)) = (int32_t)(uint32_t)w;
+          }
+        }
+        l32(entry) = __builtin_amdgcn_readlane(carry, i);
+        ++q;
+        qoff = qoff + x.entry_bytes == edge_bytes ? 0 : qoff + x.entry_bytes;
+      }
+      if (i % kSync == kSync - 1) {
+        lds_order();
+        __hip_atomic_store(prog, ((unsigned long long)(uint32_t)q << 32) | (uint32_t)(k + 1),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        lds_order();
+      }
+    }
+  }
+  if (lane == 0 && n_stale) atomicAdd(A.xl_abort + 8, n_stale);
+  if (lane == 0 && n_wait) atomicAdd(A.xl_abort + 9, n_wait);
+}
+
+// Wave W + 1: empties the block's last edge into the words of this block.
+template <int D, int kSync>
+__device__ __forceinline__ void edge_out(const DPArgs& A, const XLEdge& x, unsigned char* lds,
+                                         int W, int lane) {
+  auto l32 = [&](uint32_t byte) -> int32_t& { return *reinterpret_cast<int32_t*>(lds + byte); };
+  unsigned long long* const prog = reinterpret_cast<unsigned long long*>(lds);
+  const int32_t cstride = xl_pad(x.nrows), kdsp = xl_pad(x.kds);
+  unsigned long long* const carries = x.words + (int64_t)x.blk * cstride;
+  unsigned long long* const exps = x.words + (int64_t)(x.nb - 1) * cstride;
+  Patience pat;
+  int32_t flags = 0, rid = 0, q = 0;
+  uint32_t qoff = 0;
+  const uint32_t edge_bytes = D * x.entry_bytes;
+  for (int32_t k0 = 0; k0 < x.nrows; k0 += kSync) {
+    if ((k0 & 63) == 0) xl_rows(x, k0, lane, flags, rid);
+    for (int n = 0;; ++n) {
+      const unsigned long long pb =
+          __hip_atomic_load(prog + W, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (__builtin_amdgcn_readfirstlane((int32_t)(uint32_t)pb) > k0) break;
+      if (!pat.wait(n, A.xl_abort, x.ticket, (2 << 24) | k0)) break;
+    }
+    lds_order();
+    int32_t carry = 0;  // lane i: row k0 + i's (rows that are not full hand on any value)
+#pragma unroll
+    for (int i = 0; i < kSync; ++i) {
+      const int at = (k0 & 63) + i;
+      const int32_t fl = __builtin_amdgcn_readlane(flags, at);
+      if (fl & 1) {
+        const uint32_t entry = x.edge + qoff;
+        const int32_t c = l32(entry);
+        if (fl & 2) {
+          const int32_t r = __builtin_amdgcn_readlane(rid, at);
+          for (int32_t d0 = 0; d0 < x.kds; d0 += 64) {
+            const int32_t d = d0 + lane;
+            const int32_t v = l32(entry + 4 * min(1 + d, x.kds + 1));
+            if (d < x.kds)
+              xl_store(exps + ((int64_t)r * x.nb + x.blk) * kdsp + d, A.xl_epoch, v, x.seq);
+          }
+        }
+        carry = lane == i ? c : carry;
+        ++q;
+        qoff = qoff + x.entry_bytes == edge_bytes ? 0 : qoff + x.entry_bytes;
+      }
+    }
+    // The entries are taken (their reads are done before this write).
+    lds_order();
+    __hip_atomic_store(prog + W + 1, ((unsigned long long)(uint32_t)q << 32) | (uint32_t)k0,
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (lane < kSync && k0 + lane < x.nrows)
+      xl_store(carries + k0 + lane, A.xl_epoch, carry, x.seq);
+  }
+}
+
+// One table, or with kXL one column block of a table, on the calling
+// workgroup (64 * W threads, 128 more with kXL).
+template <int W, int C, bool kCost, bool kXL>
+__device__ __forceinline__ void scan_block(const DPArgs& A, const TaskDesc& dsc, int32_t ix,
+                                           int32_t blk, int32_t nb) {
+  constexpr bool kEdges = W > 1 || kXL;
   // TD ring slots: a power of two dividing 64.
-  constexpr int S = C >= 16 || (W == 1 && C >= 8) ? 4 : 8;
+  constexpr int S = C >= 16 || (W == 1 && C >= 8 && !kXL) || (kXL && kCost && C >= 8) ? 4 : 8;
   constexpr int PD = S - 1;                    // rows of TD prefetched
   constexpr int NW = C == 1 ? 1 : C / 2;       // words of one row: two 16-bit entries each
-  constexpr int D = kEdgeRows;
+  constexpr int D = kXL ? xl_edge_rows(W * C) : kEdgeRows;
+  constexpr int kSync = D / 2;  // a wave may fill one group while the next takes another
   extern __shared__ __align__(16) unsigned char lds[];
-
-  // Workgroups go round robin over the 8 XCDs, each with its own L2; task
-  // order keeps a pair's tables together, so kXcdRun consecutive tasks are
-  // given to one XCD (the last, partial span keeps its order). The 4096-pair
-  // batch ran 101.6 ms without, 100.1 with 16, 101.0 with 64, 104.8 with 256.
-  constexpr uint32_t kXcds = 8, kXcdRun = 16, kSpan = kXcds * kXcdRun;
-  uint32_t ix = blockIdx.x;
-  if ((ix | (kSpan - 1)) < (uint64_t)A.ntasks)
-    ix = (ix & ~(kSpan - 1)) + (ix % kXcds) * kXcdRun + (ix % kSpan) / kXcds;
-  if ((int64_t)ix >= A.ntasks) return;
-  const TaskDesc dsc = A.descs[ix];
   const bool rows_x = dsc.base_rx < 0;
   const int64_t offR = dsc.offR;
   const int64_t offC = dsc.offC;
@@ -121,11 +366,12 @@ __global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
   const int32_t orl_c0 = cmax - 1;
 
   // Uniform over the wave, so it lives in a scalar register.
-  const int wave = W > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  const int wave = kEdges ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
   const int lane = threadIdx.x & 63;
-  const int32_t tb = wave * 64 * C;      // first t of this wave's block
-  const int32_t tlane = tb + lane * C;   // t of this lane's element 0
-  const int32_t nw = W > 1 ? (ncols + 64 * C - 1) / (64 * C) : 1;  // waves with columns
+  const int32_t tb0 = kXL ? blk * (64 * W * C) : 0;  // first t of the block
+  const int32_t tb = tb0 + wave * 64 * C;            // and of this wave's part
+  const int32_t tlane = tb + lane * C;               // t of this lane's element 0
+  const int32_t nw = kEdges ? min(W, (ncols - tb0 + 64 * C - 1) / (64 * C)) : 1;  // waves used
 
   // Costs (kCost). Hpre / Vpre: prefix sums of the horizontal (column) and
   // vertical (row) edit costs over the column and row trees: insertions and
@@ -156,10 +402,11 @@ __global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
   // table's last, by leaf rank), at index wb the boundary value F[R][cmax]
   // that tree columns read, the kds imports (W > 1) and a sink that columns
   // saving nothing write.
-  const int32_t lbase0 = dsc.lbase;
-  const int32_t ltop = lrankC[cmax - 1];
+  const int32_t ltop = lrankC[max(cmax - 1 - tb0, c0)];  // (kXL) of the block's columns
+  int32_t lbase0 = dsc.lbase;
+  if constexpr (kXL) lbase0 = lrankC[max(cmax - tb0 - 64 * W * C - 1, c0)];
   int32_t lbase = lbase0, wb = ltop - lbase0, seg = 0, kds = 0, kdep_c0 = 0;
-  if constexpr (W > 1) {
+  if constexpr (kEdges) {
     const int32_t chi = max(cmax - 1 - tb, c0);
     const int32_t clo = max(c0, cmax - tb - 64 * C);
     const int32_t lhi = lrankC[chi];
@@ -169,25 +416,39 @@ __global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
     kdep_c0 = A.pool.kdep[offC + c0];
     seg = (ltop - lhi) + wave * (2 + kds);
   }
-  const uint32_t entry_bytes = W > 1 ? 4u * (uint32_t)(kds + 2) : 0u;
+  const uint32_t entry_bytes = kEdges ? 4u * (uint32_t)(kds + 2) : 0u;
   const uint32_t edge_bytes = D * entry_bytes;
-  constexpr uint32_t edges = W > 1 ? 8u * (W + 2) : 0u;  // byte offset of edge 0
-  const uint32_t slot_base = edges + (W > 1 ? (W + 1) * edge_bytes : 0u) + 2u * (uint32_t)seg;
+  constexpr uint32_t edges = kEdges ? 8u * (W + 2) : 0u;  // byte offset of edge 0
+  const uint32_t slot_base = edges + (kEdges ? (W + 1) * edge_bytes : 0u) + 2u * (uint32_t)seg;
   const uint32_t row_bytes = 2u * (uint32_t)((ltop - lbase0) + W * (2 + kds));
   const int32_t sinkix = wb + 1 + kds;
   auto l16 = [&](uint32_t byte) -> uint16_t& { return *reinterpret_cast<uint16_t*>(lds + byte); };
   auto l32 = [&](uint32_t byte) -> int32_t& { return *reinterpret_cast<int32_t*>(lds + byte); };
   auto prog = [&](int w) { return reinterpret_cast<unsigned long long*>(lds + 8 * w); };
-  if constexpr (W > 1) {
+  if constexpr (kEdges) {
     if (threadIdx.x < D) l32(edges + threadIdx.x * entry_bytes) = cin0;
     if (threadIdx.x < W + 2) {
       const int w = (int)threadIdx.x - 1;
-      *prog((int)threadIdx.x) = w < 0 || w >= nw ? 0x7FFFFFFF7FFFFFFFull : 0ull;
+      const bool open = w < 0 ? blk == 0 : w >= nw && blk + 1 == nb;  // holds nobody up
+      *prog((int)threadIdx.x) = open ? 0x7FFFFFFF7FFFFFFFull : 0ull;
     }
     __syncthreads();
+    if constexpr (kXL) {
+      if (wave >= W) {
+        XLEdge x{rrecR, A.pool.lrank + offR, r0, rmax, nrows, kds, nb, blk, ix,
+                 nrows <= A.xl_seq_rows, A.xl_words + A.xl_off[ix], edges, entry_bytes};
+        if (wave == W && blk > 0) {
+          edge_in<D, kSync>(A, x, lds, lane);
+        } else if (wave > W && blk + 1 < nb) {
+          x.edge = edges + W * edge_bytes;
+          edge_out<D, kSync>(A, x, lds, W, lane);
+        }
+        return;
+      }
+    }
     if (wave >= nw) return;
   }
-  const bool more = W > 1 && wave + 1 < nw;
+  const bool more = kEdges && (wave + 1 < nw || blk + 1 < nb);
 
   // Per-column state, element e (t = tlane + e, c = cmax-1-t).
   //   tcol: a tree column (orl_C(c) == orl_C(c0));
@@ -196,7 +457,7 @@ __global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
   //   foff: byte offset of the column's far value in this wave's segment;
   //   woff: byte offset it is saved at (c-1 a leaf of subtree(c0)), or the
   //         sink;
-  //   xoff: (W > 1) byte offset in an edge entry: for a saved column whose
+  //   xoff: (edges) byte offset in an edge entry: for a saved column whose
   //         right path's top keyroot lies in a later block the import word of
   //         the path's depth, else the trash word;
   //   Am:   the running minima A[t], shifted by T = tlane with unit costs
@@ -211,7 +472,7 @@ __global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
   uint32_t foff[C], woff[C];
   uint32_t tdq[S][NW];
   int32_t negt[kCost ? C : 1];
-  uint32_t xoff[W > 1 ? C : 1];
+  uint32_t xoff[kEdges ? C : 1];
   auto term = [&](int e) -> int32_t {
     if constexpr (kCost) return negt[e];
     else return -e;
@@ -224,14 +485,14 @@ __global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
   constexpr int B = C < 8 ? C : 8;
 #pragma unroll
   for (int e0 = 0; e0 < C; e0 += B) {
-    NodeRec cl[B], rl[W > 1 ? B : 1];  // as a table column; (W > 1) as a row: kdep of c and c-1
-    int32_t ul[W > 1 ? B : 1];         // (W > 1) the keyroot at the top of c-1's right path
+    NodeRec cl[B], rl[kEdges ? B : 1];  // as a table column; (edges) as a row: kdep of c and c-1
+    int32_t ul[kEdges ? B : 1];         // (edges) the keyroot at the top of c-1's right path
     CostRec ll[kCost ? B : 1];
 #pragma unroll
     for (int b = 0; b < B; ++b) {
       const int32_t c = max(cmax - 1 - (tlane + e0 + b), c0);
       cl[b] = crecC[c];
-      if constexpr (W > 1) {
+      if constexpr (kEdges) {
         rl[b] = A.pool.rrec[offC + c];
         ul[b] = A.pool.rtop[offC + max(c - 1, c0)];
       }
@@ -241,7 +502,7 @@ __global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
     for (int b = 0; b < B; ++b) {
       const int e = e0 + b;
       asm volatile("" : "+v"(cl[b].orl), "+v"(cl[b].label), "+v"(cl[b].x), "+v"(cl[b].y));
-      if constexpr (W > 1) asm volatile("" : "+v"(rl[b].x), "+v"(rl[b].y), "+v"(ul[b]));
+      if constexpr (kEdges) asm volatile("" : "+v"(rl[b].x), "+v"(rl[b].y), "+v"(ul[b]));
       if constexpr (kCost)
         asm volatile("" : "+v"(ll[b].del), "+v"(ll[b].ins), "+v"(ll[b].del_end),
                      "+v"(ll[b].ins_end));
@@ -267,7 +528,7 @@ __global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
       lb[e] = tree ? cr.label : kCost ? hc - hfar : cmax - oc - 1;
       const bool writes = (t < ncols) & (c > c0) & (cr.y < 0);
       int32_t fi = tree ? wb : cr.x - lbase;
-      if constexpr (W > 1) {
+      if constexpr (kEdges) {
         const NodeRec rr = rl[b];  // x, y: kdep of c and of c-1
         if (!tree & (cmax - 2 - oc < tb)) fi = wb + 1 + (rr.x - kdep_c0);
         const int32_t u = ul[b];
@@ -374,7 +635,7 @@ __global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
   // coordinates of the diagonal term (see the tree rows).
   int32_t qleft = tb - 2;
   if constexpr (kCost) qleft = hq - Hpre[max(cmax - tb, c0)];
-  // (W > 1) Lane l takes word l of an edge entry: the carry, then imports.
+  // (edges) Lane l takes word l of an edge entry: the carry, then imports.
   // The boundary value stands before the imports in the segment, so the same
   // lanes write the row's boundary value (lane 0) and imports to its slots;
   // on the outgoing entry lane 63, whose prefix minimum is the block's, writes
@@ -385,7 +646,7 @@ __global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
   const uint32_t eout = xout + 4u * (uint32_t)(lane == 0 ? kds + 1 : lane == 63 ? 0 : word);
   const uint32_t seg_imp = slot_base + 2u * (uint32_t)(wb + word);
   uint32_t qoff = 0;  // (q % D) * entry_bytes
-  int poll_limit = kEdgePolls;
+  Patience pat;
 
   // Rows go S at a time in one flat loop with the inner loop fully unrolled,
   // so row k of the table always uses ring slot k % S and every slot index is
@@ -410,10 +671,10 @@ __global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
       // Rows past the table's end: skipped where a row costs more than the
       // branch, else run as plain rows up to the next even one.
       if ((C < 8 && u % 2 == 1) || __builtin_expect(k < nrows, 1)) {
-        if constexpr (W > 1) {
-          if (u % kSyncRows == 0) {
+        if constexpr (kEdges) {
+          if (u % kSync == 0) {
             // This group's entries are there, and its full rows (at most
-            // kSyncRows) find room in the outgoing ring.
+            // kSync) find room in the outgoing ring.
             for (int n = 0;; ++n) {
               const unsigned long long pb = __hip_atomic_load(prog(wave), __ATOMIC_RELAXED,
                                                               __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -422,14 +683,8 @@ __global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
               const int32_t rows_before = __builtin_amdgcn_readfirstlane((int32_t)(uint32_t)pb);
               const int32_t full_after =
                   __builtin_amdgcn_readfirstlane((int32_t)(uint32_t)(pa >> 32));
-              if (__builtin_expect((rows_before > k) & (full_after >= q - kSyncRows), 1)) break;
-              if (n >= poll_limit) {  // raise the abort flag and wait no more
-                A.xl_abort[2] = (int32_t)ix;
-                A.xl_abort[3] = (2 << 24) | k;
-                (void)atomicExch(A.xl_abort, 1);
-                poll_limit = 0;
-                break;
-              }
+              if (__builtin_expect((rows_before > k) & (full_after >= q - kSync), 1)) break;
+              if (!pat.wait(n, A.xl_abort, ix, (2 << 24) | k)) break;
             }
             lds_order();
           }
@@ -445,7 +700,7 @@ __global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
         }
         // The edge entry of the next full row: this one's, if it is full.
         int32_t edge = 0;
-        if constexpr (W > 1) edge = l32(ein + qoff);
+        if constexpr (kEdges) edge = l32(ein + qoff);
         // Terms of a plain row: far value + TD. (A tree row computes them too,
         // from slot row 0, and replaces them: kept out of an else of the branch
         // below, the common path has no taken branch. With the terms skipped on
@@ -462,7 +717,7 @@ __global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
             d[e] = sv[e] + tdv(u, e) + (term(e) - vk);
             asm volatile("" : "+v"(d[e]));
           }
-          if constexpr (W > 1) asm volatile("" : "+v"(edge));
+          if constexpr (kEdges) asm volatile("" : "+v"(edge));
         }
         if (__builtin_expect((fw & kRowTree) != 0, 0)) {
           // Tree columns: the diagonal F[r+1][c+1] + rename (the row below is
@@ -499,12 +754,12 @@ __global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
 #pragma unroll
           for (int e = 1; e < C; ++e) Am[e] = min(Am[e], Am[e - 1]);
           int32_t x = Am[C - 1] - T;
-          if constexpr (W > 1) {
+          if constexpr (kEdges) {
             x = min(x, lane == 0 ? edge : kBig);
             cin = edge;
           }
           const int32_t incl = wave_incl_min(x);
-          const int32_t cg = wave_shr1(incl, W > 1 ? edge : kBig) + T;
+          const int32_t cg = wave_shr1(incl, kEdges ? edge : kBig) + T;
 #pragma unroll
           for (int e = 0; e < C; ++e) Am[e] = min(Am[e], cg);
           // Row values, and F[r][cmax]: the summed row costs (rmax - r = k + 1
@@ -517,7 +772,7 @@ __global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
             const uint32_t wbase = (uint32_t)__builtin_amdgcn_readlane(mwr, i);
 #pragma unroll
             for (int e = 0; e < C; ++e) l16(woff[e] + wbase) = (uint16_t)v[e];
-            if constexpr (W > 1) {
+            if constexpr (kEdges) {
               l16(seg_imp + wbase) = (uint16_t)(lane == 0 ? frc : edge);
               if (__builtin_expect(kds >= 63, 0)) {
                 for (int d0 = 63; d0 <= kds; d0 += 64) {
@@ -531,7 +786,7 @@ __global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
               l16(slot_base + wbase + 2u * wb) = (uint16_t)frc;
             }
           }
-          if constexpr (W > 1) {
+          if constexpr (kEdges) {
             // Imports pass on; then a path that starts in this block replaces
             // one of the same depth that ended in it. (Only a saved row's
             // entry is read beyond its carry.)
@@ -540,7 +795,7 @@ __global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
 #pragma unroll
             for (int e = 0; e < C; ++e) l32(xout + qoff + xoff[e]) = v[e];
           }
-          if constexpr (W > 1) {
+          if constexpr (kEdges) {
             ++q;
             qoff += entry_bytes;
             if (qoff == edge_bytes) qoff = 0;
@@ -573,8 +828,8 @@ __global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
           }
         }
       }  // k < nrows
-      if constexpr (W > 1) {
-        if (u % kSyncRows == kSyncRows - 1) {
+      if constexpr (kEdges) {
+        if (u % kSync == kSync - 1) {
           lds_order();
           __hip_atomic_store(prog(wave + 1),
                              ((unsigned long long)(uint32_t)q << 32) | (uint32_t)(k + 1),
@@ -584,6 +839,46 @@ __global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
       }
     }
   }
+}
+
+template <int W, int C, bool kCost>
+__global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
+  // Workgroups go round robin over the 8 XCDs, each with its own L2; task
+  // order keeps a pair's tables together, so kXcdRun consecutive tasks are
+  // given to one XCD (the last, partial span keeps its order). The 4096-pair
+  // batch ran 101.6 ms without, 100.1 with 16, 101.0 with 64, 104.8 with 256.
+  constexpr uint32_t kXcds = 8, kXcdRun = 16, kSpan = kXcds * kXcdRun;
+  uint32_t ix = blockIdx.x;
+  if ((ix | (kSpan - 1)) < (uint64_t)A.ntasks)
+    ix = (ix & ~(kSpan - 1)) + (ix % kXcds) * kXcdRun + (ix % kSpan) / kXcds;
+  if ((int64_t)ix >= A.ntasks) return;
+  scan_block<W, C, kCost, false>(A, A.descs[ix], (int32_t)ix, 0, 1);
+}
+
+// Column-blocked: W waves of C columns per lane and the two edge waves.
+template <int W, int C, bool kCost>
+__global__ __launch_bounds__(64 * (W + 2)) void scan_xl_kernel(DPArgs A) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  if (threadIdx.x == 0) *reinterpret_cast<uint32_t*>(lds) = atomicAdd(A.xl_ticket, 1u);
+  __syncthreads();
+  const int32_t ticket = __builtin_amdgcn_readfirstlane(*reinterpret_cast<int32_t*>(lds));
+  const int32_t ix = ticket / A.xl_nbmax;
+  int32_t blk = ticket % A.xl_nbmax;
+  if ((int64_t)ix >= A.ntasks) return;
+  const int32_t ncols = A.descs[ix].cmax - A.descs[ix].c0;
+  const int32_t nrows = A.descs[ix].rmax - A.descs[ix].r0;
+  const int32_t nb = (ncols + 64 * W * C - 1) / (64 * W * C);
+  const bool seq = nrows <= A.xl_seq_rows;
+  if (blk >= nb || (seq && blk > 0)) return;
+  do {
+    __syncthreads();  // the LDS of the block before (or the ticket) is read
+    // The task's index is made opaque for each block: what a block derives from
+    // its descriptor would otherwise be kept in registers over the blocks (50
+    // of them, and the widest form would spill).
+    int32_t ib = ix;
+    asm volatile("" : "+s"(ib));
+    scan_block<W, C, kCost, true>(A, A.descs[ib], ib, blk, nb);
+  } while (seq && ++blk < nb);
 }
 
 // ---------------------------------------------------------------------------
@@ -618,6 +913,36 @@ static void launch_c(int ci, const DPArgs& a, int lds, hipStream_t s) {
   }
 }
 
+template <int W, int C>
+static void launch_xl_one(const DPArgs& a, int lds_bytes, hipStream_t s) {
+  // Workgroups take (task, block) tickets from one counter that the pieces
+  // of a long launch share: a later piece continues where the earlier one
+  // stopped, and every block it waits on holds a lower ticket, taken by a
+  // workgroup of an earlier (finished) piece or a running one of its own.
+  constexpr int64_t kChunk = kGridThreads / (64 * (W + 2));
+  const int64_t total = a.ntasks * a.xl_nbmax;
+  for (int64_t off = 0; off < total; off += kChunk) {
+    const dim3 grid((unsigned)std::min(kChunk, total - off));
+    if (a.costs)
+      hipLaunchKernelGGL((scan_xl_kernel<W, C, true>), grid, dim3(64 * (W + 2)),
+                         (size_t)lds_bytes, s, a);
+    else
+      hipLaunchKernelGGL((scan_xl_kernel<W, C, false>), grid, dim3(64 * (W + 2)),
+                         (size_t)lds_bytes, s, a);
+  }
+}
+
+void launch_xl(int form, const DPArgs& a, int lds_bytes, hipStream_t s) {
+  switch (form) {  // must match xl_waves / xl_cpl
+    case 0: launch_xl_one<8, 8>(a, lds_bytes, s); break;
+    case 1: launch_xl_one<8, 4>(a, lds_bytes, s); break;
+    case 2: launch_xl_one<4, 4>(a, lds_bytes, s); break;
+    case 3: launch_xl_one<1, 8>(a, lds_bytes, s); break;
+    case 4: launch_xl_one<1, 4>(a, lds_bytes, s); break;
+    default: launch_xl_one<1, 2>(a, lds_bytes, s); break;
+  }
+}
+
 void launch_scan(int wi, int ci, const DPArgs& a, int lds_bytes, hipStream_t s) {
   switch (wi) {
     case 0: launch_c<1>(ci, a, lds_bytes, s); break;
@@ -648,8 +973,24 @@ static hipError_t allow_c(int limit) {
   if ((e = allow<W, 8>(limit)) != hipSuccess) return e;
   return allow<W, 16>(limit);
 }
+template <int W, int C>
+static hipError_t allow_xl(int limit) {
+  const hipError_t e =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&scan_xl_kernel<W, C, false>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, limit);
+  if (e != hipSuccess) return e;
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(&scan_xl_kernel<W, C, true>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, limit);
+}
 hipError_t scan_init_attributes(int limit) {
   hipError_t e;
+  const int xl_limit = limit + kXLEdgeBytes;
+  if ((e = allow_xl<8, 8>(xl_limit)) != hipSuccess) return e;
+  if ((e = allow_xl<8, 4>(xl_limit)) != hipSuccess) return e;
+  if ((e = allow_xl<4, 4>(xl_limit)) != hipSuccess) return e;
+  if ((e = allow_xl<1, 8>(xl_limit)) != hipSuccess) return e;
+  if ((e = allow_xl<1, 4>(xl_limit)) != hipSuccess) return e;
+  if ((e = allow_xl<1, 2>(xl_limit)) != hipSuccess) return e;
   if ((e = allow_c<1>(limit)) != hipSuccess) return e;
   if ((e = allow_c<2>(limit)) != hipSuccess) return e;
   if ((e = allow_c<4>(limit)) != hipSuccess) return e;

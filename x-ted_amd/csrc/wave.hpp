@@ -36,9 +36,6 @@ __device__ __forceinline__ int wave_shr1(int v, int fill) {
 // Words of a TD row group: 2, 4 or 8 entries of 16 bits (td_t), two to a
 // 32-bit word, at any even byte address (the target's unaligned-access mode
 // lets one dwordx2 / dwordx4 load read them).
-typedef uint32_t u32x4a2 __attribute__((ext_vector_type(4), aligned(2)));
-typedef uint32_t u32x2a2 __attribute__((ext_vector_type(2), aligned(2)));
-typedef uint32_t u32x1a2 __attribute__((aligned(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // Word 3 of a raw buffer resource on CDNA (32-bit data format, no swizzle).
