@@ -133,6 +133,7 @@ XTED_HD inline uint32_t task_j0(uint64_t t) { return (uint32_t)t & 0x7FFFFu; }
 // Classes 36..38: on-chip tables of deep column keyroots, whose waves' imports
 //   do not fit LDS beside the slot rows: slot rows shared by 4, 8 or 16 waves,
 //   with a barrier per row.
+// Class 39: tables swept by one wave, kSweepCols columns at a time.
 constexpr int kClassLane = 0;  // the leaf class
 constexpr int kNumRowClasses = 25;
 constexpr int kClassXL = 26;
@@ -142,20 +143,23 @@ constexpr int kClassTiny = kFirstXLClass + kNumXLForms;  // 33: the first tiny f
 constexpr int kNumTinyForms = 3;
 constexpr int kClassShared = kClassTiny + kNumTinyForms;  // 36: the first shared-slot form
 constexpr int kNumSharedForms = 3;
-constexpr int kNumClasses = kClassShared + kNumSharedForms;  // 39
+constexpr int kSweepForm = 3;  // column-blocked form of the same width
+constexpr int kClassSweep = kClassShared + kNumSharedForms;  // 39
+constexpr int kSweepCols = 512;
+constexpr int kNumClasses = kClassSweep + 1;  // 40
 XTED_HD inline bool is_tiny(int cls) { return cls >= kClassTiny && cls < kClassShared; }
-XTED_HD inline bool is_shared(int cls) { return cls >= kClassShared && cls < kNumClasses; }
+XTED_HD inline bool is_shared(int cls) { return cls >= kClassShared && cls < kClassSweep; }
 // Shared-slot form k: 4, 8 or 16 waves of 8 columns per lane.
 XTED_HD inline int shared_cols(int k) { return 64 * 8 * (4 << k); }
 // Lanes per table (and most columns) of tiny form k.
 XTED_HD inline int tiny_seg(int k) { return 16 << k; }
 // Slot bytes of one table of tiny form k: 32 KiB per workgroup of 256 lanes.
 XTED_HD inline int64_t tiny_max_lds(int k) { return (int64_t)2048 << k; }
-// Column-blocked forms: waves and columns per lane of one block. The narrow
-// forms serve deep trees, whose slot rows leave little LDS: one wave's edges
-// take the least.
-XTED_HD inline int xl_waves(int k) { return k <= 1 ? 8 : k == 2 ? 4 : 1; }
-XTED_HD inline int xl_cpl(int k) { return k == 0 || k == 3 ? 8 : k == 5 ? 2 : 4; }
+// Column-blocked forms: waves and columns per lane of one block. The two
+// narrowest serve deep trees, whose slot rows leave little LDS: one wave's
+// edges take the least.
+XTED_HD constexpr int xl_waves(int k) { return k <= 2 ? 8 : k == 3 ? 4 : 1; }
+XTED_HD constexpr int xl_cpl(int k) { return k == 0 ? 8 : k == 1 || k == 4 ? 4 : 2; }
 XTED_HD inline int xl_bw(int k) { return 64 * xl_waves(k) * xl_cpl(k); }  // 4096 .. 128
 // Column-blocked tables with at most this many rows are swept block after
 // block by one workgroup (forms of at most 1024 columns), with no waits
@@ -191,9 +195,10 @@ XTED_HD inline int size_band(int cls, int rows, int64_t lds, int mode, int light
     const int q = tiny_seg(cls - kClassTiny) / 4;  // row bands of a quarter segment
     return rows > 3 * q ? 0 : rows > 2 * q ? 1 : rows > q ? 2 : 3;
   }
-  if (cls < 1 || cls > kNumRowClasses) return 0;
+  if ((cls < 1 || cls > kNumRowClasses) && cls != kClassSweep) return 0;
   const int rb = rows >= 256 ? 0 : rows >= 64 ? 1 : rows >= 16 ? 2 : 3;
-  const int64_t light = (int64_t)(1 << ((cls - 1) / 5)) * light_per_wave;
+  const int waves = cls == kClassSweep ? 1 : 1 << ((cls - 1) / 5);
+  const int64_t light = (int64_t)waves * light_per_wave;
   return mode == 2 && lds > light ? kRowBands + rb : rb;
 }
 XTED_HD inline int bucket_of(int level, int cls, int band) {
@@ -223,6 +228,32 @@ constexpr int32_t kTinyDefault = 1;
 // Most columns per lane a table takes under a cost model.
 constexpr int32_t kMaxCostCpl = 8;
 
+// A row of up to 256 columns takes one wave about as long as several
+// (a 120-node pair's root table 0.21 us a row either way).
+constexpr int32_t kTallCols = 256;
+
+// How a table is split, by its level's interior cells (level_cells_kernel). A
+// level takes the longer of its work spread over the chip and its slowest
+// table's rows, one after another. A table whose rows take longer than the
+// level's work ("tall": few cells in the level per row of its own) is split
+// for speed: fewer columns a lane, and past a block's width a pipeline of
+// workgroups, since a row takes the less the fewer columns a lane holds and
+// waves a compute unit has (1000 columns: 0.38 us with 16 a lane, 0.32 with 8,
+// 0.24 with 4, 0.21 with 2; 4000: 0.39 in one workgroup of 16 waves, 0.45 /
+// 0.32 / 0.27 / 0.26 in blocks of 4096 / 2048 / 1024 / 512). The others are
+// split for throughput. Measured in ms with the bound for 2 columns a lane at
+// 4e4, 1.2e5, 4e5 cells: 20,000-node pair 93, 91, 91; deep 1000-node pair 7.9,
+// 7.7, 7.6; 128 pairs of 100-600 nodes 20.4, 20.8, 20.1. With the bound for 4
+// at 3e5, 1.5e6, 3e6, 1e7: 20,000-node pair 94, 91, 91, 87; 1024 pairs of
+// 100-1000 nodes under a cost model 64, 57, 55, 55; 4096 such pairs with unit
+// costs 90, 90, 90, 98.
+constexpr int64_t kTall2Cells = 120000;
+constexpr int64_t kTall4Cells = 3000000;
+constexpr int kTallRows = 64;
+constexpr int64_t kSweepShare = 1024;
+constexpr int kSweepLds = 20 * 1024;
+constexpr int kTall2Form = 2, kTall4Form = 1;
+
 // Tuning knobs carried by the plan builder (autotuner writes these).
 struct ClassRule {
   int32_t lds_per_wave;  // bytes of slot storage one wave may own
@@ -238,33 +269,14 @@ struct ClassRule {
   // blocks, 1: 2048, 2: 1024, ...): narrower blocks put more workgroups on
   // one table.
   int32_t xl_first = 0;
-  // Tables of at least tall_rows rows and more than kTallCols columns take at
-  // most tall_cpl columns per lane (set_tall).
-  int32_t tall_rows = 1 << 30;
-  int32_t tall_cpl = 16;
+  // Tall tables: those of at least kTallRows rows and more than kTallCols
+  // columns in a level of at most tall2 (tall4) cells per row of theirs take
+  // at most 2 (4) columns per lane, and where blocks is set go in blocks of at
+  // most form kTall2Form (kTall4Form).
+  int64_t tall2 = kTall2Cells, tall4 = kTall4Cells;
+  int64_t sweep = kSweepShare;
+  int32_t blocks = 1;
 };
-// A row of up to 256 columns takes one wave about as long as several
-// (a 120-node pair's root table 0.21 us a row either way).
-constexpr int32_t kTallCols = 256;
-
-// How tall tables are split, by the interior cells of the whole plan. A plan
-// of few cells waits for its largest tables, one after another along the
-// levels, and a row of a table takes the less the fewer columns a lane holds
-// (1000 columns: 0.38 us with 16, 0.32 with 8, 0.24 with 4, 0.21 with 2); a
-// plan of many fills the device, and more waves per table only add their rows'
-// fixed instructions. Measured, ms, without the rule and with tall_rows 64 and
-// 4 or 2 columns: a deep 1000-node pair (2.6e8 cells) 11.3, 8.4, 7.7; 128
-// pairs of 100-600 nodes (9.6e8) 23.5, 20.8, 20.2; 1024 pairs of 100-1000
-// nodes under a cost model (3.7e10) 67, 55, 61; 4096 such pairs with unit costs
-// (1.4e11) 93, 111, 143.
-constexpr int64_t kTall2Cells = 4000000000ll;
-constexpr int64_t kTall4Cells = 80000000000ll;
-XTED_HD inline void set_tall(ClassRule& rule, int64_t cells) {
-  if (cells > kTall4Cells) return;
-  rule.tall_rows = 64;
-  rule.tall_cpl = cells <= kTall2Cells ? 2 : 4;
-}
-
 XTED_HD inline int ilog2_ceil(int v) {
   int r = 0;
   while ((1 << r) < v) ++r;
@@ -285,35 +297,48 @@ XTED_HD inline int64_t scan_lds_need(int slots, int leaves_c, int kd_c, int w) {
          (int64_t)(w + 1) * kEdgeRows * (kd_c + 3) * 4 + 8 * (w + 2);
 }
 
-// The same of one block of a column-blocked table, whose own far columns are
-// at most bw, with edges of shorter rings on the narrow forms.
-XTED_HD constexpr int xl_edge_rows(int cols_per_lane) { return cols_per_lane <= 8 ? 4 : 8; }
-XTED_HD inline int64_t xl_lds_need(int kd_r, int kd_c, int leaves_c, int k) {
-  const int w = xl_waves(k), bw = xl_bw(k);
-  const int own = leaves_c < bw ? leaves_c : bw;
-  return (int64_t)(kd_r > 1 ? kd_r : 1) * (own + w * (kd_c + 3)) * 2 +
-         (int64_t)(w + 1) * xl_edge_rows(w * xl_cpl(k)) * (kd_c + 3) * 4 + 8 * (w + 2);
+// The same of one block of a column-blocked table of form k, whose blocks
+// have at most own far columns of their own each.
+XTED_HD constexpr int xl_edge_rows(int w) { return w == 1 ? 4 : kEdgeRows; }
+XTED_HD inline int64_t xl_lds_need(int slots, int own, int kd_c, int k) {
+  const int w = xl_waves(k);
+  return (int64_t)slots * (own + w * (kd_c + 3)) * 2 +
+         (int64_t)(w + 1) * xl_edge_rows(w) * (kd_c + 3) * 4 + 8 * (w + 2);
+}
+// The same of a swept table (kClassSweep) of that many rows: the slot rows of
+// one block, and one edge entry per row.
+XTED_HD inline int64_t sweep_lds_need(int slots, int own, int kd_c, int rows) {
+  return (int64_t)slots * (own + kd_c + 3) * 2 + (int64_t)(rows + 1) * (kd_c + 3) * 4;
 }
 // Which of these forms, from form k on, takes a table: the widest whose blocks
-// fit lds_max. A table the narrowest form's slot rows fit is never refused:
-// its edges, at most kXLEdgeBytes, come on top of lds_max (a workgroup may
-// have 160 KiB). -1: none. *need receives the form's bytes.
-constexpr int kXLEdgeBytes = 2 * 4 * (kMaxImports + 2) * 4 + 8 * 3;
-XTED_HD inline int xl_form(int kd_r, int kd_c, int leaves_c, int k, int lds_max, int64_t* need) {
-  if (kd_c + 1 > kMaxImports) return -1;
-  for (; k < kNumXLForms; ++k) {
-    *need = xl_lds_need(kd_r, kd_c, leaves_c, k);
-    if (*need <= lds_max + (k == kNumXLForms - 1 ? 8 * (kd_c + 3) * 4 + 24 : 0)) return k;
+// fit lds_max; the narrowest takes every table whose slot rows fit it by the
+// bound min(leaves, columns) on a block's far columns, its edges (at most
+// kXLEdgeBytes) coming on top of lds_max (a workgroup may have 160 KiB). -1:
+// none. own(k): the most far columns of any one block of form k. *need
+// receives the form's bytes.
+constexpr int kXLEdgeBytes = 2 * xl_edge_rows(1) * (kMaxImports + 2) * 4 + 8 * 3;
+template <class Own>
+XTED_HD inline int xl_form(int slots, int kd_c, int leaves_c, int k, int lds_max, const Own& own,
+                           int64_t* need) {
+  constexpr int kLast = kNumXLForms - 1;
+  const int most = leaves_c < xl_bw(kLast) ? leaves_c : xl_bw(kLast);
+  if (kd_c + 1 > kMaxImports || (int64_t)slots * (most + kd_c + 3) * 2 > lds_max) return -1;
+  for (; k < kLast; ++k) {
+    *need = xl_lds_need(slots, own(k), kd_c, k);
+    if (*need <= lds_max) return k;
   }
-  return -1;
+  *need = xl_lds_need(slots, most, kd_c, kLast);
+  return kLast;
 }
 
 // Class of table (a x b): kd_r / kd_c / leaves_c (row keyroot height, column
-// keyroot height and leaves) of its oriented form size its LDS storage. Single-row tables are
-// the leaf class when leaf_form is set. *need receives the slot bytes of the
-// chosen form.
+// keyroot height and leaves) of its oriented form size its LDS storage, with
+// own (xl_form) as blocks; level_cells(): the interior cells of its level. Single-row tables are the leaf class when leaf_form
+// is set. *need receives the slot bytes of the chosen form.
+template <class Cells, class Own>
 XTED_HD inline int table_class(int a, int b, int kd_r, int kd_c, int leaves_c, bool leaf_form,
-                               const ClassRule& rule, int64_t* need) {
+                               const ClassRule& rule, const Cells& level_cells, const Own& own,
+                               int64_t* need) {
   const int rows = a <= b ? a : b;
   const int cols = a <= b ? b : a;
   const int slots = kd_r > 1 ? kd_r : 1;
@@ -327,8 +352,18 @@ XTED_HD inline int table_class(int a, int b, int kd_r, int kd_c, int leaves_c, b
   int wi = 0;
   while (wi < 4 && lds_need > (int64_t)rule.lds_per_wave * (1 << wi)) ++wi;
   while (wi < 4 && cols > 64 * rule.max_cpl * (1 << wi)) ++wi;
-  if (rows >= rule.tall_rows && cols > kTallCols) {
-    while (wi < 4 && cols > 64 * rule.tall_cpl * (1 << wi)) ++wi;
+  int tall = 0;
+  const int64_t cells = cols > kTallCols ? level_cells() : 0;
+  if (rows >= kTallRows && cols > kTallCols) {
+    tall = cells <= rows * rule.tall2 ? 2 : cells <= rows * rule.tall4 ? 4 : 0;
+    while (tall && wi < 4 && cols > 64 * tall * (1 << wi)) ++wi;
+  }
+  if (!tall && wi > 0 && cols > 2 * kSweepCols && cells >= (int64_t)rows * cols * rule.sweep) {
+    const int64_t n = sweep_lds_need(slots, own(kSweepForm), kd_c, rows);
+    if (n <= kSweepLds && n <= rule.lds_max) {
+      *need = n;
+      return kClassSweep;
+    }
   }
   if (cols >= rule.wide_cols) {
     while (wi < 4 && (1 << wi) < rule.min_waves) ++wi;
@@ -337,6 +372,19 @@ XTED_HD inline int table_class(int a, int b, int kd_r, int kd_c, int leaves_c, b
   while (wi > 0 && scan_lds_need(slots, leaves_c, kd_c, 1 << wi) > rule.lds_max &&
          cols <= 64 * 16 * (1 << (wi - 1)))
     --wi;
+  const int first_tall = tall == 2 ? kTall2Form : tall == 4 ? kTall4Form : 0;
+  const int first = rule.xl_first > first_tall ? rule.xl_first : first_tall;
+  auto blocked = [&](int k) {
+    const int form = xl_form(slots, kd_c, leaves_c, k, rule.lds_max, own, need);
+    return form < 0 ? kClassXL : kFirstXLClass + form;
+  };
+  // Tall tables go in blocks where they are wider than one, and where LDS
+  // leaves them more columns per lane.
+  if (tall && rule.blocks && rows > rule.xl_seq_rows &&
+      (cols > xl_bw(first_tall) || cols > 64 * tall * (1 << wi))) {
+    const int cls = blocked(first);
+    if (cls != kClassXL) return cls;
+  }
   *need = scan_lds_need(slots, leaves_c, kd_c, 1 << wi);
   if (*need > rule.lds_max && lds_need <= rule.lds_max) {
     for (int k = 0; k < kNumSharedForms; ++k) {
@@ -346,13 +394,9 @@ XTED_HD inline int table_class(int a, int b, int kd_r, int kd_c, int leaves_c, b
       }
     }
   }
-  if (cols > 64 * cpl_cap * kMaxRowWaves || *need > rule.lds_max) {
-    // Short tables take the forms one workgroup sweeps.
-    const int k = xl_form(kd_r, kd_c, leaves_c,
-                          rows <= rule.xl_seq_rows ? kFirstSeqXLForm : rule.xl_first,
-                          rule.lds_max, need);
-    return k < 0 ? kClassXL : kFirstXLClass + k;
-  }
+  // Short tables take the forms one workgroup sweeps.
+  if (cols > 64 * cpl_cap * kMaxRowWaves || *need > rule.lds_max)
+    return blocked(rows <= rule.xl_seq_rows ? kFirstSeqXLForm : first);
   int w = 1 << wi;
   int c = (cols + 64 * w - 1) / (64 * w);
   int ci = ilog2_ceil(c);

@@ -548,7 +548,7 @@ int Context::plan(Group& g, int32_t npairs, const int32_t* xs, const int32_t* ys
   ST_TRY(g.cursor.grow(sizeof(unsigned long long) * nb, false, ps));
   ST_TRY(g.maxlds.grow(sizeof(int32_t) * nb, false, ps));
   ST_TRY(g.tickets.grow(sizeof(unsigned int) * nb, false, ps));
-  ST_TRY(g.abort.grow(sizeof(int32_t) * kAbortInts, false, ps));
+  ST_TRY(g.abort.grow(sizeof(int32_t) * (kAbortInts + 2), false, ps));
   ST_TRY(g.tasks.grow(sizeof(uint64_t) * std::max<int64_t>(planned, 1), false, ps));
   ST_TRY(g.descs.grow(sizeof(TaskDesc) * std::max<int64_t>(planned, 1), false, ps));
   ST_TRY(g.td.grow((size_t)g.td_bytes, false, ps));
@@ -598,11 +598,19 @@ int Context::plan(Group& g, int32_t npairs, const int32_t* xs, const int32_t* ys
   // SIMD): under a cost model a table gets more waves instead (the 4096-pair
   // batch under a cost model ran 125.5 ms against 131.3 with up to 16).
   if (cost_alphabet_ > 0) pa.rule.max_cpl = std::min(pa.rule.max_cpl, kMaxCostCpl);
-  if (g.maxn <= kMaxOnChipCols) set_tall(pa.rule, st.cells);
   pa.rule_tail = ClassRule{lds_limit, 1, 1 << 30, lds_limit, 16, rule.xl_seq_rows};
   pa.rule_tail.xl_first = rule.xl_first;
   pa.rule_tail.tiny = rule.tiny;
-  if (g.maxn <= kMaxOnChipCols) set_tall(pa.rule_tail, st.cells);
+  pa.mean_cells = st.cells / nlevels;
+  pa.level_cells = nullptr;
+  if (&g == &na_) {
+    // Blocks need words in device memory: the no-allocation array holds those
+    // of the tables that go in no other way.
+    pa.rule.blocks = pa.rule_tail.blocks = 0;
+  } else if (g.maxn > kTallCols) {  // no rule looks at narrower tables' levels
+    ST_TRY(g.level_cells.grow(sizeof(unsigned long long) * nlevels, false, ps));
+    pa.level_cells = g.level_cells.as<unsigned long long>();
+  }
   pa.tail_level = g.tail_lv.as<uint8_t>();
   pa.force_class = force_class;
   pa.bands = size_bands;
@@ -616,6 +624,7 @@ int Context::plan(Group& g, int32_t npairs, const int32_t* xs, const int32_t* ys
   pa.tasks = g.tasks.as<uint64_t>();
   pa.descs = g.descs.as<TaskDesc>();
   pa.tickets = g.tickets.as<unsigned int>();
+  pa.xl_base = g.abort.as<uint32_t>() + kAbortInts;
   pa.abort_flag = g.abort.as<int32_t>();
   launch_plan(pa, blk[npairs], ps);
   HIP_TRY(hipGetLastError());
@@ -782,6 +791,7 @@ int Context::launch_levels(Group* const* gs, int ng, std::vector<ProfLaunch>* pr
       da.xl_abort = g.abort.as<int32_t>();
       da.xl_off = nullptr;
       da.xl_ticket = nullptr;
+      da.xl_base = g.abort.as<uint32_t>() + kAbortInts;
       da.xl_epoch = 0;
       da.xl_nbmax = 1;
       da.xl_seq_rows = rule.xl_seq_rows;
@@ -792,9 +802,7 @@ int Context::launch_levels(Group* const* gs, int ng, std::vector<ProfLaunch>* pr
         const int bw = xl_bw(w.cls - kFirstXLClass);
         da.xl_off = g.xl_off.as<int64_t>() + g.xl_first[w.bucket];
         da.xl_ticket = g.tickets.as<unsigned int>() + w.bucket;
-        // never 0 (a zeroed word) nor 0xFFFFFFFF (the reads' compare value)
-        if (++xl_epoch_ == 0xFFFFFFFFu) xl_epoch_ = 1;
-        da.xl_epoch = xl_epoch_;
+        da.xl_epoch = (uint32_t)(w.level * kNumXLForms + (w.cls - kFirstXLClass));
         da.xl_nbmax = (g.maxn + bw - 1) / bw;
       }
       const int lds = std::max(64, (w.lds + 15) & ~15);
@@ -927,8 +935,10 @@ std::vector<uint64_t> Context::graph_signature(const Group& g, int lane) const {
   s.push_back((uint64_t)g.npairs);
   s.push_back((uint64_t)g.nlevels);
   s.push_back((uint64_t)g.lines[g.npairs]);
-  for (const void* p : {g.pairs.p, g.td.p, g.tasks.p, g.descs.p, g.lines_d.p, g.abort.p})
+  for (const void* p : {g.pairs.p, g.td.p, g.tasks.p, g.descs.p, g.lines_d.p, g.abort.p,
+                        g.tickets.p, g.xl_words.p, g.xl_off.p})
     s.push_back((uint64_t)(uintptr_t)p);
+  s.push_back((uint64_t)g.maxn << 32 | (uint32_t)rule.xl_seq_rows);
   const PoolView v = view();
   const uint64_t* pv = reinterpret_cast<const uint64_t*>(&v);
   s.insert(s.end(), pv, pv + sizeof(PoolView) / sizeof(uint64_t));
@@ -943,7 +953,7 @@ std::vector<uint64_t> Context::graph_signature(const Group& g, int lane) const {
 // All levels of a planned group on its lane: as launches, or as a graph.
 int Context::run_levels(Group& g, int lane, std::vector<ProfLaunch>* prof) {
   Group* one = &g;
-  if (!use_graphs || prof || g.nxl > 0) {
+  if (!use_graphs || prof) {
     while (g.next_level < g.nlevels) {
       const int st = launch_levels(&one, 1, prof, lane);
       if (st != OK) return st;

@@ -98,7 +98,7 @@ struct Group {
   std::vector<int32_t> h_maxlds;
   std::vector<uint8_t> h_tail;
   DevBuf pairs, blk, counts, cells, cursor, maxlds, tickets, tasks, descs, td, dist, lines_d,
-      tail_lv, xl_off, xl_total, loff_d, leaf_d;
+      tail_lv, level_cells, xl_off, xl_total, loff_d, leaf_d;
   DevBuf tdw;  // requested tables widened to int32 on their way out
   DevBuf abort, xl_words;
   // finish_async: distances then the abort flag land in pinned memory
@@ -122,8 +122,8 @@ struct Group {
   template <class F>
   void for_each_buf(F f) {
     for (DevBuf* b : {&pairs, &blk, &counts, &cells, &cursor, &maxlds, &tickets, &abort, &tasks,
-                      &descs, &td, &dist, &lines_d, &tail_lv, &xl_off, &xl_total, &xl_words,
-                      &loff_d, &leaf_d, &tdw})
+                      &descs, &td, &dist, &lines_d, &tail_lv, &level_cells, &xl_off, &xl_total,
+                      &xl_words, &loff_d, &leaf_d, &tdw})
       f(*b);
   }
 };
@@ -304,7 +304,6 @@ class Context {
   // cost model both trees within the cost form's stack.
   bool leaf_form(int32_t x, int32_t y) const;
   LeafArgs leaf_args(const Group& g) const;
-  uint32_t xl_epoch_ = 0;  // tag of the latest column-blocked launch
   std::vector<hipEvent_t> prof_ev_;
   int grow_pool(int64_t nodes);
   int cost_prefix(int32_t first, int32_t ntrees);  // pdel_ / pins_ and totals of those trees

@@ -921,15 +921,18 @@ void launch_tiny(int form, const DPArgs& a, int slot_bytes, hipStream_t s) {
 }
 
 // Arena offsets of every column-blocked task of a batch, in bucket order
-// (level, then form), and their total (one workgroup).
+// (level, then form), and the words of the level that takes most: levels run
+// one after another and every launch has its own epoch, so each starts at
+// offset 0 (one workgroup).
 __global__ __launch_bounds__(1024) void xl_layout_kernel(XLLayoutArgs A) {
   __shared__ unsigned long long part[1024];
   __shared__ unsigned long long run;
   const int tid = threadIdx.x;
-  if (tid == 0) run = 0;
-  __syncthreads();
+  unsigned long long most = 0;
   int64_t ord = 0;
   for (int L = 0; L < A.nlevels; ++L) {
+    if (tid == 0) run = 0;
+    __syncthreads();
     for (int k = 0; k < kNumXLForms; ++k) {
       const int bkt = bucket_of(L, kFirstXLClass + k, 0);
       const int64_t cnt = (int64_t)A.counts[bkt];
@@ -957,8 +960,9 @@ __global__ __launch_bounds__(1024) void xl_layout_kernel(XLLayoutArgs A) {
       }
       ord += cnt;
     }
+    if (tid == 0) most = max(most, run);
   }
-  if (tid == 0) *A.total = run;
+  if (tid == 0) *A.total = most;
 }
 
 void launch_xl_layout(const XLLayoutArgs& a, hipStream_t s) {
@@ -1024,6 +1028,10 @@ bool launch_forest(int cls, const DPArgs& a, int lds_bytes, hipStream_t s) {
   }
   if (cls >= 1 && cls <= kNumRowClasses) {
     launch_scan((cls - 1) / 5, (cls - 1) % 5, a, lds_bytes, s);
+    return true;
+  }
+  if (cls == kClassSweep) {
+    launch_sweep(a, lds_bytes, s);
     return true;
   }
   switch (cls - kClassShared) {

@@ -73,6 +73,10 @@ struct PlanArgs {
   int32_t light_per_wave;      // bands 2: heavier tables take launches of their own
   int32_t lane_enable;         // 0 = single-row tables use the row-scan kernels
   const uint8_t* pair_leaf;    // per pair: its lines are in closed form (null: lane_enable)
+  // Per level: interior cells of the tables that are planned (null: every
+  // level counts mean_cells).
+  unsigned long long* level_cells;
+  int64_t mean_cells;
   unsigned long long* counts;  // per bucket (bucket_of: level, class, band)
   unsigned long long* cells;   // per bucket: interior cells
   unsigned long long* cursor;  // scatter cursors (bucket offsets)
@@ -80,6 +84,8 @@ struct PlanArgs {
   uint64_t* tasks;
   TaskDesc* descs;             // one per task, same order
   unsigned int* tickets;       // per bucket: column-blocked launch counters
+  uint32_t* xl_base;           // tag base of the column-blocked launches (DPArgs::xl_base), and
+                               // the next plan's
   int32_t* abort_flag;         // kAbortInts: column-blocked waits gave up, what they waited for,
                                // and their stale-read / wait counts
 };
@@ -164,7 +170,9 @@ struct DPArgs {
   unsigned int* xl_ticket;       // (task, block) counter of this launch, zeroed
   int32_t* xl_abort;             // [0] raised when a wait gives up, [1..3] what it waited for,
                                  // [8] stale prefetched reads, [9] throttle checks that waited
-  uint32_t xl_epoch;             // tag of this launch's words (never 0)
+  const uint32_t* xl_base;       // *xl_base + xl_epoch: tag of this launch's words (never 0);
+  uint32_t xl_epoch;             // the plan advances the base, so a captured launch has a new tag
+                                 // each time
   int32_t xl_nbmax;              // workgroups per task in the grid
   int32_t xl_seq_rows;           // tables this short: one workgroup sweeps all blocks
   // Non-unit costs (costs != 0): the pool's pdel / pins prefix sums carry
@@ -193,6 +201,8 @@ hipError_t scan_init_attributes(int lds_limit);
 // On-chip row scan of W = 2^wi waves and C = 2^ci columns per lane, and
 // column-blocked form k (scan.hip).
 void launch_scan(int wi, int ci, const DPArgs& a, int lds_bytes, hipStream_t s);
+// (kClassSweep)
+void launch_sweep(const DPArgs& a, int lds_bytes, hipStream_t s);
 void launch_xl(int form, const DPArgs& a, int lds_bytes, hipStream_t s);
 // Launches the row-scan kernel of class `cls` over a.tasks[0..ntasks).
 // Returns false when the class has no kernel (the leaf class runs as one

@@ -47,15 +47,27 @@ __device__ __forceinline__ void classify(const PlanArgs& A, const TreeMeta& tx,
   const int32_t leaves_c = a <= b ? A.pool.sleaf[ly] : A.pool.sleaf[kx];
   int64_t need = 0;
   // With the leaf kernel off, single-row tables take the row-scan forms.
+  const int64_t offC = a <= b ? ty.node_off : tx.node_off;
+  const int32_t c0 = A.pool.skr[a <= b ? ly : kx], cmax = c0 + max(a, b);
+  auto own = [&](int k) {
+    const int32_t bw = xl_bw(k);
+    int32_t most = 0;
+    for (int32_t c = cmax; c > c0; c -= bw)  // the block of columns [c - bw, c)
+      most = max(most, A.pool.lrank[offC + c - 1] - A.pool.lrank[offC + max(c - bw - 1, c0)]);
+    return most;
+  };
+  auto level_cells = [&] {
+    return (int64_t)(A.level_cells ? A.level_cells[level] : A.mean_cells);
+  };
   int cls = table_class(a, b, a <= b ? kdx : kdy, a <= b ? kdy : kdx, leaves_c, leaf_form, rule,
-                        &need);
+                        level_cells, own, &need);
   // A forced column-blocked form takes every multi-row table it can hold.
   if (A.force_class >= kFirstXLClass && A.force_class < kFirstXLClass + kNumXLForms && cls >= 1 &&
       cls != kClassXL) {
     const int k = A.force_class - kFirstXLClass;
     const int32_t kd_c = a <= b ? kdy : kdx;
     int64_t n = 0;
-    if (xl_form(a <= b ? kdx : kdy, kd_c, leaves_c, k, A.rule.lds_max, &n) == k) {
+    if (xl_form(slots, kd_c, leaves_c, k, A.rule.lds_max, own, &n) == k) {
       cls = A.force_class;
       need = n;
     }
@@ -379,12 +391,46 @@ __global__ void plan_clear_kernel(PlanArgs a, int nb) {
     a.maxlds[i] = 0;
     a.tickets[i] = 0;
   }
+  if (a.level_cells && i < a.nlevels) a.level_cells[i] = 0;
   if (i < kAbortInts) a.abort_flag[i] = 0;
+  if (i == 0) {
+    // Every column-blocked launch of the group tags its words with the base
+    // and its ordinal: past those of the last plan (whose end the second word
+    // holds), never 0 nor 0xFFFFFFFF.
+    const uint32_t next = a.xl_base[1];
+    const uint32_t base = next == 0 || next > 0xF0000000u ? 1 : next;
+    a.xl_base[0] = base;
+    a.xl_base[1] = base + (uint32_t)a.nlevels * kNumXLForms;
+  }
+}
+
+// Interior cells of every level over all pairs, leaf keyroots' tables not
+// counted: a pair's level L holds the tables of x's keyroots of height h
+// against y's of height L - h, whose cells are the product of their summed
+// sizes (one workgroup per pair, one level per thread).
+__global__ __launch_bounds__(256) void level_cells_kernel(PlanArgs A) {
+  const int p = blockIdx.x;
+  const PairMeta pm = A.pairs[p];
+  const TreeMeta tx = A.pool.trees[pm.tx], ty = A.pool.trees[pm.ty];
+  const int32_t loff = A.level_off ? A.level_off[p] : 0;
+  auto sum = [&](const TreeMeta& t, int h) {
+    const int32_t* pre = A.pool.spre + t.node_off + t.K1;
+    const int32_t* off = A.pool.kdoff + t.node_off;
+    return (unsigned long long)(pre[off[h + 1]] - pre[off[h]]);
+  };
+  for (int L = threadIdx.x; L <= tx.kdmax + ty.kdmax; L += 256) {
+    unsigned long long cells = 0;
+    for (int h = max(0, L - ty.kdmax); h <= min(L, tx.kdmax); ++h)
+      cells += sum(tx, h) * sum(ty, L - h);
+    if (cells) atomicAdd(&A.level_cells[L + loff], cells);
+  }
 }
 
 void launch_plan(const PlanArgs& a, int64_t nblocks, hipStream_t s) {
   const int nb = a.nlevels * kNumClasses * kBands;
   hipLaunchKernelGGL(plan_clear_kernel, dim3((nb + 255) / 256), dim3(256), 0, s, a, nb);
+  if (a.level_cells)
+    hipLaunchKernelGGL(level_cells_kernel, dim3((unsigned)a.npairs), dim3(256), 0, s, a);
   if (nblocks > 0)
     hipLaunchKernelGGL(plan_kernel<false>, dim3((unsigned)nblocks), dim3(kPlanThreads), 0, s, a);
   hipLaunchKernelGGL(plan_scan_kernel, dim3(1), dim3(1024), 0, s, a.counts, a.cursor, nb);

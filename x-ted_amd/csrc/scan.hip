@@ -104,9 +104,9 @@ __device__ __forceinline__ void lds_order() {
 // workgroup; their words stay in its XCD and need no atomics.
 //
 // What bounds a row: the instructions of one wave, as on chip, with at most
-// two waves to a SIMD. Measured, us a row over the blocks of an 8000-node RRT
-// pair's root table, of 4096 / 2048 / 1024 / 512 columns: 0.45 / 0.32 / 0.29 /
-// 0.40 (on chip 16 waves of 8 columns 0.63). With a barrier per row and every
+// two or three waves to a SIMD. Measured, us a row over the blocks of an
+// 8000-node RRT pair's root table, of 4096 / 2048 / 1024 / 512 columns: 0.45 /
+// 0.32 / 0.27 / 0.26 (on chip 16 waves of 8 columns 0.63). With a barrier per row and every
 // wave reading the words itself, a 20,000-node pair's pipelined blocks took
 // 138 ms against 34 here, its tables of at most 256 rows 42 against 29.
 // ---------------------------------------------------------------------------
@@ -163,6 +163,7 @@ struct XLEdge {
   int32_t r0, rmax, nrows, kds, nb, blk, ticket;
   bool seq;
   unsigned long long* words;
+  uint32_t epoch;
   uint32_t edge;         // LDS byte offset of the edge to fill or empty
   uint32_t entry_bytes;
 };
@@ -190,6 +191,7 @@ __device__ __forceinline__ void edge_in(const DPArgs& A, const XLEdge& x, unsign
                                         int lane) {
   auto l32 = [&](uint32_t byte) -> int32_t& { return *reinterpret_cast<int32_t*>(lds + byte); };
   unsigned long long* const prog = reinterpret_cast<unsigned long long*>(lds);
+  const uint32_t epoch = x.epoch;
   const int32_t cstride = xl_pad(x.nrows), kdsp = xl_pad(x.kds);
   unsigned long long* const carries = x.words + (int64_t)(x.blk - 1) * cstride;
   unsigned long long* const exps = x.words + (int64_t)(x.nb - 1) * cstride;
@@ -208,9 +210,9 @@ __device__ __forceinline__ void edge_in(const DPArgs& A, const XLEdge& x, unsign
   unsigned long long cw = poll_line(0);
   for (int32_t k0 = 0; k0 < x.nrows; k0 += kXLLineRows) {
     if ((k0 & 63) == 0) xl_rows(x, k0, lane, flags, rid);
-    if (__ballot((uint32_t)(cw >> 32) != A.xl_epoch)) {
+    if (__ballot((uint32_t)(cw >> 32) != epoch)) {
       ++n_wait;
-      for (int n = 0; __ballot((uint32_t)(cw >> 32) != A.xl_epoch); ++n) {
+      for (int n = 0; __ballot((uint32_t)(cw >> 32) != epoch); ++n) {
         if (!pat.wait(n, A.xl_abort, x.ticket, k0)) break;
         cw = poll_line(k0);
       }
@@ -221,7 +223,7 @@ __device__ __forceinline__ void edge_in(const DPArgs& A, const XLEdge& x, unsign
 #pragma unroll
     for (int i = 0; i < kXLLineRows; ++i) {
       const int at = (k0 & 63) + i;
-      iw[i] = (unsigned long long)A.xl_epoch << 32;  // nothing to read: valid
+      iw[i] = (unsigned long long)epoch << 32;  // nothing to read: valid
       if ((__builtin_amdgcn_readlane(flags, at) & 2) && lane < x.kds)
         iw[i] = xl_peek(imp_word(__builtin_amdgcn_readlane(rid, at), lane));
     }
@@ -243,10 +245,10 @@ __device__ __forceinline__ void edge_in(const DPArgs& A, const XLEdge& x, unsign
       const int at = (k0 & 63) + i;
       const int32_t fl = __builtin_amdgcn_readlane(flags, at);
       if (fl & 1) {
-        if ((fl & 2) && __ballot((uint32_t)(iw[i] >> 32) != A.xl_epoch)) {
+        if ((fl & 2) && __ballot((uint32_t)(iw[i] >> 32) != epoch)) {
           ++n_stale;
-          for (int n = 0; __ballot((uint32_t)(iw[i] >> 32) != A.xl_epoch); ++n) {
-            if ((uint32_t)(iw[i] >> 32) != A.xl_epoch)
+          for (int n = 0; __ballot((uint32_t)(iw[i] >> 32) != epoch); ++n) {
+            if ((uint32_t)(iw[i] >> 32) != epoch)
               iw[i] = xl_load(imp_word(__builtin_amdgcn_readlane(rid, at), lane));
             if (!pat.wait(n, A.xl_abort, x.ticket, (1 << 24) | k)) break;
           }
@@ -256,10 +258,10 @@ __device__ __forceinline__ void edge_in(const DPArgs& A, const XLEdge& x, unsign
         if (fl & 2) {
           for (int32_t d0 = 64; d0 < x.kds; d0 += 64) {
             const int32_t d = d0 + lane;
-            unsigned long long w = (unsigned long long)A.xl_epoch << 32;
+            unsigned long long w = (unsigned long long)epoch << 32;
             if (d < x.kds) w = xl_peek(imp_word(__builtin_amdgcn_readlane(rid, at), d));
-            for (int n = 0; __ballot((uint32_t)(w >> 32) != A.xl_epoch); ++n) {
-              if ((uint32_t)(w >> 32) != A.xl_epoch)
+            for (int n = 0; __ballot((uint32_t)(w >> 32) != epoch); ++n) {
+              if ((uint32_t)(w >> 32) != epoch)
                 w = xl_load(imp_word(__builtin_amdgcn_readlane(rid, at), d));
               if (!pat.wait(n, A.xl_abort, x.ticket, (1 << 24) | k)) break;
             }
@@ -288,6 +290,7 @@ __device__ __forceinline__ void edge_out(const DPArgs& A, const XLEdge& x, unsig
                                          int W, int lane) {
   auto l32 = [&](uint32_t byte) -> int32_t& { return *reinterpret_cast<int32_t*>(lds + byte); };
   unsigned long long* const prog = reinterpret_cast<unsigned long long*>(lds);
+  const uint32_t epoch = x.epoch;
   const int32_t cstride = xl_pad(x.nrows), kdsp = xl_pad(x.kds);
   unsigned long long* const carries = x.words + (int64_t)x.blk * cstride;
   unsigned long long* const exps = x.words + (int64_t)(x.nb - 1) * cstride;
@@ -318,7 +321,7 @@ __device__ __forceinline__ void edge_out(const DPArgs& A, const XLEdge& x, unsig
             const int32_t d = d0 + lane;
             const int32_t v = l32(entry + 4 * min(1 + d, x.kds + 1));
             if (d < x.kds)
-              xl_store(exps + ((int64_t)r * x.nb + x.blk) * kdsp + d, A.xl_epoch, v, x.seq);
+              xl_store(exps + ((int64_t)r * x.nb + x.blk) * kdsp + d, epoch, v, x.seq);
           }
         }
         carry = lane == i ? c : carry;
@@ -331,21 +334,26 @@ __device__ __forceinline__ void edge_out(const DPArgs& A, const XLEdge& x, unsig
     __hip_atomic_store(prog + W + 1, ((unsigned long long)(uint32_t)q << 32) | (uint32_t)k0,
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     if (lane < kSync && k0 + lane < x.nrows)
-      xl_store(carries + k0 + lane, A.xl_epoch, carry, x.seq);
+      xl_store(carries + k0 + lane, epoch, carry, x.seq);
   }
 }
 
-// One table, or with kXL one column block of a table, on the calling
-// workgroup (64 * W threads, 128 more with kXL).
-template <int W, int C, bool kCost, bool kXL>
+// One table (kTable), or one column block of a table: of a pipeline of
+// workgroups (kBlocked) or of the sweep of one wave (kSwept). On the calling
+// workgroup (64 * W threads, 128 more with kBlocked).
+enum ScanMode { kTable, kBlocked, kSwept };
+template <int W, int C, bool kCost, ScanMode kMode>
 __device__ __forceinline__ void scan_block(const DPArgs& A, const TaskDesc& dsc, int32_t ix,
                                            int32_t blk, int32_t nb) {
-  constexpr bool kEdges = W > 1 || kXL;
+  constexpr bool kXL = kMode == kBlocked;
+  constexpr bool kRing = W > 1 || kXL;                // edges are rings between waves
+  constexpr bool kEdges = kRing || kMode == kSwept;
+  static_assert(kMode != kSwept || W == 1);
   // TD ring slots: a power of two dividing 64.
   constexpr int S = C >= 16 || (W == 1 && C >= 8 && !kXL) || (kXL && kCost && C >= 8) ? 4 : 8;
   constexpr int PD = S - 1;                    // rows of TD prefetched
   constexpr int NW = C == 1 ? 1 : C / 2;       // words of one row: two 16-bit entries each
-  constexpr int D = kXL ? xl_edge_rows(W * C) : kEdgeRows;
+  constexpr int D = kXL ? xl_edge_rows(W) : kEdgeRows;
   constexpr int kSync = D / 2;  // a wave may fill one group while the next takes another
   extern __shared__ __align__(16) unsigned char lds[];
   const bool rows_x = dsc.base_rx < 0;
@@ -366,12 +374,12 @@ __device__ __forceinline__ void scan_block(const DPArgs& A, const TaskDesc& dsc,
   const int32_t orl_c0 = cmax - 1;
 
   // Uniform over the wave, so it lives in a scalar register.
-  const int wave = kEdges ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  const int wave = kRing ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
   const int lane = threadIdx.x & 63;
-  const int32_t tb0 = kXL ? blk * (64 * W * C) : 0;  // first t of the block
+  const int32_t tb0 = kMode != kTable ? blk * (64 * W * C) : 0;  // first t of the block
   const int32_t tb = tb0 + wave * 64 * C;            // and of this wave's part
   const int32_t tlane = tb + lane * C;               // t of this lane's element 0
-  const int32_t nw = kEdges ? min(W, (ncols - tb0 + 64 * C - 1) / (64 * C)) : 1;  // waves used
+  const int32_t nw = kRing ? min(W, (ncols - tb0 + 64 * C - 1) / (64 * C)) : 1;  // waves used
 
   // Costs (kCost). Hpre / Vpre: prefix sums of the horizontal (column) and
   // vertical (row) edit costs over the column and row trees: insertions and
@@ -402,9 +410,9 @@ __device__ __forceinline__ void scan_block(const DPArgs& A, const TaskDesc& dsc,
   // table's last, by leaf rank), at index wb the boundary value F[R][cmax]
   // that tree columns read, the kds imports (W > 1) and a sink that columns
   // saving nothing write.
-  const int32_t ltop = lrankC[max(cmax - 1 - tb0, c0)];  // (kXL) of the block's columns
+  const int32_t ltop = lrankC[max(cmax - 1 - tb0, c0)];  // of the block's columns
   int32_t lbase0 = dsc.lbase;
-  if constexpr (kXL) lbase0 = lrankC[max(cmax - tb0 - 64 * W * C - 1, c0)];
+  if constexpr (kMode != kTable) lbase0 = lrankC[max(cmax - tb0 - 64 * W * C - 1, c0)];
   int32_t lbase = lbase0, wb = ltop - lbase0, seg = 0, kds = 0, kdep_c0 = 0;
   if constexpr (kEdges) {
     const int32_t chi = max(cmax - 1 - tb, c0);
@@ -418,14 +426,19 @@ __device__ __forceinline__ void scan_block(const DPArgs& A, const TaskDesc& dsc,
   }
   const uint32_t entry_bytes = kEdges ? 4u * (uint32_t)(kds + 2) : 0u;
   const uint32_t edge_bytes = D * entry_bytes;
-  constexpr uint32_t edges = kEdges ? 8u * (W + 2) : 0u;  // byte offset of edge 0
-  const uint32_t slot_base = edges + (kEdges ? (W + 1) * edge_bytes : 0u) + 2u * (uint32_t)seg;
+  constexpr uint32_t edges = kRing ? 8u * (W + 2) : 0u;  // byte offset of edge 0
+  const uint32_t all_edges = kRing ? (W + 1) * edge_bytes : (uint32_t)(nrows + 1) * entry_bytes;
+  const uint32_t slot_base = edges + (kEdges ? all_edges : 0u) + 2u * (uint32_t)seg;
   const uint32_t row_bytes = 2u * (uint32_t)((ltop - lbase0) + W * (2 + kds));
   const int32_t sinkix = wb + 1 + kds;
   auto l16 = [&](uint32_t byte) -> uint16_t& { return *reinterpret_cast<uint16_t*>(lds + byte); };
   auto l32 = [&](uint32_t byte) -> int32_t& { return *reinterpret_cast<int32_t*>(lds + byte); };
   auto prog = [&](int w) { return reinterpret_cast<unsigned long long*>(lds + 8 * w); };
-  if constexpr (kEdges) {
+  if constexpr (kMode == kSwept) {
+    if (blk == 0)
+      for (int32_t k = lane; k <= nrows; k += 64) l32(k * entry_bytes) = cin0;
+  }
+  if constexpr (kRing) {
     if (threadIdx.x < D) l32(edges + threadIdx.x * entry_bytes) = cin0;
     if (threadIdx.x < W + 2) {
       const int w = (int)threadIdx.x - 1;
@@ -436,7 +449,8 @@ __device__ __forceinline__ void scan_block(const DPArgs& A, const TaskDesc& dsc,
     if constexpr (kXL) {
       if (wave >= W) {
         XLEdge x{rrecR, A.pool.lrank + offR, r0, rmax, nrows, kds, nb, blk, ix,
-                 nrows <= A.xl_seq_rows, A.xl_words + A.xl_off[ix], edges, entry_bytes};
+                 nrows <= A.xl_seq_rows, A.xl_words + A.xl_off[ix],
+                 *A.xl_base + A.xl_epoch, edges, entry_bytes};
         if (wave == W && blk > 0) {
           edge_in<D, kSync>(A, x, lds, lane);
         } else if (wave > W && blk + 1 < nb) {
@@ -641,8 +655,9 @@ __device__ __forceinline__ void scan_block(const DPArgs& A, const TaskDesc& dsc,
   // on the outgoing entry lane 63, whose prefix minimum is the block's, writes
   // the carry.
   const int32_t word = min(lane, kds + 1);
-  const uint32_t ein = edges + (uint32_t)wave * edge_bytes + 4u * (uint32_t)word;
-  const uint32_t xout = edges + (uint32_t)(wave + 1) * edge_bytes;
+  const uint32_t xin = edges + (kRing ? (uint32_t)wave * edge_bytes : 0u);
+  const uint32_t xout = edges + (kRing ? (uint32_t)(wave + 1) * edge_bytes : 0u);
+  const uint32_t ein = xin + 4u * (uint32_t)word;
   const uint32_t eout = xout + 4u * (uint32_t)(lane == 0 ? kds + 1 : lane == 63 ? 0 : word);
   const uint32_t seg_imp = slot_base + 2u * (uint32_t)(wb + word);
   uint32_t qoff = 0;  // (q % D) * entry_bytes
@@ -671,7 +686,7 @@ __device__ __forceinline__ void scan_block(const DPArgs& A, const TaskDesc& dsc,
       // Rows past the table's end: skipped where a row costs more than the
       // branch, else run as plain rows up to the next even one.
       if ((C < 8 && u % 2 == 1) || __builtin_expect(k < nrows, 1)) {
-        if constexpr (kEdges) {
+        if constexpr (kRing) {
           if (u % kSync == 0) {
             // This group's entries are there, and its full rows (at most
             // kSync) find room in the outgoing ring.
@@ -777,7 +792,7 @@ __device__ __forceinline__ void scan_block(const DPArgs& A, const TaskDesc& dsc,
               if (__builtin_expect(kds >= 63, 0)) {
                 for (int d0 = 63; d0 <= kds; d0 += 64) {
                   const int dd = min(d0 + lane, kds + 1);
-                  const int32_t far = l32(xout - edge_bytes + qoff + 4 * dd);
+                  const int32_t far = l32(xin + qoff + 4 * dd);
                   l16(slot_base + wbase + 2 * (wb + dd)) = (uint16_t)far;
                   l32(xout + qoff + 4 * dd) = far;
                 }
@@ -798,7 +813,7 @@ __device__ __forceinline__ void scan_block(const DPArgs& A, const TaskDesc& dsc,
           if constexpr (kEdges) {
             ++q;
             qoff += entry_bytes;
-            if (qoff == edge_bytes) qoff = 0;
+            if (kRing && qoff == edge_bytes) qoff = 0;
           }
           // (Tested afresh: one flag kept over the row costs more.)
           int32_t fw2 = fw;
@@ -828,7 +843,7 @@ __device__ __forceinline__ void scan_block(const DPArgs& A, const TaskDesc& dsc,
           }
         }
       }  // k < nrows
-      if constexpr (kEdges) {
+      if constexpr (kRing) {
         if (u % kSync == kSync - 1) {
           lds_order();
           __hip_atomic_store(prog(wave + 1),
@@ -841,18 +856,44 @@ __device__ __forceinline__ void scan_block(const DPArgs& A, const TaskDesc& dsc,
   }
 }
 
-template <int W, int C, bool kCost>
-__global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
-  // Workgroups go round robin over the 8 XCDs, each with its own L2; task
-  // order keeps a pair's tables together, so kXcdRun consecutive tasks are
-  // given to one XCD (the last, partial span keeps its order). The 4096-pair
-  // batch ran 101.6 ms without, 100.1 with 16, 101.0 with 64, 104.8 with 256.
+// Workgroups go round robin over the 8 XCDs, each with its own L2; task
+// order keeps a pair's tables together, so kXcdRun consecutive tasks are
+// given to one XCD (the last, partial span keeps its order). The 4096-pair
+// batch ran 101.6 ms without, 100.1 with 16, 101.0 with 64, 104.8 with 256.
+__device__ __forceinline__ uint32_t xcd_task(int64_t ntasks) {
   constexpr uint32_t kXcds = 8, kXcdRun = 16, kSpan = kXcds * kXcdRun;
   uint32_t ix = blockIdx.x;
-  if ((ix | (kSpan - 1)) < (uint64_t)A.ntasks)
+  if ((ix | (kSpan - 1)) < (uint64_t)ntasks)
     ix = (ix & ~(kSpan - 1)) + (ix % kXcds) * kXcdRun + (ix % kSpan) / kXcds;
+  return ix;
+}
+
+template <int W, int C, bool kCost>
+__global__ __launch_bounds__(64 * W) void scan_kernel(DPArgs A) {
+  const uint32_t ix = xcd_task(A.ntasks);
   if ((int64_t)ix >= A.ntasks) return;
-  scan_block<W, C, kCost, false>(A, A.descs[ix], (int32_t)ix, 0, 1);
+  scan_block<W, C, kCost, kTable>(A, A.descs[ix], (int32_t)ix, 0, 1);
+}
+
+// One table per wave, block after block of kSweepCols columns, for wide tables
+// of few rows in levels of many: the edge is one entry per full row, read by a
+// block and overwritten for the next, and a slot row holds one block's far
+// columns. What bounds it: the columns' records (36 bytes a column against 2 a
+// cell) and the set-up of each block, of which a SIMD holds 4 at a time.
+// 6165 tables of 8,000-20,000 columns and about 17 rows: 1.6 ms against 14
+// in blocks of 1024 columns swept by a workgroup of 8 waves.
+template <bool kCost>
+__global__ __launch_bounds__(64, kCost ? 3 : 4) void scan_sweep_kernel(DPArgs A) {
+  const uint32_t ix = xcd_task(A.ntasks);
+  if ((int64_t)ix >= A.ntasks) return;
+  const int32_t nb = (A.descs[ix].cmax - A.descs[ix].c0 + kSweepCols - 1) / kSweepCols;
+  for (int32_t blk = 0; blk < nb; ++blk) {
+    // (Opaque for each block, as in scan_xl_kernel.)
+    uint32_t ib = ix;
+    asm volatile("" : "+s"(ib));
+    scan_block<1, kSweepCols / 64, kCost, kSwept>(A, A.descs[ib], (int32_t)ib, blk, nb);
+    lds_order();
+  }
 }
 
 // Column-blocked: W waves of C columns per lane and the two edge waves.
@@ -877,7 +918,7 @@ __global__ __launch_bounds__(64 * (W + 2)) void scan_xl_kernel(DPArgs A) {
     // of them, and the widest form would spill).
     int32_t ib = ix;
     asm volatile("" : "+s"(ib));
-    scan_block<W, C, kCost, true>(A, A.descs[ib], ib, blk, nb);
+    scan_block<W, C, kCost, kBlocked>(A, A.descs[ib], ib, blk, nb);
   } while (seq && ++blk < nb);
 }
 
@@ -913,6 +954,22 @@ static void launch_c(int ci, const DPArgs& a, int lds, hipStream_t s) {
   }
 }
 
+void launch_sweep(const DPArgs& a, int lds_bytes, hipStream_t s) {
+  constexpr int64_t kChunk = kGridThreads / 64;
+  for (int64_t off = 0; off < a.ntasks; off += kChunk) {
+    DPArgs c = a;
+    c.tasks = a.tasks + off;
+    c.descs = a.descs + off;
+    c.ntasks = std::min(kChunk, a.ntasks - off);
+    if (a.costs)
+      hipLaunchKernelGGL(scan_sweep_kernel<true>, dim3((unsigned)c.ntasks), dim3(64),
+                         (size_t)lds_bytes, s, c);
+    else
+      hipLaunchKernelGGL(scan_sweep_kernel<false>, dim3((unsigned)c.ntasks), dim3(64),
+                         (size_t)lds_bytes, s, c);
+  }
+}
+
 template <int W, int C>
 static void launch_xl_one(const DPArgs& a, int lds_bytes, hipStream_t s) {
   // Workgroups take (task, block) tickets from one counter that the pieces
@@ -936,8 +993,8 @@ void launch_xl(int form, const DPArgs& a, int lds_bytes, hipStream_t s) {
   switch (form) {  // must match xl_waves / xl_cpl
     case 0: launch_xl_one<8, 8>(a, lds_bytes, s); break;
     case 1: launch_xl_one<8, 4>(a, lds_bytes, s); break;
-    case 2: launch_xl_one<4, 4>(a, lds_bytes, s); break;
-    case 3: launch_xl_one<1, 8>(a, lds_bytes, s); break;
+    case 2: launch_xl_one<8, 2>(a, lds_bytes, s); break;
+    case 3: launch_xl_one<4, 2>(a, lds_bytes, s); break;
     case 4: launch_xl_one<1, 4>(a, lds_bytes, s); break;
     default: launch_xl_one<1, 2>(a, lds_bytes, s); break;
   }
@@ -985,10 +1042,15 @@ static hipError_t allow_xl(int limit) {
 hipError_t scan_init_attributes(int limit) {
   hipError_t e;
   const int xl_limit = limit + kXLEdgeBytes;
+  for (const void* f : {reinterpret_cast<const void*>(&scan_sweep_kernel<false>),
+                        reinterpret_cast<const void*>(&scan_sweep_kernel<true>)}) {
+    e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, limit);
+    if (e != hipSuccess) return e;
+  }
   if ((e = allow_xl<8, 8>(xl_limit)) != hipSuccess) return e;
   if ((e = allow_xl<8, 4>(xl_limit)) != hipSuccess) return e;
-  if ((e = allow_xl<4, 4>(xl_limit)) != hipSuccess) return e;
-  if ((e = allow_xl<1, 8>(xl_limit)) != hipSuccess) return e;
+  if ((e = allow_xl<8, 2>(xl_limit)) != hipSuccess) return e;
+  if ((e = allow_xl<4, 2>(xl_limit)) != hipSuccess) return e;
   if ((e = allow_xl<1, 4>(xl_limit)) != hipSuccess) return e;
   if ((e = allow_xl<1, 2>(xl_limit)) != hipSuccess) return e;
   if ((e = allow_c<1>(limit)) != hipSuccess) return e;

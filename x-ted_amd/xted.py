@@ -26,10 +26,11 @@ ERR_CANCELLED = 10
 
 CLASS_AUTO = -1
 CLASS_LANE = 0
-NUM_CLASSES = 39
+NUM_CLASSES = 40
 CLASS_TINY = 33  # tiny forms 33, 34, 35: 16, 32, 64 lanes per table
 TINY_SEG = (16, 32, 64)
 CLASS_SHARED = 36  # shared-slot forms 36, 37, 38: 4, 8, 16 waves of 8 columns per lane
+CLASS_SWEEP = 39  # swept by one wave, 512 columns at a time
 XL_BW = (4096, 2048, 1024, 512, 256, 128)  # column-block widths of classes 27..32
 
 
@@ -38,7 +39,8 @@ def class_name(cls):
     'rowscan_w{W}_c{C}' (W waves, C columns per lane) or 'xl_bw{B}' (column
     blocks of B columns, one workgroup each) or 'tiny_s{S}' (tables of at
     most S = 16, 32 or 64 columns, 64 / S to a wave) or 'shared_w{W}_c8' (W
-    waves sharing slot rows: deep column keyroots) or 'too_large'."""
+    waves sharing slot rows: deep column keyroots) or 'sweep' (one wave, 512
+    columns at a time) or 'too_large'."""
     if cls == 0:
         return "leaf"
     if 1 <= cls <= 25:
@@ -48,7 +50,9 @@ def class_name(cls):
         return f"xl_bw{XL_BW[cls - 27]}"
     if CLASS_TINY <= cls < CLASS_TINY + len(TINY_SEG):
         return f"tiny_s{TINY_SEG[cls - CLASS_TINY]}"
-    if CLASS_SHARED <= cls < NUM_CLASSES:
+    if cls == CLASS_SWEEP:
+        return "sweep"
+    if CLASS_SHARED <= cls < CLASS_SWEEP:
         return f"shared_w{4 << (cls - CLASS_SHARED)}_c8"
     return "too_large"
 
