@@ -12,6 +12,7 @@
 #include <algorithm>
 #include <array>
 #include <chrono>
+#include <cmath>
 #include <cstring>
 
 #include "engine.hpp"
@@ -706,6 +707,31 @@ int Context::launch_levels(Group* const* gs, int ng, std::vector<ProfLaunch>* pr
     int32_t lds;      // largest slot storage over the bands
     int level;
     bool heavy;       // the tables that need more slot storage than light_lds
+    double us;        // expected time alone
+  };
+  // A launch takes its longest table's rows one after another, or its cells
+  // at the chip's rate. The rows are those of the largest tables' band on
+  // average, their columns three quarters of what the form holds (column
+  // blocks hold any number: at least a block, and as many as rows).
+  auto expected_us = [](int cls, bool heavy, unsigned long long cells,
+                        unsigned long long big_cells, unsigned long long big_cnt) {
+    const double area = (double)big_cells / (double)std::max(big_cnt, 1ull);
+    double row = 0.2, cols = 512;  // us a row, columns
+    if (cls >= 1 && cls <= kNumRowClasses) {
+      const int wc = (1 << (cls - 1) / 5) * (1 << (cls - 1) % 5);
+      row = 0.18 + 0.0037 * wc;
+      cols = 48.0 * wc;
+    } else if (cls >= kFirstXLClass && cls < kFirstXLClass + kNumXLForms) {
+      const int bw = xl_bw(cls - kFirstXLClass);
+      row = 0.18 + 0.0037 * bw / 64;
+      cols = std::max((double)bw, std::sqrt(area));
+    } else if (is_shared(cls)) {
+      row = 0.5;
+      cols = 0.75 * shared_cols(cls - kClassShared);
+    } else if (is_tiny(cls)) {
+      cols = 0.75 * tiny_seg(cls - kClassTiny);
+    }
+    return std::max(5.0 + row * area / cols, (double)cells / (heavy ? 150e3 : 500e3));
   };
   std::vector<Launch> lv, leaf;
   for (int gi = 0; gi < ng; ++gi) {
@@ -722,38 +748,51 @@ int Context::launch_levels(Group* const* gs, int ng, std::vector<ProfLaunch>* pr
     // tables with placeholders, so it runs before the group's first level.
     if (L == 0 && g.lines[g.npairs] > 0 && !g.leaf_early)
       leaf.push_back({&g, kClassLane, -1, 0, (unsigned long long)g.lines[g.npairs],
-                      (unsigned long long)g.leaf_cells, 0, -1, false});
+                      (unsigned long long)g.leaf_cells, 0, -1, false, 0.0});
     unsigned long long off = g.level_off;
     for (int c = 0; c < kNumClasses; ++c) {
       // The bands of (L, c) are contiguous in the task array, largest first:
       // light tables, then heavy ones (size_band), one launch each.
       for (int half = 0; half < kBands / kRowBands; ++half) {
-        unsigned long long cnt = 0, cells = 0;
+        unsigned long long cnt = 0, cells = 0, big_cnt = 0, big_cells = 0;
         int32_t lds = 0;
         for (int bd = half * kRowBands; bd < (half + 1) * kRowBands; ++bd) {
           const size_t b = bucket_of(L, c, bd);
+          if (cnt == 0) {
+            big_cnt = g.h_counts[b];
+            big_cells = g.h_cells[b];
+          }
           cnt += g.h_counts[b];
           cells += g.h_cells[b];
           lds = std::max(lds, g.h_maxlds[b]);
         }
-        if (cnt) lv.push_back({&g, c, bucket_of(L, c, 0), off, cnt, cells, lds, L, half > 0});
+        if (cnt)
+          lv.push_back({&g, c, bucket_of(L, c, 0), off, cnt, cells, lds, L, half > 0,
+                        expected_us(c, half > 0, cells, big_cells, big_cnt)});
         off += cnt;
       }
     }
     g.level_off = off;
     ++g.next_level;
   }
-  // Launches whose time is set by their longest tables first: the heavy
-  // ones (few long tables at low occupancy) and those of 4 or more waves
-  // per table, each on a stream of its own where there are enough; then the
-  // rest by class id, descending. (Heavy launches last ran 110 ms against
-  // 101 ms per batch; among the rest, class order measured about 1% faster
-  // than ordering by cells.)
+  // Launches whose time is set by their longest tables first, longest first:
+  // the heavy ones (few long tables at low occupancy) and those of 4 or more
+  // waves per table or column blocks; then the rest by class id, descending.
+  // (Heavy launches last ran 110 ms against 101 ms per batch; among the rest,
+  // class order measured about 1% faster than ordering by cells.) In levels of
+  // up to kBalancedUs each goes on the stream that is due to be free first,
+  // in longer ones, which fill the chip, on the streams in turn, so that long
+  // and short launches mix. Measured in ms with no level balanced, those up to
+  // 0.5, 1, 2, 4 ms, every one: 128 pairs of 100-600 nodes 20.4, 18.9, 18.8,
+  // 18.9, 18.9, 18.9; 1024 pairs under a cost model 56.9, 56.7, 56.1, 53.9,
+  // 53.9, 53.1; 4096 pairs 89.4, 89.1, 89.0, 89.1, 89.5, 91.1.
+  constexpr double kBalancedUs = 2000;
   auto latency_bound = [](const Launch& l) {
-    return l.heavy || is_shared(l.cls) || (l.cls >= row_class(2, 0) && l.cls <= kNumRowClasses);
+    return l.heavy || is_shared(l.cls) || (l.cls >= row_class(2, 0) && l.cls < kClassTiny);
   };
   std::stable_sort(lv.begin(), lv.end(), [&](const Launch& x, const Launch& y) {
-    return latency_bound(x) != latency_bound(y) ? latency_bound(x) : x.cls > y.cls;
+    if (latency_bound(x) != latency_bound(y)) return latency_bound(x);
+    return latency_bound(x) ? x.us > y.us : x.cls > y.cls;
   });
   if (prof) {
     while (prof_ev_.size() < 2 * (prof->size() + lv.size() + leaf.size())) {
@@ -767,6 +806,10 @@ int Context::launch_levels(Group* const* gs, int ng, std::vector<ProfLaunch>* pr
   // Leaf launches go first on the main stream; the fork follows them, so
   // every table of the level starts after them.
   const size_t nleaf = leaf.size();
+  double due[kMaxLevelStreams] = {};  // us of the launches on each stream so far
+  double total = 0;
+  for (const Launch& l : lv) total += l.us;
+  const bool in_turn = total > kBalancedUs;
   lv.insert(lv.begin(), leaf.begin(), leaf.end());
   for (size_t i = 0; i < lv.size(); ++i) {
     if (i == nleaf) {
@@ -775,7 +818,11 @@ int Context::launch_levels(Group* const* gs, int ng, std::vector<ProfLaunch>* pr
     }
     const Launch& w = lv[i];
     Group& g = *w.g;
-    hipStream_t s = i < nleaf ? sl[0] : sl[(i - nleaf) % ns];
+    const int si = i < nleaf ? 0
+                   : in_turn ? (int)((i - nleaf) % ns)
+                             : (int)(std::min_element(due, due + ns) - due);
+    hipStream_t s = sl[si];
+    due[si] += w.us;
     if (prof) HIP_TRY(hipEventRecord(prof_ev_[2 * prof->size()], s));
     if (w.cls == kClassLane) {
       launch_leaf(leaf_args(g), (int64_t)w.cnt, s);
