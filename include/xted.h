@@ -168,8 +168,8 @@ int xted_all_pairs(xted_context* ctx, int32_t ntrees, const int32_t* sizes,
  * Granularity cut-overs, the role of the fixed thresholds 15 / 18,750 /
  * 25,250,000 in X-TED_GPU/parallel_X_TED.cu:382. lds_per_wave: slot bytes
  * one wave may own before a table gets more waves; max_cpl (1, 2, 4, 8 or
- * 16): columns per lane before a table gets more waves (at most 8 under a
- * cost model, whose 16-column forms run at 2 waves per SIMD); tables with at
+ * 16, the default): columns per lane before a table gets more waves (at most
+ * 8 under a cost model, whose 16-column forms run at 2 waves per SIMD); tables with at
  * least wide_cols columns get at least min_waves waves. */
 int xted_set_tuning(xted_context* ctx, int32_t lds_per_wave, int32_t max_cpl,
                     int32_t min_waves, int32_t wide_cols);
@@ -185,7 +185,9 @@ int xted_force_class(xted_context* ctx, int32_t cls, int32_t lane_enable);
 int xted_set_tail_rule(xted_context* ctx, int32_t tail_pairs);
 /* Column-blocked tables with at most seq_rows rows are swept block after
  * block by one workgroup (no waits between workgroups); taller ones run one
- * workgroup per block, chained per row. */
+ * workgroup per block, chained per row. Tables of more rows are column-blocked
+ * also where they would fit one workgroup, if their rows one after another
+ * would take longer than the rest of their level. */
 int xted_set_xl_rule(xted_context* ctx, int32_t seq_rows);
 /* Widest column block (128 to 4096 columns; default 4096) that a taller
  * column-blocked table may use: narrower blocks put more workgroups on one
@@ -203,10 +205,10 @@ int xted_set_level_streams(xted_context* ctx, int32_t n);
  * plan overlaps the levels of the groups before it. No counterpart in the
  * reference, which runs one pair at a time. Results do not depend on it. */
 int xted_set_batch_groups(xted_context* ctx, int32_t groups, int32_t split_min);
-/* Where each pair's levels sit among the batch's levels: 0 (the default)
- * starts every pair at level 0, as the reference's single pair does
- * (X-TED_GPU/parallel_X_TED.cu:214-220); 1 ends every pair at the batch's
- * last level; 2 places it midway. A pair's own levels keep their order
+/* Where each pair's levels sit among the batch's levels: 0 starts every pair
+ * at level 0, as the reference's single pair does
+ * (X-TED_GPU/parallel_X_TED.cu:214-220); 1 (the default) ends every pair at
+ * the batch's last level; 2 places it midway. A pair's own levels keep their order
  * (level = depth_x + depth_y + offset), so results do not depend on it; the
  * offsets move the tables of shallow pairs into the levels whose time is set
  * by the few large tables of the deepest pairs. */

@@ -219,11 +219,12 @@ constexpr int kMaxCols = 64 * 16 * kMaxRowWaves;  // 16384
 // 16 columns per lane at 16 waves would spill); wider tables are column-blocked.
 constexpr int kMaxOnChipCols = 64 * 8 * kMaxRowWaves;  // 8192
 
-// 16-lane form only by default. Under the default rule the 32-lane form ran
-// the 4096-pair batch in the same time (100.6 against 100.9 ms unit, 125.0
-// against 124.4 ms under a cost model); the tuned rule (x-ted_amd/tuning.json:
-// up to 16 columns per lane) turns it on (96.5 against 99.6 ms). The 64-lane
-// form ran 4% slower (4 waves per SIMD for its 64 TD registers per lane).
+// 16-lane form only by default: with the 32-lane form as well the 96-tree
+// distance matrix took 99.8 against 99.9 ms, 128 pairs of 100-600 nodes 19.0
+// against 19.0, 1024 pairs under a cost model 55.4 against 53.8. The tuned
+// rule of the 4096-pair batch (x-ted_amd/tuning.json) turns it on (96.5
+// against 99.6 ms when it was tuned). The 64-lane form ran 8% slower there (4
+// waves per SIMD for its 64 TD registers per lane).
 constexpr int32_t kTinyDefault = 1;
 // Most columns per lane a table takes under a cost model.
 constexpr int32_t kMaxCostCpl = 8;

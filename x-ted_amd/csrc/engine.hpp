@@ -231,7 +231,9 @@ class Context {
   int poll(Group& g, bool wait, int32_t* dist);
 
   // Tuning / test hooks -----------------------------------------------------
-  ClassRule rule{kLdsPerWave, 1, 1 << 30, kLdsMaxTable, 8, kXLSeqRows};
+  // (Up to 16 columns per lane: the distance matrix of 96 trees of 100-1000
+  // nodes took 99.9 ms against 110.8 with 8, and 89.4 with level_align 1.)
+  ClassRule rule{kLdsPerWave, 1, 1 << 30, kLdsMaxTable, 16, kXLSeqRows};
   int32_t lds_limit = 0;  // device's dynamic LDS per workgroup for the slots
   int32_t force_class = -1;
   int32_t lane_enable = 1;
@@ -255,16 +257,18 @@ class Context {
   // as a tail level by the pairs of the whole batch that reach it
   // (estimated as the group's count times this).
   int32_t plan_share = 1;
-  // Level launches of a batch without column-blocked tables run as a
-  // captured graph (re-launched while the plan's launches stay the same);
-  // not while profiling, which times each launch with events.
+  // Level launches of a batch run as a captured graph (re-launched while the
+  // plan's launches stay the same); not while profiling, which times each
+  // launch with events.
   int32_t use_graphs = 1;
   // Where a pair's levels sit among the batch's: 0 = every pair starts at
   // level 0, 1 = every pair ends at the batch's last level, 2 = midway. A
   // pair's own levels keep their order, so each is a valid schedule; the
   // choice moves shallow pairs' tables into levels whose time is set by the
-  // few large tables of the deepest pairs.
-  int32_t level_align = 0;
+  // few large tables of the deepest pairs. In ms with 0, 1, 2: the 96-tree
+  // matrix 99.9, 89.3, 90; 128 pairs of 100-600 nodes 18.8, 17.2, 17.6; 1024
+  // pairs under a cost model 54.0, 50.3, 49.4.
+  int32_t level_align = 1;
   // 1: the tables of a launch start largest first (size bands); 2: and the
   // tables that need more slot storage than light_lds take launches of
   // their own; 0: plan order.
