@@ -148,6 +148,7 @@ int Context::init() {
   HIP_TRY(hipGetDeviceProperties(&prop, device_));
   lds_limit = (int32_t)std::min<size_t>(kLdsMaxTable, prop.sharedMemPerBlock - 256);
   HIP_TRY(forest_init_attributes(lds_limit));
+  HIP_TRY(prep_init_attributes());
   rule.lds_max = lds_limit;
   // This device's copy of the no-allocation array, and what its batch group
   // needs besides memory, so that run_batch_noalloc creates nothing.
@@ -218,6 +219,7 @@ int Context::pool_add(int32_t ntrees, const int32_t* sizes, const int32_t* paren
   HIP_TRY(hipSetDevice(device_));
   // Validate on the host and lay out the padded staging arrays.
   int64_t total = 0, in_off = 0, scratch_total = 0;
+  int32_t maxn = 0;
   std::vector<int64_t> offs(ntrees), scr(ntrees);
   for (int32_t t = 0; t < ntrees; ++t) {
     const int32_t n = sizes[t];
@@ -237,7 +239,8 @@ int Context::pool_add(int32_t ntrees, const int32_t* sizes, const int32_t* paren
     offs[t] = pool_nodes_ + total;
     scr[t] = scratch_total;
     total += n + 1;
-    scratch_total += 6 * (int64_t)(n + 1);
+    maxn = std::max(maxn, n);
+    if (n > kPrepLdsNodes) scratch_total += kPrepArrays * (int64_t)(n + 1);
     in_off += n;
   }
   std::vector<int32_t> hp(total, -1), hl(total, 0);
@@ -268,16 +271,18 @@ int Context::pool_add(int32_t ntrees, const int32_t* sizes, const int32_t* paren
   const int32_t first = (int32_t)meta_.size();
   ST_TRY(grow_pool(pool_nodes_ + total));
   ST_TRY(trees_.grow(sizeof(TreeMeta) * (first + ntrees), true, stream_));
-  ST_TRY(prep_scratch_.grow(sizeof(int32_t) * scratch_total, false, stream_));
-  ST_TRY(prep_off_.grow(sizeof(int64_t) * ntrees, false, stream_));
+  if (scratch_total > 0) {
+    ST_TRY(prep_scratch_.grow(sizeof(int32_t) * scratch_total, false, stream_));
+    ST_TRY(prep_off_.grow(sizeof(int64_t) * ntrees, false, stream_));
+    HIP_TRY(hipMemcpyAsync(prep_off_.p, scr.data(), sizeof(int64_t) * ntrees,
+                           hipMemcpyHostToDevice, stream_));
+  }
   HIP_TRY(hipMemcpyAsync(parent_.as<int32_t>() + pool_nodes_, hp.data(), sizeof(int32_t) * total,
                          hipMemcpyHostToDevice, stream_));
   HIP_TRY(hipMemcpyAsync(label_.as<int32_t>() + pool_nodes_, hl.data(), sizeof(int32_t) * total,
                          hipMemcpyHostToDevice, stream_));
   HIP_TRY(hipMemcpyAsync(trees_.as<TreeMeta>() + first, tm.data(), sizeof(TreeMeta) * ntrees,
                          hipMemcpyHostToDevice, stream_));
-  HIP_TRY(hipMemcpyAsync(prep_off_.p, scr.data(), sizeof(int64_t) * ntrees, hipMemcpyHostToDevice,
-                         stream_));
   PrepArgs pa;
   pa.parent = parent_.as<int32_t>();
   pa.label = label_.as<int32_t>();
@@ -302,7 +307,7 @@ int Context::pool_add(int32_t ntrees, const int32_t* sizes, const int32_t* paren
   pa.scratch = prep_scratch_.as<int32_t>();
   pa.scratch_off = prep_off_.as<int64_t>();
   pa.first_tree = first;
-  launch_tree_prep(pa, ntrees, stream_);
+  launch_tree_prep(pa, ntrees, maxn, stream_);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipMemcpyAsync(tm.data(), trees_.as<TreeMeta>() + first, sizeof(TreeMeta) * ntrees,
                          hipMemcpyDeviceToHost, stream_));

@@ -28,11 +28,18 @@ struct PrepArgs {
   NodeRec* crec;
   NodeRec* rrec;
   TreeMeta* trees;
-  int32_t* scratch;            // 6*(n+1) ints per tree at scratch_off[b]
-  const int64_t* scratch_off;  // per block of this launch
+  // Trees of more than kPrepLdsNodes nodes: kPrepArrays*(n+1) ints at
+  // scratch_off[b], b the tree's block of this launch (null: no such tree).
+  int32_t* scratch;
+  const int64_t* scratch_off;
   int32_t first_tree;
 };
-void launch_tree_prep(const PrepArgs& a, int ntrees, hipStream_t s);
+// Working arrays of n + 1 ints per tree, and the nodes of which they fit LDS.
+constexpr int kPrepArrays = 7;
+constexpr int kPrepLdsNodes = 150 * 1024 / (4 * kPrepArrays) - 1;  // 5485
+// maxn: the largest tree's nodes.
+void launch_tree_prep(const PrepArgs& a, int ntrees, int maxn, hipStream_t s);
+hipError_t prep_init_attributes();
 
 // Cost prefix sums of trees [first_tree, first_tree + ntrees): per node i in
 // [0, n], pdel[off + i] / pins[off + i] = the deletion / insertion costs of
