@@ -522,11 +522,16 @@ int Context::plan(Group& g, int32_t npairs, const int32_t* xs, const int32_t* ys
       g.leaf_tables += (int64_t)a.K1 * b.K + (int64_t)(a.K - a.K1) * b.K1;
       g.leaf_cells += (int64_t)a.K1 * info_[y].ksum + (int64_t)b.K1 * (info_[x].ksum - a.K1);
     }
-    blk[i + 1] = blk[i] + plan_blocks(ka, kb, plan_chunk);
     planned += (int64_t)ka * kb;
     nlevels = std::max(nlevels, a.kdmax + b.kdmax + 1);
     st.tables += (int64_t)a.K * b.K;
     st.cells += info_[x].ksum * info_[y].ksum;
+  }
+  const int32_t plan_chunk = plan_chunk_tables(planned);
+  for (int32_t i = 0; i < npairs; ++i) {
+    const TreeMeta &a = meta_[xs[i]], &b = meta_[ys[i]];
+    const int32_t leaves_out = leaf[i] ? 1 : 0;
+    blk[i + 1] = blk[i] + plan_blocks(a.K - leaves_out * a.K1, b.K - leaves_out * b.K1, plan_chunk);
   }
   g.td_bytes = (int64_t)sizeof(td_t) * td_total;
   const int nb = nlevels * kNumClasses * kBands;

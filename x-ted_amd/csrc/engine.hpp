@@ -237,7 +237,6 @@ class Context {
   int32_t lds_limit = 0;  // device's dynamic LDS per workgroup for the slots
   int32_t force_class = -1;
   int32_t lane_enable = 1;
-  int32_t plan_chunk = 2048;  // tables per plan block
   int32_t profile = 0;        // time every forest launch with events
   int32_t level_streams = kMaxLevelStreams;  // streams one level's launches spread over
   // Levels reached by at most this many pairs of a batch take the latency

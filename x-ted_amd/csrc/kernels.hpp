@@ -101,6 +101,14 @@ inline int64_t plan_blocks(int32_t Kx, int32_t Ky, int32_t chunk) {
   const int32_t lper = chunk / (Kx > 0 ? Kx : 1) > 0 ? chunk / (Kx > 0 ? Kx : 1) : 1;
   return (Ky + lper - 1) / lper;
 }
+// Tables per plan block: at most kPlanChunk, fewer in a plan of few tables,
+// whose time is one block's; at least one pass of a block's threads.
+constexpr int kPlanChunk = 2048;
+inline int32_t plan_chunk_tables(int64_t tables) {
+  int32_t c = kPlanChunk;
+  while (c > 256 && tables < (int64_t)c * 512) c /= 2;
+  return c;
+}
 void launch_plan(const PlanArgs& a, int64_t nblocks, hipStream_t s);
 constexpr int32_t kDistAborted = INT32_MIN;  // what a gather writes for a group that gave up
 void launch_gather_dist(const PairMeta* pairs, const td_t* td, int32_t npairs,

@@ -100,37 +100,12 @@ __device__ __forceinline__ void classify(const PlanArgs& A, const TreeMeta& tx,
   *j0 = (uint32_t)A.pool.skr[ly];
 }
 
-#define DPP_ROW_SHR(n) (0x110 + (n))
-#define DPP_ROW_BCAST15 0x142
-#define DPP_ROW_BCAST31 0x143
-
-// Wave-wide sum / max of 32-bit values, result in every lane (DPP prefix,
-// then lane 63 broadcast).
-__device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
-  v += __builtin_amdgcn_update_dpp(0u, v, DPP_ROW_SHR(1), 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0u, v, DPP_ROW_SHR(2), 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0u, v, DPP_ROW_SHR(4), 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0u, v, DPP_ROW_SHR(8), 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0u, v, DPP_ROW_BCAST15, 0xa, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0u, v, DPP_ROW_BCAST31, 0xc, 0xf, false);
-  return __builtin_amdgcn_readlane(v, 63);
-}
-__device__ __forceinline__ int32_t wave_max_i32(int32_t v) {
-  v = max(v, __builtin_amdgcn_update_dpp(0, v, DPP_ROW_SHR(1), 0xf, 0xf, false));
-  v = max(v, __builtin_amdgcn_update_dpp(0, v, DPP_ROW_SHR(2), 0xf, 0xf, false));
-  v = max(v, __builtin_amdgcn_update_dpp(0, v, DPP_ROW_SHR(4), 0xf, 0xf, false));
-  v = max(v, __builtin_amdgcn_update_dpp(0, v, DPP_ROW_SHR(8), 0xf, 0xf, false));
-  v = max(v, __builtin_amdgcn_update_dpp(0, v, DPP_ROW_BCAST15, 0xa, 0xf, false));
-  v = max(v, __builtin_amdgcn_update_dpp(0, v, DPP_ROW_BCAST31, 0xc, 0xf, false));
-  return __builtin_amdgcn_readlane(v, 63);
-}
-
 // Per-workgroup bucket table in LDS: the plan's global atomics go to a few
 // thousand (level, class) buckets and device-scope atomics are performed
-// memory-side, so a wave's per-bucket partials are first combined per
-// workgroup (open addressing on the bucket id), and each workgroup then
-// makes one global atomic per bucket it touched. A bucket that finds the
-// table full takes the global atomics directly.
+// memory-side, so they are first combined per workgroup (open addressing on
+// the bucket id), and each workgroup then makes one global atomic per bucket
+// it touched. A bucket that finds the table full takes the global atomics
+// directly.
 constexpr int kHTBits = 8;
 constexpr int kHT = 1 << kHTBits;
 struct PlanLds {
@@ -143,8 +118,12 @@ struct PlanLds {
 __device__ __forceinline__ int ht_slot(PlanLds& T, int bucket, bool insert) {
   int h = (int)(((uint32_t)bucket * 0x9E3779B1u) >> (32 - kHTBits));
   for (int probe = 0; probe < kHT; ++probe) {
-    const int k = insert ? atomicCAS(&T.key[h], -1, bucket) : T.key[h];
-    if (k == bucket || (insert && k == -1)) return h;
+    int k = __hip_atomic_load(&T.key[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (k == -1 && insert) {
+      k = atomicCAS(&T.key[h], -1, bucket);
+      if (k == -1) return h;
+    }
+    if (k == bucket) return h;
     if (k == -1) return -1;  // lookup: absent
     h = (h + 1) & (kHT - 1);
   }
@@ -185,81 +164,36 @@ __device__ __forceinline__ PlanChunk plan_chunk(const PlanArgs& A, const TreeMet
   return c;
 }
 
-// Count pass: per distinct bucket of a wave, the table count, the interior
-// cells (a table has < 2^30 cells; the wave sum is taken over 16-bit halves
-// so 32-bit sums cannot overflow) and the largest slot-storage need, added
-// into the workgroup's table.
-__device__ __forceinline__ void wave_count(const PlanArgs& A, PlanLds& T, int bucket, bool active,
-                                           uint32_t cells, int32_t lds) {
-  unsigned long long todo = __ballot(active);
-  const int lane = (int)(threadIdx.x & 63);
-  while (todo) {
-    const int leader = __ffsll((long long)todo) - 1;
-    const int lb = __shfl(bucket, leader);
-    const bool mine = active && bucket == lb;
-    const unsigned long long same = __ballot(mine);
-    const uint32_t lo = wave_sum_u32(mine ? (cells & 0xFFFFu) : 0u);
-    const uint32_t hi = wave_sum_u32(mine ? (cells >> 16) : 0u);
-    const int32_t mx = wave_max_i32(mine ? lds : 0);
-    if (lane == leader) {
-      const unsigned long long n = (unsigned long long)__popcll(same);
-      const unsigned long long sum = ((unsigned long long)hi << 16) + lo;
-      const int h = ht_slot(T, lb, true);
-      if (h >= 0) {
-        atomicAdd(&T.cnt[h], (uint32_t)n);
-        atomicAdd(&T.cells[h], sum);
-        atomicMax(&T.lds[h], mx);
-      } else {
-        atomicAdd(&A.counts[lb], n);
-        atomicAdd(&A.cells[lb], sum);
-        if (mx > 0) atomicMax(&A.maxlds[lb], mx);
-      }
-    }
-    todo &= ~same;
+// Count pass: one table's count, interior cells and slot-storage need, into
+// the workgroup's table. (LDS atomics of lanes on one entry are performed one
+// after another, a cycle each: less than the wave-wide sums per distinct
+// bucket that would merge them, with some 6 distinct buckets among 64 tables.)
+__device__ __forceinline__ void count_table(const PlanArgs& A, PlanLds& T, int bucket,
+                                            unsigned long long cells, int32_t lds) {
+  const int h = ht_slot(T, bucket, true);
+  if (h >= 0) {
+    atomicAdd(&T.cnt[h], 1u);
+    atomicAdd(&T.cells[h], cells);
+    atomicMax(&T.lds[h], lds);
+  } else {
+    atomicAdd(&A.counts[bucket], 1ull);
+    atomicAdd(&A.cells[bucket], cells);
+    if (lds > 0) atomicMax(&A.maxlds[bucket], lds);
   }
 }
 
-// Scatter pass, first sweep: tables per distinct bucket into the table.
-__device__ __forceinline__ void wave_tally(PlanLds& T, int bucket, bool active) {
-  unsigned long long todo = __ballot(active);
-  const int lane = (int)(threadIdx.x & 63);
-  while (todo) {
-    const int leader = __ffsll((long long)todo) - 1;
-    const int lb = __shfl(bucket, leader);
-    const unsigned long long same = __ballot(active && bucket == lb);
-    if (lane == leader) {
-      const int h = ht_slot(T, lb, true);
-      if (h >= 0) atomicAdd(&T.cnt[h], (uint32_t)__popcll(same));
-    }
-    todo &= ~same;
-  }
+// Scatter pass, first sweep: tables per bucket into the table.
+__device__ __forceinline__ void tally_table(PlanLds& T, int bucket) {
+  const int h = ht_slot(T, bucket, true);
+  if (h >= 0) atomicAdd(&T.cnt[h], 1u);
 }
 
 // Scatter pass, second sweep: this lane's slot, from the workgroup's range
 // of the bucket (or, for a bucket not in the table, a global reservation).
-__device__ __forceinline__ unsigned long long wave_reserve(const PlanArgs& A, PlanLds& T,
-                                                           int bucket, bool active) {
-  unsigned long long pos = 0;
-  const unsigned long long lt = __lanemask_lt();
-  unsigned long long todo = __ballot(active);
-  const int lane = (int)(threadIdx.x & 63);
-  while (todo) {
-    const int leader = __ffsll((long long)todo) - 1;
-    const int lb = __shfl(bucket, leader);
-    const bool mine = active && bucket == lb;
-    const unsigned long long same = __ballot(mine);
-    unsigned long long base = 0;
-    if (lane == leader) {
-      const uint32_t n = (uint32_t)__popcll(same);
-      const int h = ht_slot(T, lb, false);
-      base = h >= 0 ? T.cells[h] + atomicAdd(&T.cnt[h], n)
-                    : atomicAdd(&A.cursor[lb], (unsigned long long)n);
-    }
-    base = __shfl(base, leader);
-    if (mine) pos = base + __popcll(same & lt);
-    todo &= ~same;
-  }
-  return pos;
+__device__ __forceinline__ unsigned long long reserve_table(const PlanArgs& A, PlanLds& T,
+                                                            int bucket) {
+  const int h = ht_slot(T, bucket, false);
+  return h >= 0 ? T.cells[h] + atomicAdd(&T.cnt[h], 1u) : atomicAdd(&A.cursor[bucket], 1ull);
 }
 
 // The start-up values of table (i0, j0) of a pair.
@@ -285,9 +219,18 @@ __device__ __forceinline__ TaskDesc make_desc(const PlanArgs& A, const PairMeta&
   return d;
 }
 
+// What bounds the passes: the loads that classify a table. So the scatter pass
+// keeps its tables' buckets in LDS between its two sweeps, and a plan of few
+// tables goes in small chunks (plan_chunk_tables).
+// Count and scatter pass, us, with wave-wide sums per distinct bucket, every
+// sweep classifying, and 2048 tables a chunk whatever the plan, against now:
+// RRT 100-node pair 31 + 48, now 7 + 8; deep 1000-node pair 68 + 105, 12 + 10;
+// 4096 pairs of 100-1000 nodes 2764 + 3259, 1188 + 2539 (the scatter writes 72
+// bytes a table).
 template <bool kScatter>
 __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs A) {
   __shared__ PlanLds T;
+  __shared__ int32_t bucket_at[kScatter ? kPlanChunk : 1];
   const int p = find_pair(A.blk_start, A.npairs, blockIdx.x);
   const PairMeta pm = A.pairs[p];
   const TreeMeta tx = A.pool.trees[pm.tx], ty = A.pool.trees[pm.ty];
@@ -299,7 +242,8 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs A) {
   // Table idx of the chunk is (l, k) = (idx / Kx, idx % Kx); a chunk holds
   // at most max(lchunk_tables, Kx) < 2^15 tables. One division per thread,
   // then each step of kPlanThreads tables adds (dl, dk) with one carry.
-  auto sweep = [&](auto body) {
+  const bool kept = ch.total <= kPlanChunk;  // in bucket_at (a lane reads back what it wrote)
+  auto sweep = [&](bool again, auto body) {
     const int32_t total = (int32_t)ch.total;
     const int32_t kx = max(ch.Kx, 1);
     const int32_t dl = kPlanThreads / kx, dk = kPlanThreads % kx;
@@ -309,9 +253,15 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs A) {
       int bucket = 0, lds = 0;
       uint32_t i0 = 0, j0 = 0;
       unsigned long long cells = 0;
-      if (active)
-        classify(A, tx, ty, loff, leaf_form, ch.kbase + kr, ch.lbase + ch.l_lo + lq, &bucket,
-                 &lds, &i0, &j0, &cells);
+      const int k = ch.kbase + kr, l = ch.lbase + ch.l_lo + lq;
+      if (active && again && kept) {
+        bucket = bucket_at[base + threadIdx.x];
+        i0 = (uint32_t)A.pool.skr[tx.node_off + k];
+        j0 = (uint32_t)A.pool.skr[ty.node_off + l];
+      } else if (active) {
+        classify(A, tx, ty, loff, leaf_form, k, l, &bucket, &lds, &i0, &j0, &cells);
+        if (kScatter && kept) bucket_at[base + threadIdx.x] = bucket;
+      }
       body(active, bucket, lds, i0, j0, cells);
       lq += dl;
       kr += dk;
@@ -322,8 +272,8 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs A) {
     }
   };
   if (!kScatter) {
-    sweep([&](bool active, int bucket, int lds, uint32_t, uint32_t, unsigned long long cells) {
-      wave_count(A, T, bucket, active, (uint32_t)cells, lds);
+    sweep(false, [&](bool active, int bucket, int lds, uint32_t, uint32_t, unsigned long long cells) {
+      if (active) count_table(A, T, bucket, cells, lds);
     });
     __syncthreads();
     for (int h = threadIdx.x; h < kHT; h += kPlanThreads) {
@@ -334,8 +284,8 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs A) {
       if (T.lds[h] > 0) atomicMax(&A.maxlds[b], T.lds[h]);
     }
   } else {
-    sweep([&](bool active, int bucket, int, uint32_t, uint32_t, unsigned long long) {
-      wave_tally(T, bucket, active);
+    sweep(false, [&](bool active, int bucket, int, uint32_t, uint32_t, unsigned long long) {
+      if (active) tally_table(T, bucket);
     });
     __syncthreads();
     // One range per bucket for the workgroup; cnt becomes its cursor.
@@ -346,9 +296,9 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs A) {
       T.cnt[h] = 0;
     }
     __syncthreads();
-    sweep([&](bool active, int bucket, int, uint32_t i0, uint32_t j0, unsigned long long) {
-      const unsigned long long pos = wave_reserve(A, T, bucket, active);
+    sweep(true, [&](bool active, int bucket, int, uint32_t i0, uint32_t j0, unsigned long long) {
       if (active) {
+        const unsigned long long pos = reserve_table(A, T, bucket);
         const TaskDesc d = make_desc(A, pm, tx, ty, (int32_t)i0, (int32_t)j0);
         A.descs[pos] = d;
         A.tasks[pos] = task_pack((uint32_t)ch.p, i0, j0, d.base_rx < 0);
