@@ -103,6 +103,10 @@ Context::~Context() {
   }
   for (Group& g : batch_) g.release();
   na_.release();
+  if (tables_pin_) {
+    (void)hipHostFree(tables_pin_);
+    for (hipEvent_t e : tables_ev_) (void)hipEventDestroy(e);
+  }
   for (DevBuf* b : {&parent_, &label_, &orl_, &kdep_, &kdn_, &lrank_, &kr_, &krkd_, &krsize_,
                     &krleaf_, &trees_, &prep_scratch_, &prep_off_, &skr_, &skd_, &ssize_, &sleaf_,
                     &spre_, &kdoff_, &rtop_, &cdel_, &cins_, &cren_, &pdel_, &pins_, &ctot_, &crec_,
@@ -1047,6 +1051,87 @@ int Context::run_levels(Group& g, int lane, std::vector<ProfLaunch>* prof) {
   return OK;
 }
 
+// Tables leave the device as they lie in the arena, 16 bits an entry, into two
+// halves of a pinned buffer, and are widened to the caller's int32 by a few
+// host threads, one half while the other is filled; while the levels run, the
+// same threads touch the caller's pages. (Widened on the device and copied to
+// the caller's pageable memory, the 62 MB of 128 pairs' tables took 7.5 ms
+// after the last level, one copy and one host thread's page faults after
+// another; now 2.0.)
+int Context::copy_tables(Group& g, const std::vector<int32_t*>& outs, hipStream_t s) {
+  struct Piece {
+    const td_t* src;  // device, then its place in the pinned buffer
+    int32_t* out;
+    int64_t n;
+  };
+  constexpr int64_t kPiece = 64 * 1024, kPage = 4096;
+  std::vector<Piece> pieces;
+  for (size_t j = 0; j < outs.size(); ++j) {
+    if (!outs[j]) continue;
+    const int64_t mn = (int64_t)meta_[g.xs[j]].n * meta_[g.ys[j]].n;
+    const td_t* td = g.td.as<td_t>() + g.pm[j].td_off;
+    for (int64_t at = 0; at < mn; at += kPiece)
+      pieces.push_back(Piece{td + at, outs[j] + at, std::min(kPiece, mn - at)});
+  }
+  if (pieces.empty()) return OK;
+  if (!tables_pin_) {
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&tables_pin_), 2 * kTablesHalf * sizeof(td_t),
+                          hipHostMallocDefault));
+    for (hipEvent_t& e : tables_ev_) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  }
+  size_t next = 0, end[2] = {0, 0};
+  // Pieces [next, end[h]) go to half h, neighbours in the arena in one copy.
+  auto fill = [&](int h) -> int {
+    int64_t used = 0;
+    end[h] = next;
+    while (end[h] < pieces.size() && used + pieces[end[h]].n <= kTablesHalf) {
+      const td_t* src = pieces[end[h]].src;
+      td_t* dst = tables_pin_ + h * kTablesHalf + used;
+      int64_t n = 0;
+      do {
+        pieces[end[h]].src = dst + n;
+        n += pieces[end[h]++].n;
+      } while (end[h] < pieces.size() && pieces[end[h]].src == src + n &&
+               used + n + pieces[end[h]].n <= kTablesHalf);
+      HIP_TRY(hipMemcpyAsync(dst, src, sizeof(td_t) * n, hipMemcpyDeviceToHost, s));
+      used += n;
+    }
+    HIP_TRY(hipEventRecord(tables_ev_[h], s));
+    next = end[h];
+    return OK;
+  };
+  // Tables that a caller has overlap are written one after another, in order.
+  std::vector<std::pair<int32_t*, int64_t>> spans;
+  for (const Piece& p : pieces) spans.push_back({p.out, p.n});
+  std::sort(spans.begin(), spans.end());
+  bool apart = true;
+  for (size_t i = 1; i < spans.size(); ++i)
+    apart = apart && spans[i - 1].first + spans[i - 1].second <= spans[i].first;
+  auto each = [&](size_t n, const std::function<void(int64_t)>& fn) {
+    if (apart) host_pool_.run((int64_t)n, fn);
+    else for (size_t i = 0; i < n; ++i) fn((int64_t)i);
+  };
+  size_t begin = 0;
+  ST_TRY(fill(0));
+  ST_TRY(fill(1));
+  each(pieces.size(), [&](int64_t i) {
+    volatile char* p = reinterpret_cast<volatile char*>(pieces[i].out);
+    const int64_t bytes = pieces[i].n * (int64_t)sizeof(int32_t);
+    for (int64_t at = 0; at < bytes; at += kPage) p[at] = p[at];
+    p[bytes - 1] = p[bytes - 1];
+  });
+  for (int h = 0; begin < pieces.size(); h ^= 1) {
+    HIP_TRY(hipEventSynchronize(tables_ev_[h]));
+    each(end[h] - begin, [&](int64_t i) {
+      const Piece& p = pieces[begin + i];
+      for (int64_t k = 0; k < p.n; ++k) p.out[k] = p.src[k];
+    });
+    begin = end[h];
+    if (next < pieces.size()) ST_TRY(fill(h));
+  }
+  return OK;
+}
+
 int Context::run_batch(int32_t npairs, const int32_t* xs, const int32_t* ys, int32_t* dist,
                        int32_t* const* td_out, BatchStats* stats) {
   std::lock_guard<std::mutex> lk(mu_);
@@ -1099,28 +1184,22 @@ int Context::run_batch(int32_t npairs, const int32_t* xs, const int32_t* ys, int
     launch_gather_dist(g.pairs.as<PairMeta>(), g.td.as<td_t>(), g.npairs,
                        g.abort.as<int32_t>(), g.dist.as<int32_t>(), s);
     HIP_TRY(hipGetLastError());
+  }
+  if (td_out) {
+    for (int k = 0; k < ng; ++k) {
+      std::vector<int32_t*> outs(batch_[k].npairs);
+      for (size_t j = 0; j < outs.size(); ++j) outs[j] = td_out[idx[k][j]];
+      ST_TRY(copy_tables(batch_[k], outs, lane_stream(ng > 1 ? k : -1)));
+    }
+  }
+  for (int k = 0; k < ng; ++k) {
+    Group& g = batch_[k];
+    hipStream_t s = lane_stream(ng > 1 ? k : -1);
     HIP_TRY(hipMemcpyAsync(gd[k].data(), g.dist.p, sizeof(int32_t) * g.npairs,
                            hipMemcpyDeviceToHost, s));
     if (g.nxl > 0)
       HIP_TRY(hipMemcpyAsync(aborted[k].data(), g.abort.p, sizeof(int32_t) * kAbortInts,
                              hipMemcpyDeviceToHost, s));
-    if (td_out) {
-      // Each requested table is widened to int32 in a staging buffer, then
-      // copied out (in stream order, so the next widening waits for it).
-      int64_t most = 0;
-      for (int32_t j = 0; j < g.npairs; ++j)
-        if (td_out[idx[k][j]])
-          most = std::max(most, (int64_t)meta_[g.xs[j]].n * meta_[g.ys[j]].n);
-      if (most > 0) ST_TRY(g.tdw.grow(sizeof(int32_t) * (size_t)most, false, s));
-      for (int32_t j = 0; j < g.npairs; ++j) {
-        int32_t* out = td_out[idx[k][j]];
-        if (!out) continue;
-        const int64_t mn = (int64_t)meta_[g.xs[j]].n * meta_[g.ys[j]].n;
-        launch_widen_td(g.td.as<td_t>() + g.pm[j].td_off, g.tdw.as<int32_t>(), mn, s);
-        HIP_TRY(hipGetLastError());
-        HIP_TRY(hipMemcpyAsync(out, g.tdw.p, sizeof(int32_t) * mn, hipMemcpyDeviceToHost, s));
-      }
-    }
   }
   for (int k = 0; k < ng; ++k) HIP_TRY(hipStreamSynchronize(lane_stream(ng > 1 ? k : -1)));
   for (int k = 0; k < ng; ++k) {

@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "device.hpp"
+#include "host_pool.hpp"
 #include "trees.hpp"
 
 namespace xted {
@@ -99,7 +100,6 @@ struct Group {
   std::vector<uint8_t> h_tail;
   DevBuf pairs, blk, counts, cells, cursor, maxlds, tickets, tasks, descs, td, dist, lines_d,
       tail_lv, level_cells, xl_off, xl_total, loff_d, leaf_d;
-  DevBuf tdw;  // requested tables widened to int32 on their way out
   DevBuf abort, xl_words;
   // finish_async: distances then the abort flag land in pinned memory
   int32_t* h_dist_pin = nullptr;
@@ -123,7 +123,7 @@ struct Group {
   void for_each_buf(F f) {
     for (DevBuf* b : {&pairs, &blk, &counts, &cells, &cursor, &maxlds, &tickets, &abort, &tasks,
                       &descs, &td, &dist, &lines_d, &tail_lv, &level_cells, &xl_off, &xl_total,
-                      &xl_words, &loff_d, &leaf_d, &tdw})
+                      &xl_words, &loff_d, &leaf_d})
       f(*b);
   }
 };
@@ -297,6 +297,13 @@ class Context {
   DevBuf skr_, skd_, ssize_, sleaf_, spre_, kdoff_, rtop_, crec_, rrec_, ccrec_;
   DevBuf prep_scratch_, prep_off_;
   Group batch_[kMaxLevelStreams];  // the groups run_batch reuses
+  // Copies group g's tables to outs[j] (null: not wanted) after what stream s
+  // holds, and waits for them.
+  int copy_tables(Group& g, const std::vector<int32_t*>& outs, hipStream_t s);
+  static constexpr int64_t kTablesHalf = 2 << 20;  // entries of half the pinned buffer
+  td_t* tables_pin_ = nullptr;
+  hipEvent_t tables_ev_[2] = {};
+  HostPool host_pool_;
   Group na_;                        // run_batch_noalloc's group, bound to na_arena_
   std::vector<void*> retired_;      // see retire_list()
   Arena na_arena_;                  // this device's fixed array (kNoAllocArray)

@@ -113,10 +113,6 @@ void launch_plan(const PlanArgs& a, int64_t nblocks, hipStream_t s);
 constexpr int32_t kDistAborted = INT32_MIN;  // what a gather writes for a group that gave up
 void launch_gather_dist(const PairMeta* pairs, const td_t* td, int32_t npairs,
                         const int32_t* abort_flag, int32_t* dist, hipStream_t s);
-// dst[i] = src[i] for i < n: a table of the arena widened to the int32 a
-// caller receives.
-void launch_widen_td(const td_t* src, int32_t* dst, int64_t n, hipStream_t s);
-
 // Tables with a leaf keyroot, in closed form. For a single node v and a
 // subtree T (unit costs), TED({v}, T) = |T| - [label(v) occurs in T]: map v
 // onto a node of T with its label if there is one, insert the rest. So the

@@ -403,17 +403,4 @@ void launch_gather_dist(const PairMeta* pairs, const td_t* td, int32_t npairs,
                      npairs, abort_flag, dist);
 }
 
-__global__ __launch_bounds__(256) void widen_td_kernel(const td_t* __restrict__ src,
-                                                       int32_t* __restrict__ dst, int64_t n) {
-  const int64_t step = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += step)
-    dst[i] = src[i];
-}
-
-void launch_widen_td(const td_t* src, int32_t* dst, int64_t n, hipStream_t s) {
-  if (n <= 0) return;
-  const int64_t blocks = std::min<int64_t>((n + 255) / 256, 8192);
-  hipLaunchKernelGGL(widen_td_kernel, dim3((unsigned)blocks), dim3(256), 0, s, src, dst, n);
-}
-
 }  // namespace xted
