@@ -151,8 +151,17 @@ int Context::init() {
   hipDeviceProp_t prop;
   HIP_TRY(hipGetDeviceProperties(&prop, device_));
   lds_limit = (int32_t)std::min<size_t>(kLdsMaxTable, prop.sharedMemPerBlock - 256);
-  HIP_TRY(forest_init_attributes(lds_limit));
-  HIP_TRY(prep_init_attributes());
+  {
+    // The kernels' LDS limits hold for the process and device: set once.
+    static std::mutex mu;
+    static std::vector<int> set;
+    std::lock_guard<std::mutex> once(mu);
+    if (std::find(set.begin(), set.end(), device_) == set.end()) {
+      HIP_TRY(forest_init_attributes(lds_limit));
+      HIP_TRY(prep_init_attributes());
+      set.push_back(device_);
+    }
+  }
   rule.lds_max = lds_limit;
   // This device's copy of the no-allocation array, and what its batch group
   // needs besides memory, so that run_batch_noalloc creates nothing.

@@ -307,27 +307,41 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs A) {
   }
 }
 
-// Exclusive scan of the bucket counts into the scatter cursors (one block).
+// Exclusive scan of the bucket counts into the scatter cursors (one block):
+// 4096 buckets a round, 4 a thread in one 32-byte read, so that the reads are
+// whole lines in flight together. (A contiguous run of buckets per thread, one
+// dependent read after another, took 433 us for the 38,720 buckets of the
+// 4096-pair batch and 37 us for a deep 1000-node pair's 21,120; now 85 and 14.)
 __global__ __launch_bounds__(1024) void plan_scan_kernel(const unsigned long long* counts,
                                                           unsigned long long* cursor, int nb) {
-  __shared__ unsigned long long part[1024];
-  const int tid = threadIdx.x;
-  const int per = (nb + 1023) / 1024;
-  const int lo = min(nb, tid * per), hi = min(nb, lo + per);
-  unsigned long long s = 0;
-  for (int i = lo; i < hi; ++i) s += counts[i];
-  part[tid] = s;
-  __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {
-    unsigned long long v = tid >= off ? part[tid - off] : 0;
-    __syncthreads();
-    part[tid] += v;
-    __syncthreads();
-  }
-  unsigned long long run = tid ? part[tid - 1] : 0;
-  for (int i = lo; i < hi; ++i) {
-    cursor[i] = run;
-    run += counts[i];
+  __shared__ unsigned long long part[2][16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  unsigned long long before = 0;  // the counts of earlier rounds
+  for (int b0 = 0, r = 0; b0 < nb; b0 += 4096, r ^= 1) {
+    const int b = b0 + 4 * tid;
+    unsigned long long c[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) c[i] = b + i < nb ? counts[b + i] : 0;
+    const unsigned long long sum = c[0] + c[1] + c[2] + c[3];
+    unsigned long long incl = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const unsigned long long v = __shfl_up(incl, d);
+      if (lane >= d) incl += v;
+    }
+    if (lane == 63) part[r][wave] = incl;
+    __syncthreads();  // (two parts: the round before may still be read)
+    unsigned long long run = before + incl - sum;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+      run += w < wave ? part[r][w] : 0;
+      before += part[r][w];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (b + i < nb) cursor[b + i] = run;
+      run += c[i];
+    }
   }
 }
 
