@@ -163,8 +163,15 @@ XTED_HD constexpr int xl_cpl(int k) { return k == 0 ? 8 : k == 1 || k == 4 ? 4 :
 XTED_HD inline int xl_bw(int k) { return 64 * xl_waves(k) * xl_cpl(k); }  // 4096 .. 128
 // Column-blocked tables with at most this many rows are swept block after
 // block by one workgroup (forms of at most 1024 columns), with no waits
-// between workgroups; taller ones pipeline one workgroup per block.
-constexpr int32_t kXLSeqRows = 256;  // default of ClassRule::xl_seq_rows
+// between workgroups; taller ones pipeline one workgroup per block. Measured
+// on the 20,000-node pair's tables of more than 8192 columns, ms a pair with
+// 256, 128, 64, 32 and 16 rows: 76.9, 75.1, 74.1, 73.7, 74.0.
+constexpr int32_t kXLSeqRows = 32;  // default of ClassRule::xl_seq_rows
+// A table that fits one workgroup goes in blocks for being tall only above
+// this: filling the pipeline of blocks takes about 16 rows and 3 us a block
+// (tables of up to 237 rows and 4999 columns, ms a pair: 12.8 in one
+// workgroup, 15.1 in blocks).
+constexpr int32_t kTallBlockRows = 256;
 constexpr int kFirstSeqXLForm = 2;
 // Far values a block takes from earlier blocks are indexed by the nesting
 // depth of their right path below the column keyroot: at most this many.
@@ -381,7 +388,7 @@ XTED_HD inline int table_class(int a, int b, int kd_r, int kd_c, int leaves_c, b
   };
   // Tall tables go in blocks where they are wider than one, and where LDS
   // leaves them more columns per lane.
-  if (tall && rule.blocks && rows > rule.xl_seq_rows &&
+  if (tall && rule.blocks && rows > kTallBlockRows && rows > rule.xl_seq_rows &&
       (cols > xl_bw(first_tall) || cols > 64 * tall * (1 << wi))) {
     const int cls = blocked(first);
     if (cls != kClassXL) return cls;
