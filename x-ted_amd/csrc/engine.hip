@@ -456,8 +456,12 @@ void Group::release() {
 
 int Context::lane_streams(int lane, hipStream_t* out) const {
   if (lane >= 0 && lane < kMaxLevelStreams) {
-    out[0] = lane == 0 ? stream_ : side_[lane - 1];
-    return 1;
+    auto of = [&](int l) { return l == 0 ? stream_ : side_[l - 1]; };
+    int n = 0;
+    out[n++] = of(lane);
+    for (int l = 0; l < kMaxLevelStreams; ++l)
+      if (l != lane && (lent_streams >> l & 1) && n < level_streams) out[n++] = of(l);
+    return n;
   }
   out[0] = stream_;
   for (int k = 1; k < kMaxLevelStreams; ++k) out[k] = side_[k - 1];

@@ -208,8 +208,8 @@ class Context {
   // The steps of run_batch, for callers that interleave several groups (the
   // server). The caller holds mutex() across them.
   // Plans pairs (xs[i], ys[i]) into g: device plan, one sync for the counts.
-  // lane: -1 = all streams (a batch); 0 .. kMaxLevelStreams-1 = server lanes,
-  // one stream each, whose ticks run independently of each other.
+  // lane: -1 = all streams (a batch); 0 .. kMaxLevelStreams-1 = that stream
+  // (and lent_streams), independently of the others'.
   int plan(Group& g, int32_t npairs, const int32_t* xs, const int32_t* ys, int lane = -1);
   // One tick: launches the next level of every group in gs (groups past
   // their last level are skipped) and advances them. Asynchronous.
@@ -227,6 +227,9 @@ class Context {
   std::vector<void*>* retire_list() { return &retired_; }
   int release_retired();
   hipStream_t lane_stream(int lane) const;  // where a lane's ticks end
+  // Streams (bit l: lane l's) that the next tick of a lane spreads over besides
+  // its own. Set around launch_levels, under mutex().
+  uint32_t lent_streams = 0;
   int lane_streams(int lane, hipStream_t* out) const;
   int poll(Group& g, bool wait, int32_t* dist);
 

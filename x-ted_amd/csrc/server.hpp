@@ -8,12 +8,11 @@
 // group in flight together (levels of different groups are independent, so
 // their tables share the same launches' streams); a group whose last level
 // has run publishes its results and frees its share of the budget. So a
-// query that arrives while others are on the device starts within a tick.
-// A tick lasts as long as its slowest table, so groups run in lanes with
-// ticks of their own, one stream each: light pairs (the smaller tree at
-// most kLightSide nodes and at most kLightLevels levels) in lane 0, heavy
-// ones in the least-loaded of lanes 1..3; a light pair never waits for a
-// tick of a heavy one, and heavy groups only share ticks within a lane.
+// query that arrives while others are on the device starts within a few ticks.
+// A tick lasts as long as its slowest table, so groups run in two lanes with
+// ticks and streams of their own: light pairs (the smaller tree at most
+// kLightSide nodes and at most kLightLevels levels) in lane 0, heavy ones in
+// lane 1; a light pair never waits for a tick of a heavy one.
 #pragma once
 #include <chrono>
 #include <condition_variable>
@@ -53,7 +52,8 @@ class Server {
     Clock::time_point t_submit;
     int64_t bytes;
   };
-  static constexpr int kLanes = kMaxLevelStreams;
+  static constexpr int kLanes = 2;
+  static constexpr std::chrono::microseconds kAdmitPace{2000};
   struct Active {
     std::unique_ptr<Group> g;
     std::vector<Req> reqs;
@@ -75,6 +75,7 @@ class Server {
   struct Lane {
     std::vector<Active> active;
     std::deque<hipEvent_t> ticks;
+    Clock::time_point next_admit{};  // not before, while groups are active
   };
   Lane lanes_[kLanes];
   std::vector<Active> completing_;             // gathers enqueued, not landed
