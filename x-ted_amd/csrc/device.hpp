@@ -233,8 +233,6 @@ constexpr int kMaxOnChipCols = 64 * 8 * kMaxRowWaves;  // 8192
 // against 99.6 ms when it was tuned). The 64-lane form ran 8% slower there (4
 // waves per SIMD for its 64 TD registers per lane).
 constexpr int32_t kTinyDefault = 1;
-// Most columns per lane a table takes under a cost model.
-constexpr int32_t kMaxCostCpl = 8;
 
 // A row of up to 256 columns takes one wave about as long as several
 // (a 120-node pair's root table 0.21 us a row either way).

@@ -235,7 +235,9 @@ class Context {
 
   // Tuning / test hooks -----------------------------------------------------
   // (Up to 16 columns per lane: the distance matrix of 96 trees of 100-1000
-  // nodes took 99.9 ms against 110.8 with 8, and 89.4 with level_align 1.)
+  // nodes took 99.9 ms against 110.8 with 8, and 89.4 with level_align 1;
+  // under a cost model, whose 16-column form holds 204 VGPRs, 4096 pairs took
+  // 120 against 146, 1024 pairs 44 against 49.)
   ClassRule rule{kLdsPerWave, 1, 1 << 30, kLdsMaxTable, 16, kXLSeqRows};
   int32_t lds_limit = 0;  // device's dynamic LDS per workgroup for the slots
   int32_t force_class = -1;

@@ -32,16 +32,18 @@ def short(name):
     """'rowscan_w4_c4', 'xl_bw1024', 'rowscan_w4_c4_cost' (the variant under a
     cost model), 'leaf_kernel', ... from a demangled kernel name."""
     base = name.split("(")[0].replace("void ", "").replace("xted::", "")
+    parts = [p.strip() for p in base[base.find("<") + 1:-1].split(",")] if "<" in base else []
+    cost = "_cost" if parts and parts[-1] == "true" else ""
+    if base.startswith("scan_kernel<"):
+        return f"rowscan_w{parts[0]}_c{parts[1]}{cost}"
+    if base.startswith("scan_xl_kernel<"):
+        return f"xl_bw{64 * int(parts[0]) * int(parts[1])}{cost}"
+    if base.startswith("scan_sweep_kernel<"):
+        return f"sweep{cost}"
     if base.startswith("rowscan_kernel<"):
-        parts = [p.strip() for p in base[len("rowscan_kernel<"):-1].split(",")]
-        w, c = int(parts[0]), int(parts[1])
-        cost = "_cost" if len(parts) > 3 and parts[3] == "true" else ""
-        if len(parts) > 2 and parts[2] == "true":
-            return f"xl_bw{64 * w * c}{cost}"
-        return f"rowscan_w{w}_c{c}{cost}"
+        return f"shared_w{parts[0]}_c8{cost}"
     if base.startswith("tiny_kernel<"):
-        parts = [p.strip() for p in base[len("tiny_kernel<"):-1].split(",")]
-        return f"tiny_s{parts[0]}" + ("_cost" if parts[-1] == "true" else "")
+        return f"tiny_s{parts[0]}{cost}"
     return base
 
 
@@ -131,15 +133,18 @@ def resources(src, hipcc="/opt/rocm/bin/hipcc", arch="gfx950"):
                 cur[key] = int(m.group(1))
 
     def pretty(mangled):
-        m = re.search(r"rowscan_kernelILi(\d+)ELi(\d+)ELb([01])ELb([01])", mangled)
+        m = re.search(r"(scan_xl|scan_sweep|rowscan|scan)_kernelI((?:Li\d+E)*)Lb([01])E", mangled)
         if m:
-            w, c, xl, cost = (int(v) for v in m.groups())
-            base = f"xl_bw{64 * w * c}" if xl else f"rowscan_w{w}_c{c}"
-            return base + ("_cost" if cost else "")
+            n = [int(v) for v in re.findall(r"Li(\d+)E", m.group(2))]
+            base = {"scan": "rowscan_w{}_c{}", "scan_xl": "xl_bw{2}", "rowscan": "shared_w{}_c8",
+                    "scan_sweep": "sweep"}[m.group(1)]
+            wide = [64 * n[0] * n[1]] if len(n) == 2 else []
+            return base.format(*n, *wide) + ("_cost" if m.group(3) == "1" else "")
         m = re.search(r"N4xted\d+(\w+?)E", mangled) or re.search(r"4xted(\d+)(\w+)", mangled)
         for name in ("leaf_cost_kernel", "leaf_kernel", "tiny_kernel", "plan_kernel", "tree_prep_kernel",
                      "cost_prefix_kernel", "xl_layout_kernel", "xl_zero_kernel",
-                     "plan_scan_kernel", "plan_clear_kernel", "gather_dist_kernel"):
+                     "plan_scan_kernel", "plan_clear_kernel", "gather_dist_kernel",
+                     "level_cells_kernel"):
             if name in mangled:
                 if name == "tiny_kernel":
                     m = re.search(r"tiny_kernelILi(\d+)ELb([01])E", mangled)
