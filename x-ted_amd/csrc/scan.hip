@@ -45,9 +45,10 @@
 // Measured, us per row of the root table of 1000-node deep / wide pairs, best
 // form of a scan over every row with a barrier per row against this kernel's 8
 // waves of 2 columns per lane: 0.40 / 0.44 against 0.21 / 0.28. Many tables at
-// once (the 4096-pair batch, one stream): one wave of 16 columns 27.3 against
-// 24.4 ms, of 8 18.5 against 16.2, 8 waves of 2 16.2 against 7.4; those are
-// bound by TD traffic (about 2 bytes a cell, 4 TB/s over the batch's streams).
+// once (the 4096-pair batch, one stream, ms): one wave of 16 columns 27.3
+// against 21.6, of 8 18.5 against 14.1, 8 waves of 2 16.2 against 7.4; those
+// are bound by TD traffic (about 2 bytes a cell, 4 TB/s over the batch's
+// streams).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
