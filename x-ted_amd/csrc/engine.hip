@@ -1062,18 +1062,19 @@ int Context::run_levels(Group& g, int lane, std::vector<ProfLaunch>* prof) {
 
 // Tables leave the device as they lie in the arena, 16 bits an entry, into two
 // halves of a pinned buffer, and are widened to the caller's int32 by a few
-// host threads, one half while the other is filled; while the levels run, the
-// same threads touch the caller's pages. (Widened on the device and copied to
-// the caller's pageable memory, the 62 MB of 128 pairs' tables took 7.5 ms
-// after the last level, one copy and one host thread's page faults after
-// another; now 2.0.)
+// host threads, one half while the other is filled. (Widened on the device and
+// copied to the caller's pageable memory, the 62 MB of 128 pairs' tables took
+// 7.5 ms after the last level, one copy and one host thread's page faults after
+// another; now 2.0. Touching the caller's pages with reads and writes while the
+// levels ran was no faster, and 80 ms against 20 on memory never written before,
+// whose zero pages were first mapped and then replaced.)
 int Context::copy_tables(Group& g, const std::vector<int32_t*>& outs, hipStream_t s) {
   struct Piece {
     const td_t* src;  // device, then its place in the pinned buffer
     int32_t* out;
     int64_t n;
   };
-  constexpr int64_t kPiece = 64 * 1024, kPage = 4096;
+  constexpr int64_t kPiece = 64 * 1024;
   std::vector<Piece> pieces;
   for (size_t j = 0; j < outs.size(); ++j) {
     if (!outs[j]) continue;
@@ -1123,12 +1124,6 @@ int Context::copy_tables(Group& g, const std::vector<int32_t*>& outs, hipStream_
   size_t begin = 0;
   ST_TRY(fill(0));
   ST_TRY(fill(1));
-  each(pieces.size(), [&](int64_t i) {
-    volatile char* p = reinterpret_cast<volatile char*>(pieces[i].out);
-    const int64_t bytes = pieces[i].n * (int64_t)sizeof(int32_t);
-    for (int64_t at = 0; at < bytes; at += kPage) p[at] = p[at];
-    p[bytes - 1] = p[bytes - 1];
-  });
   for (int h = 0; begin < pieces.size(); h ^= 1) {
     HIP_TRY(hipEventSynchronize(tables_ev_[h]));
     each(end[h] - begin, [&](int64_t i) {

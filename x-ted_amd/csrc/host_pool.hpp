@@ -1,5 +1,5 @@
 // A few host threads that share a loop with the thread that runs it: tables on
-// their way out are page-faulted in and widened faster than one thread can.
+// their way out are widened faster than one thread can.
 #pragma once
 #include <algorithm>
 #include <atomic>
