@@ -305,7 +305,8 @@ class Context {
   // Copies group g's tables to outs[j] (null: not wanted) after what stream s
   // holds, and waits for them.
   int copy_tables(Group& g, const std::vector<int32_t*>& outs, hipStream_t s);
-  static constexpr int64_t kTablesHalf = 2 << 20;  // entries of half the pinned buffer
+  static constexpr int64_t kTablesHalf = 2 << 20;  // most entries of half the pinned buffer
+  int64_t tables_half_ = 0;                        // and its entries now
   td_t* tables_pin_ = nullptr;
   hipEvent_t tables_ev_[2] = {};
   HostPool host_pool_;
