@@ -87,3 +87,49 @@ def test_server_rejects_unknown_tree():
                 srv.submit(0, 99, 0)
         finally:
             srv.close()
+
+
+def test_light_queries_do_not_wait_for_heavy_ticks():
+    """Light queries that arrive while a heavy pair's ticks (milliseconds each)
+    are on the device take about as long as alone."""
+    with xted.Context(0) as ctx:
+        small = ctx.pool_add([xted.generate(xted.GEN_RRT, 60 + i, 25, xted.derive_seed(95, i))
+                              for i in range(16)])
+        big = ctx.pool_add([xted.generate(xted.GEN_RRT, 20000, 25, xted.derive_seed(95, 50 + i))
+                            for i in range(2)])
+        want = ctx.batch(small[0::2].copy(), small[1::2].copy())[0]
+        heavy_want = int(ctx.batch(big[:1], big[1:])[0][0])
+        srv = xted.Server(ctx, hbm_budget=8 << 30)
+
+        def light(first_tag):
+            """Eight queries, one after another: their latencies, and results
+            of other tags that came in meanwhile."""
+            lat, others = [], {}
+            for k in range(8):
+                srv.submit(int(small[2 * k]), int(small[2 * k + 1]), first_tag + k)
+                while len(lat) == k:
+                    for tag, status, dist, ms, _ in srv.poll(timeout_ms=20):
+                        assert status == 0
+                        if tag == first_tag + k:
+                            assert dist == want[k]
+                            lat.append(ms)
+                        else:
+                            others[tag] = dist
+            return lat, others
+
+        try:
+            light(0)
+            alone = float(np.median(light(100)[0]))
+            beside = []
+            for rep in range(3):
+                srv.submit(int(big[0]), int(big[1]), 1)
+                time.sleep(0.01)  # its first ticks are on the device
+                lat, others = light(200)
+                beside += lat
+                got = others or _drain(srv, 1)
+                dist = got[1] if others else got[1][1]
+                assert dist == heavy_want
+        finally:
+            srv.close()
+    # (Behind two heavy ticks it was 10 to 25 ms.)
+    assert np.median(beside) < max(5 * alone, 5.0), (alone, beside)

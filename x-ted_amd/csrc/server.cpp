@@ -165,6 +165,14 @@ void Server::admit(int lane) {
   L.next_admit = Clock::now() + kAdmitPace * (int)L.active.size();
 }
 
+void Server::reap(Lane& L) {
+  while (!L.ticks.empty() && hipEventQuery(L.ticks.front()) == hipSuccess) {
+    free_ev_.push_back(L.ticks.front());
+    L.ticks.pop_front();
+  }
+  (void)hipGetLastError();  // a not-ready query leaves its status behind
+}
+
 // One tick of a lane: the next level of every group in it. Ticks are
 // enqueued without waiting for them, at most kTicksInFlight ahead of the
 // device; a group whose last level is enqueued gets its distance gather
@@ -172,11 +180,7 @@ void Server::admit(int lane) {
 bool Server::tick(int lane) {
   constexpr int kTicksInFlight = 2;
   Lane& L = lanes_[lane];
-  while (!L.ticks.empty() && hipEventQuery(L.ticks.front()) == hipSuccess) {
-    free_ev_.push_back(L.ticks.front());
-    L.ticks.pop_front();
-  }
-  (void)hipGetLastError();  // a not-ready query leaves its status behind
+  reap(L);
   if (L.active.empty() || (int)L.ticks.size() >= kTicksInFlight) return false;
   std::lock_guard<std::mutex> lk(ctx_->mutex());
   // Groups planned under a cost model that has since changed cannot finish:
@@ -195,14 +199,19 @@ bool Server::tick(int lane) {
   if (L.active.empty()) return false;
   std::vector<Group*> gs;
   for (auto& a : L.active) gs.push_back(a.g.get());
-  // Streams 0 and 1 are the lanes' own; 2 and 3 are the heavy and the light
-  // lane's second ones, or both the one's while the other has nothing to run.
-  // Bursts of 64 pairs of 50-5000 nodes, four pools, ms: one stream per lane,
-  // one light and three heavy lanes, admitted at once 151, 195, 184, 141; so,
-  // with a pace of 0.5, 1, 2, 4 ms: 179, 172, 147, 146; 149, 113, 113, 115;
-  // 103, 101, 96, 97; 97, 95, 84, 94.
-  const bool alone = lanes_[1 - lane].active.empty();
-  ctx_->lent_streams = alone ? 0xCu : lane == 0 ? 0x8u : 0x4u;
+  // Streams 0 and 1 are the lanes' own. The heavy lane has stream 2 as well;
+  // the light lane has 2 and 3 while no heavy tick is in flight, and its own
+  // alone beside heavy ones: a tick joins all its streams and would wait for
+  // what a heavy tick has put on them, or on another stream of the same
+  // hardware queue (a process has 4, for the lanes' streams and the plan's).
+  // Latency of a light query beside a pair of 20,000 nodes, 8 of 5000, 120 of
+  // 2500, p50 ms: 1.1, 1.1, 1.1; with the second streams of both lanes lent to
+  // the one that was alone 23, 17, 14, each lane keeping its own second one
+  // 17, 9, 15. Bursts of 64 pairs of 50-5000 nodes, mean over six pools, ms:
+  // 135 to 140, 148 and 160; one stream a lane 228.
+  reap(lanes_[1]);
+  const bool heavy_idle = lanes_[1].active.empty() && lanes_[1].ticks.empty();
+  ctx_->lent_streams = lane == 1 ? 0x4u : heavy_idle ? 0xCu : 0u;
   const int st = ctx_->launch_levels(gs.data(), (int)gs.size(), nullptr, lane);
   ctx_->lent_streams = 0;
   hipEvent_t ev = nullptr;

@@ -12,7 +12,7 @@
 // A tick lasts as long as its slowest table, so groups run in two lanes with
 // ticks and streams of their own: light pairs (the smaller tree at most
 // kLightSide nodes and at most kLightLevels levels) in lane 0, heavy ones in
-// lane 1; a light pair never waits for a tick of a heavy one.
+// lane 1; a light pair never waits for a tick of a heavy one (Server::tick).
 #pragma once
 #include <chrono>
 #include <condition_variable>
@@ -78,6 +78,7 @@ class Server {
     Clock::time_point next_admit{};  // not before, while groups are active
   };
   Lane lanes_[kLanes];
+  void reap(Lane& L);  // takes the events of finished ticks back
   std::vector<Active> completing_;             // gathers enqueued, not landed
   std::vector<hipEvent_t> free_ev_;
   std::vector<std::unique_ptr<Group>> spare_;  // finished groups, buffers kept
