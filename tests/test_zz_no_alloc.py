@@ -65,3 +65,35 @@ def test_batch_noalloc_refuses_what_does_not_fit():
         small = ctx.pool_add([xted.generate(xted.GEN_RRT, 100, 50, xted.derive_seed(72, 9))] * 2)
         d = ctx.batch_noalloc(small[:1], small[1:])
         assert d[0] == 0
+
+
+def test_batch_noalloc_accepts_the_same_pairs_whatever_their_levels():
+    """Where a pair's levels sit takes no room from the array: the most pairs
+    that fit with every pair at level 0 fit with the other placements too."""
+    with xted.Context(0) as ctx:
+        ids = ctx.pool_add([xted.generate(xted.GEN_RRT, n, 5, xted.derive_seed(73, n))
+                            for n in (2, 3)])
+
+        def fits(n):
+            try:
+                d = ctx.batch_noalloc(np.full(n, ids[0], np.int32), np.full(n, ids[1], np.int32))
+            except xted.XtedError as e:
+                assert e.status == xted.ERR_TOO_LARGE
+                return False
+            assert (d == d[0]).all()
+            return True
+
+        ctx.set_level_align(0)
+        lo, hi = 1, 1 << 20
+        assert fits(lo) and not fits(hi)
+        while hi - lo > 1:
+            mid = (lo + hi) // 2
+            lo, hi = (mid, hi) if fits(mid) else (lo, mid)
+        with xted.Context(0) as fresh:  # as created
+            f = fresh.pool_add([xted.generate(xted.GEN_RRT, n, 5, xted.derive_seed(73, n))
+                                for n in (2, 3)])
+            d = fresh.batch_noalloc(np.full(lo, f[0], np.int32), np.full(lo, f[1], np.int32))
+            assert (d == d[0]).all()
+        for mode in (1, 2):
+            ctx.set_level_align(mode)
+            assert fits(lo) and not fits(hi)

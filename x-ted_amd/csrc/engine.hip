@@ -1270,7 +1270,9 @@ int Context::run_batch(int32_t npairs, const int32_t* xs, const int32_t* ys, int
 // the arena does (the column-blocked words, sized on the device, come on top).
 // classes: granularity classes the bucket counters are counted for.
 int64_t Context::noalloc_bytes(int32_t npairs, const int32_t* xs, const int32_t* ys,
-                               int32_t classes) const {
+                               int32_t classes, bool level_offsets) const {
+  static_assert(sizeof(PairMeta) + 2 * sizeof(int64_t) + 3 * kTdPad * sizeof(td_t) >=
+                kNoAllocPairBytes);
   auto r = [](int64_t b) { return (b + 255) & ~int64_t{255}; };
   int64_t td = 0, planned = 0;
   int32_t nlevels = 0;
@@ -1286,7 +1288,7 @@ int64_t Context::noalloc_bytes(int32_t npairs, const int32_t* xs, const int32_t*
   return r(sizeof(PairMeta) * npairs) + r(nlevels) + 2 * r(8 * (int64_t)(npairs + 1)) +
          3 * r(8 * nb) + 2 * r(4 * nb) + r(32) + r(8 * planned) + r(64 * planned) +
          r((int64_t)sizeof(td_t) * td) +
-         r(4 * (int64_t)npairs) + (level_align ? r(4 * (int64_t)npairs) : 0) + r(npairs);
+         r(4 * (int64_t)npairs) + (level_offsets ? r(4 * (int64_t)npairs) : 0) + r(npairs);
 }
 
 int Context::run_batch_noalloc(int32_t npairs, const int32_t* xs, const int32_t* ys,
@@ -1308,8 +1310,9 @@ int Context::run_batch_noalloc(int32_t npairs, const int32_t* xs, const int32_t*
       return ERR_NOT_FOUND;
     }
   }
-  const int64_t need = noalloc_bytes(npairs, xs, ys, kNoAllocClasses);
-  na_arena_.cap = kNoAllocBytes + (noalloc_bytes(npairs, xs, ys, kNumClasses) - need);
+  const int64_t need = noalloc_bytes(npairs, xs, ys, kNoAllocClasses, false);
+  na_arena_.cap =
+      kNoAllocBytes + (noalloc_bytes(npairs, xs, ys, kNumClasses, level_align != 0) - need);
   if (need > (int64_t)kNoAllocBytes) {
     set_error("batch_noalloc: the pairs need " + std::to_string(need) +
               " bytes of device scratch; the array holds " + std::to_string(kNoAllocBytes));

@@ -29,11 +29,15 @@ constexpr int kMaxLevelStreams = 4;
 // buffers from (one per device, held until the process ends).
 constexpr size_t kNoAllocBytes = size_t{64} << 20;
 // Which requests fit is decided with the plan's counters of the first
-// kNoAllocClasses granularity classes; the array holds those of the classes
-// after them on top (their share of the counters, which are less than all).
+// kNoAllocClasses granularity classes and without the pairs' level offsets; the
+// array holds both on top: the other classes' counters (their share of the
+// counters, which are less than all) and 4 bytes for every pair that fits, a
+// pair taking at least kNoAllocPairBytes.
 constexpr int kNoAllocClasses = kClassShared;
+constexpr size_t kNoAllocPairBytes = 128;
 constexpr size_t kNoAllocArray =
-    kNoAllocBytes + kNoAllocBytes / kNoAllocClasses * (kNumClasses - kNoAllocClasses) + 8192;
+    kNoAllocBytes + kNoAllocBytes / kNoAllocClasses * (kNumClasses - kNoAllocClasses) +
+    kNoAllocBytes / kNoAllocPairBytes * sizeof(int32_t) + 8192;
 
 struct BatchStats {
   double plan_ms = 0;      // device plan build incl. the count read-back
@@ -313,8 +317,8 @@ class Context {
   Group na_;                        // run_batch_noalloc's group, bound to na_arena_
   std::vector<void*> retired_;      // see retire_list()
   Arena na_arena_;                  // this device's fixed array (kNoAllocArray)
-  int64_t noalloc_bytes(int32_t npairs, const int32_t* xs, const int32_t* ys,
-                        int32_t classes) const;
+  int64_t noalloc_bytes(int32_t npairs, const int32_t* xs, const int32_t* ys, int32_t classes,
+                        bool level_offsets) const;
   // Whether the leaf lines of pair (x, y) are written in closed form (the
   // leaf kernel) rather than planned as tables: lane_enable, and under a
   // cost model both trees within the cost form's stack.
