@@ -85,3 +85,36 @@ def test_command_line_all_pairs(gpu_ctx):
                          capture_output=True, text=True, timeout=120, check=True).stdout
     rows = [list(map(int, line.split())) for line in out.strip().split("\n")[1:]]
     assert np.array_equal(np.array(rows), want)
+
+
+def test_words_of_split_tables_stay_within_the_bound():
+    """A tall table is split over several workgroups, whose words take device
+    memory of their own, only where the chunk's bytes leave room for them."""
+    trees = [xted.generate(xted.GEN_RRT, n, 20, xted.derive_seed(9404, n)) for n in (1500, 1600)]
+    want = oracle.ted(*trees, threads=8, want_td=False)[0]
+    split = range(27, 33)
+    with xted.Context(0) as ctx:
+        ctx.set_profile(True)
+        for max_bytes, expected in ((0, True), (1, False)):
+            dist, _ = ctx.all_pairs(trees, max_bytes)
+            assert dist[0, 1] == want and dist[1, 0] == want
+            assert any(c in split for c in ctx.class_profile()) == expected, max_bytes
+        # The server's budget bounds them in the same way.
+        ctx.set_profile(False)
+        ids = ctx.pool_add(trees)
+        lo, hi = 1, 64 << 20
+        while hi - lo > 4096:  # the smallest budget that takes the pair
+            mid = (lo + hi) // 2
+            srv = xted.Server(ctx, hbm_budget=mid)
+            try:
+                srv.submit(int(ids[0]), int(ids[1]), 7)
+                got = []
+                while not got:
+                    got = srv.poll(timeout_ms=50)
+            finally:
+                srv.close()
+            assert got[0][1] in (xted.OK, xted.ERR_TOO_LARGE)
+            if got[0][1] == xted.OK:
+                assert got[0][2] == want
+            lo, hi = (lo, mid) if got[0][1] == xted.OK else (mid, hi)
+        assert 4 * 1500 * 1600 < hi < 64 << 20

@@ -322,14 +322,15 @@ int xted_all_pairs(xted_context* ctx, int32_t ntrees, const int32_t* sizes,
     const int64_t nn = (int64_t)ntrees * ntrees;
     std::fill(dist, dist + nn, 0);
     // Pairs in row order, cut into chunks by their device bytes (TD + TD^T
-    // and the plan arrays).
+    // and the plan arrays); what a chunk leaves is for column blocks' words.
     std::vector<int32_t> xs, ys, out;
     int64_t bytes = 0;
     auto flush = [&]() -> int {
       if (xs.empty()) return OK;
       out.resize(xs.size());
       BatchStats bs;
-      const int r = c.run_batch((int32_t)xs.size(), xs.data(), ys.data(), out.data(), nullptr, &bs);
+      const int r = c.run_batch((int32_t)xs.size(), xs.data(), ys.data(), out.data(), nullptr, &bs,
+                                max_bytes - bytes);
       if (r != OK) return r;
       for (size_t k = 0; k < xs.size(); ++k) {
         const int32_t i = xs[k] - ids[0], j = ys[k] - ids[0];

@@ -473,7 +473,8 @@ hipStream_t Context::lane_stream(int lane) const {
   return s[0];
 }
 
-int Context::plan(Group& g, int32_t npairs, const int32_t* xs, const int32_t* ys, int lane) {
+int Context::plan(Group& g, int32_t npairs, const int32_t* xs, const int32_t* ys, int lane,
+                  int64_t words_limit) {
   BatchStats& st = g.st;
   st = BatchStats{};
   g.npairs = 0;
@@ -626,11 +627,7 @@ int Context::plan(Group& g, int32_t npairs, const int32_t* xs, const int32_t* ys
   pa.rule_tail.tiny = rule.tiny;
   pa.mean_cells = st.cells / nlevels;
   pa.level_cells = nullptr;
-  if (&g == &na_) {
-    // Blocks need words in device memory: the no-allocation array holds those
-    // of the tables that go in no other way.
-    pa.rule.blocks = pa.rule_tail.blocks = 0;
-  } else if (g.maxn > kTallCols) {  // no rule looks at narrower tables' levels
+  if (&g != &na_ && g.maxn > kTallCols) {  // no rule looks at narrower tables' levels
     ST_TRY(g.level_cells.grow(sizeof(unsigned long long) * nlevels, false, ps));
     pa.level_cells = g.level_cells.as<unsigned long long>();
   }
@@ -649,38 +646,45 @@ int Context::plan(Group& g, int32_t npairs, const int32_t* xs, const int32_t* ys
   pa.tickets = g.tickets.as<unsigned int>();
   pa.xl_base = g.abort.as<uint32_t>() + kAbortInts;
   pa.abort_flag = g.abort.as<int32_t>();
-  launch_plan(pa, blk[npairs], ps);
-  HIP_TRY(hipGetLastError());
   g.h_counts.assign(nb, 0);
   g.h_maxlds.assign(nb, 0);
   g.h_cells.assign(nb, 0);
-  HIP_TRY(hipMemcpyAsync(g.h_counts.data(), g.counts.p, sizeof(unsigned long long) * nb,
-                         hipMemcpyDeviceToHost, ps));
-  HIP_TRY(hipMemcpyAsync(g.h_maxlds.data(), g.maxlds.p, sizeof(int32_t) * nb,
-                         hipMemcpyDeviceToHost, ps));
-  HIP_TRY(hipMemcpyAsync(g.h_cells.data(), g.cells.p, sizeof(unsigned long long) * nb,
-                         hipMemcpyDeviceToHost, ps));
-  HIP_TRY(hipStreamSynchronize(ps));
-  HIP_TRY(hipEventRecord(g.ev_plan1, ps));
-  // Column-blocked tables: ordinal of each bucket's first task, then (with a
-  // second short sync, only in plans that have such tables) the arena
-  // layout computed on the device.
   g.xl_first.assign(nb, 0);
-  g.nxl = 0;
-  for (int L = 0; L < nlevels; ++L) {
-    if (g.h_counts[bucket_of(L, kClassXL, 0)]) {
-      set_error("run_batch: a table fits no form (nesting height above " +
-                std::to_string(kMaxImports - 1) + " or slot storage above " +
-                std::to_string(lds_limit) + " bytes even in 256-column blocks)");
-      return ERR_TOO_LARGE;
+  // Blocks need words in device memory: the no-allocation array holds those of
+  // the tables that go in no other way, and a plan whose words are too many is
+  // made again with those alone.
+  bool blocks = &g != &na_;
+  for (;; blocks = false) {
+    pa.rule.blocks = pa.rule_tail.blocks = blocks ? 1 : 0;
+    launch_plan(pa, blk[npairs], ps);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemcpyAsync(g.h_counts.data(), g.counts.p, sizeof(unsigned long long) * nb,
+                           hipMemcpyDeviceToHost, ps));
+    HIP_TRY(hipMemcpyAsync(g.h_maxlds.data(), g.maxlds.p, sizeof(int32_t) * nb,
+                           hipMemcpyDeviceToHost, ps));
+    HIP_TRY(hipMemcpyAsync(g.h_cells.data(), g.cells.p, sizeof(unsigned long long) * nb,
+                           hipMemcpyDeviceToHost, ps));
+    HIP_TRY(hipStreamSynchronize(ps));
+    HIP_TRY(hipEventRecord(g.ev_plan1, ps));
+    // Column-blocked tables: ordinal of each bucket's first task, then (with a
+    // second short sync, only in plans that have such tables) the arena
+    // layout computed on the device.
+    g.nxl = 0;
+    g.words_bytes = 0;
+    for (int L = 0; L < nlevels; ++L) {
+      if (g.h_counts[bucket_of(L, kClassXL, 0)]) {
+        set_error("run_batch: a table fits no form (nesting height above " +
+                  std::to_string(kMaxImports - 1) + " or slot storage above " +
+                  std::to_string(lds_limit) + " bytes even in 256-column blocks)");
+        return ERR_TOO_LARGE;
+      }
+      for (int k = 0; k < kNumXLForms; ++k) {
+        const size_t bkt = bucket_of(L, kFirstXLClass + k, 0);
+        g.xl_first[bkt] = g.nxl;
+        g.nxl += (int64_t)g.h_counts[bkt];
+      }
     }
-    for (int k = 0; k < kNumXLForms; ++k) {
-      const size_t bkt = bucket_of(L, kFirstXLClass + k, 0);
-      g.xl_first[bkt] = g.nxl;
-      g.nxl += (int64_t)g.h_counts[bkt];
-    }
-  }
-  if (g.nxl > 0) {
+    if (g.nxl == 0) break;
     ST_TRY(g.xl_off.grow(sizeof(int64_t) * g.nxl, false, ps));
     ST_TRY(g.xl_total.grow(sizeof(unsigned long long), false, ps));
     XLLayoutArgs xa;
@@ -698,11 +702,16 @@ int Context::plan(Group& g, int32_t npairs, const int32_t* xs, const int32_t* ys
     HIP_TRY(hipMemcpyAsync(&words, xa.total, sizeof(words), hipMemcpyDeviceToHost, ps));
     HIP_TRY(hipStreamSynchronize(ps));
     const size_t bytes = sizeof(unsigned long long) * std::max<unsigned long long>(words, 1);
+    if (blocks && (int64_t)bytes > words_limit) continue;
+    g.words_bytes = (int64_t)bytes;
     if (bytes > g.xl_words.cap) {
-      ST_TRY(g.xl_words.grow(bytes, false, ps));
+      const int grown = g.xl_words.grow(bytes, false, ps);
+      if (blocks && grown == ERR_OUT_OF_MEMORY) continue;
+      ST_TRY(grown);
       launch_xl_zero(g.xl_words.as<unsigned long long>(), (int64_t)(g.xl_words.cap / 8), ps);
       HIP_TRY(hipGetLastError());
     }
+    break;
   }
   // Level launches (main stream, and the side streams forked from it) come
   // after everything the plan enqueued, the arena fill included.
@@ -1147,7 +1156,7 @@ int Context::copy_tables(Group& g, const std::vector<int32_t*>& outs, hipStream_
 }
 
 int Context::run_batch(int32_t npairs, const int32_t* xs, const int32_t* ys, int32_t* dist,
-                       int32_t* const* td_out, BatchStats* stats) {
+                       int32_t* const* td_out, BatchStats* stats, int64_t words_limit) {
   std::lock_guard<std::mutex> lk(mu_);
   const auto t_start = std::chrono::steady_clock::now();
   if (npairs < 0 || (npairs > 0 && (!xs || !ys || !dist))) {
@@ -1176,7 +1185,7 @@ int Context::run_batch(int32_t npairs, const int32_t* xs, const int32_t* ys, int
     Group& g = batch_[k];
     const int lane = ng > 1 ? k : -1;
     plan_share = ng;
-    st = plan(g, (int32_t)gx[k].size(), gx[k].data(), gy[k].data(), lane);
+    st = plan(g, (int32_t)gx[k].size(), gx[k].data(), gy[k].data(), lane, words_limit / ng);
     plan_share = 1;
     if (st == OK) st = run_levels(g, lane, profile ? &prof : nullptr);
     if (st != OK) {

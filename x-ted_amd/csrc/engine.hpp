@@ -95,6 +95,7 @@ struct Group {
   int32_t next_level = 0;           // next level to launch
   unsigned long long level_off = 0; // tasks of the levels already launched
   int64_t nxl = 0, leaf_tables = 0, leaf_cells = 0, td_bytes = 0;
+  int64_t words_bytes = 0;  // of the column-blocked tables' words, on top of pair_device_bytes
   std::vector<int32_t> xs, ys;
   std::vector<PairMeta> pm;
   std::vector<int64_t> lines, xl_first;  // lines: prefix of leaf-kernel tiles per pair
@@ -206,15 +207,20 @@ class Context {
   // fit are refused with ERR_TOO_LARGE. Calls that overlap on one device
   // (from different contexts) share the array and race.
   int run_batch_noalloc(int32_t npairs, const int32_t* xs, const int32_t* ys, int32_t* dist);
+  // words_limit: as in plan().
   int run_batch(int32_t npairs, const int32_t* xs, const int32_t* ys, int32_t* dist,
-                int32_t* const* td_out, BatchStats* stats);
+                int32_t* const* td_out, BatchStats* stats, int64_t words_limit = INT64_MAX);
 
   // The steps of run_batch, for callers that interleave several groups (the
   // server). The caller holds mutex() across them.
   // Plans pairs (xs[i], ys[i]) into g: device plan, one sync for the counts.
   // lane: -1 = all streams (a batch); 0 .. kMaxLevelStreams-1 = that stream
   // (and lent_streams), independently of the others'.
-  int plan(Group& g, int32_t npairs, const int32_t* xs, const int32_t* ys, int lane = -1);
+  // words_limit: bytes that the words of column-blocked tables may take; where
+  // they would take more (or cannot be allocated), tables that fit one workgroup
+  // run in one, and only those that go no other way are column-blocked.
+  int plan(Group& g, int32_t npairs, const int32_t* xs, const int32_t* ys, int lane = -1,
+           int64_t words_limit = INT64_MAX);
   // One tick: launches the next level of every group in gs (groups past
   // their last level are skipped) and advances them. Asynchronous.
   int launch_levels(Group* const* gs, int ng, std::vector<ProfLaunch>* prof, int lane = -1);

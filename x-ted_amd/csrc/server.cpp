@@ -141,7 +141,8 @@ void Server::admit(int lane) {
   int st;
   {
     std::lock_guard<std::mutex> lk(ctx_->mutex());
-    st = ctx_->plan(*g, (int32_t)batch.size(), xs.data(), ys.data(), lane);
+    st = ctx_->plan(*g, (int32_t)batch.size(), xs.data(), ys.data(), lane,
+                    budget_ - inflight_bytes_ - bytes);
     if (st == ERR_TOO_LARGE && batch.size() > 1) {
       // One pair has a table no form holds: plan pair by pair, reject those,
       // and re-plan the rest together.
@@ -152,7 +153,8 @@ void Server::admit(int lane) {
       batch = std::move(keep);
       bytes = fill(xs, ys);
       st = batch.empty() ? ERR_TOO_LARGE
-                         : ctx_->plan(*g, (int32_t)batch.size(), xs.data(), ys.data(), lane);
+                         : ctx_->plan(*g, (int32_t)batch.size(), xs.data(), ys.data(), lane,
+                                      budget_ - inflight_bytes_ - bytes);
     }
   }
   if (st != OK) {
@@ -160,6 +162,7 @@ void Server::admit(int lane) {
     recycle(std::move(g));
     return;
   }
+  bytes += g->words_bytes;
   inflight_bytes_ += bytes;
   L.active.push_back(Active{std::move(g), std::move(batch), bytes, t_admit});
   L.next_admit = Clock::now() + kAdmitPace * (int)L.active.size();

@@ -2,9 +2,10 @@
 //
 // Queries (x_id, y_id) are queued on submit. The server thread works in
 // ticks. Each tick it admits queued queries in arrival order while their
-// device bytes fit what is left of the HBM budget (TD + TD^T, 8*m*n bytes,
+// device bytes fit what is left of the HBM budget (TD + TD^T, 4*m*n bytes,
 // plus the plan's 72 bytes per planned keyroot-pair table)
-// and plans them as a new group; then it launches the next level of every
+// and plans them as a new group, whose column-blocked tables' words take what
+// the budget leaves and count against it; then it launches the next level of every
 // group in flight together (levels of different groups are independent, so
 // their tables share the same launches' streams); a group whose last level
 // has run publishes its results and frees its share of the budget. So a
