@@ -46,7 +46,8 @@ extern "C" {
  * 32 or 64 columns, four, two or one to a wave (the role of the reference's
  * single-thread tasks, X-TED_GPU/parallel_X_TED.cu:382); 36, 37, 38 = on-chip
  * tables of deep column keyroots, 4, 8 or 16 waves of 8 columns per lane that
- * share their slot rows (never forced). */
+ * share their slot rows; 39 = wide tables of few rows, swept by one wave, 512
+ * columns at a time (36..39 are never forced). */
 #define XTED_CLASS_AUTO (-1)
 #define XTED_CLASS_LANE 0
 
@@ -172,9 +173,9 @@ int xted_all_pairs(xted_context* ctx, int32_t ntrees, const int32_t* sizes,
  * with at least wide_cols columns get at least min_waves waves. */
 int xted_set_tuning(xted_context* ctx, int32_t lds_per_wave, int32_t max_cpl,
                     int32_t min_waves, int32_t wide_cols);
-/* Forces every table that fits into class cls, a row-scan class (1..25), a
- * column-blocked one (27..32) or a tiny form (33..35); XTED_CLASS_AUTO
- * restores the rule.
+/* Forces every table that fits into class cls, a row-scan class (1..25; tables
+ * of up to 8192 columns), a column-blocked one (27..32) or a tiny form (33..35);
+ * XTED_CLASS_AUTO restores the rule.
  * lane_enable = 0 sends single-row tables to the row-scan kernels. */
 int xted_force_class(xted_context* ctx, int32_t cls, int32_t lane_enable);
 /* Levels of a batch that at most tail_pairs pairs reach (the last levels of

@@ -105,3 +105,19 @@ def test_shared_slot_rows():
         assert any(xted.class_name(c).startswith("shared") for c in classes), classes
         with pytest.raises(xted.XtedError):
             ctx.force_class(xted.CLASS_SHARED)
+
+
+@pytest.mark.parametrize("waves,cpl", [(4, 8), (8, 4), (16, 2)])
+def test_forced_class_on_tall_tables(waves, cpl):
+    """The rule splits the largest tables of this pair over workgroups; a
+    forced row-scan class takes them all the same."""
+    x, y = tree(xted.GEN_RRT, 400, 900), tree(xted.GEN_RRT, 1300, 901)
+    split = range(27, 33)
+    with xted.Context(0) as ctx:
+        ctx.set_profile(True)
+        check(ctx, x, y)
+        assert any(c in split for c in ctx.class_profile())
+        cls = row_class(waves, cpl)
+        ctx.force_class(cls, lane_enable=True)
+        check(ctx, x, y)
+        assert set(ctx.class_profile()) == {xted.CLASS_LANE, cls}

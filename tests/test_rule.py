@@ -1,0 +1,91 @@
+"""The granularity rule (x-ted_amd/csrc/device.hpp) on the host: which class a
+table of given sides, nesting and leaves takes, and what a caller's settings
+promise about it."""
+import ctypes
+import itertools
+import os
+import random
+import subprocess
+
+import pytest
+
+import xted
+from conftest import ROOT
+
+NO_FORM, FIRST_XL, LDS_MAX = 26, 27, 150 * 1024
+
+
+class Rule(ctypes.Structure):
+    _fields_ = [(f, ctypes.c_int) for f in
+                ("lds_per_wave", "max_cpl", "min_waves", "wide_cols", "tail")]
+
+
+class Table(ctypes.Structure):
+    _fields_ = [(f, ctypes.c_int) for f in ("a", "b", "kd_r", "kd_c", "leaves_c")] + \
+               [("cells", ctypes.c_longlong)]
+
+
+@pytest.fixture(scope="module")
+def shim(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("rule") / "rule.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC",
+                    os.path.join(ROOT, "tests", "rule_shim.cpp"), "-o", so], check=True)
+    return ctypes.CDLL(so)
+
+
+def classify(shim, table, rule=None, force=-1):
+    """(class, LDS bytes) of Table fields under Rule fields (the default's)."""
+    need = ctypes.c_longlong()
+    r = Rule(*(rule or (10 * 1024, 16, 1, 1 << 30, 0)))
+    cls = shim.rule_class(ctypes.byref(r), ctypes.byref(Table(*table)), force, ctypes.byref(need))
+    return cls, need.value
+
+
+def tables(seed, count):
+    """Tables of every size a rule tells apart, short and tall, shallow and
+    deep, in levels of few and of many cells."""
+    rnd = random.Random(seed)
+    sides = [2, 3, 16, 17, 33, 64, 65, 128, 256, 257, 400, 512, 513, 1000, 1024, 1025, 2000, 2048,
+             2049, 3000, 4096, 4097, 8000, 8192, 8193, 12000, 20000]
+    for _ in range(count):
+        a, b = rnd.choice(sides), rnd.choice(sides)
+        rows, cols = min(a, b), max(a, b)
+        kd_r = min(rnd.choice([1, 2, 5, 20, 60]), (rows - 1) // 2)
+        kd_c = min(rnd.choice([1, 2, 5, 20, 60, 120, 250, 550]), (cols - 1) // 2)
+        leaves = max(kd_c + 1, min(cols - kd_c, rnd.choice([2, 10, cols // 4, cols // 2, cols - 1])))
+        yield a, b, kd_r, kd_c, leaves, rows * cols * rnd.choice([1, 10, 500, 5000])
+
+
+def test_forced_row_class_takes_every_table_that_fits(shim):
+    """Whatever the rule would choose: column blocks for tall tables, one
+    wave's sweep for short ones of a large level. (A table takes shared slot
+    rows only where no row-scan class fits it.)"""
+    replaced = set()
+    for t in tables(1, 6000):
+        cols = max(t[0], t[1])
+        auto, _ = classify(shim, t)
+        for waves, cpl in itertools.product((1, 2, 4, 8, 16), (1, 2, 4, 8, 16)):
+            cls = 1 + 5 * (waves.bit_length() - 1) + (cpl.bit_length() - 1)
+            need = shim.scan_need(max(t[2], 1), t[4], t[3], waves)
+            fits = cols <= min(64 * waves * cpl, 8192) and need <= LDS_MAX
+            got, lds = classify(shim, t, force=cls)
+            if auto != NO_FORM and fits:
+                assert (got, lds) == (cls, need), (t, waves, cpl)
+                replaced.add(auto)
+            else:
+                assert got == auto
+    assert replaced & set(range(FIRST_XL, FIRST_XL + 6)) and xted.CLASS_SWEEP in replaced
+    assert not replaced & {xted.CLASS_SHARED + k for k in range(3)}
+
+
+def test_forced_blocks_and_tiny_forms(shim):
+    for t in tables(2, 3000):
+        auto, _ = classify(shim, t)
+        for force in list(range(FIRST_XL, FIRST_XL + 6)) + [xted.CLASS_TINY + k for k in range(3)]:
+            got, lds = classify(shim, t, force=force)
+            assert got == force or got == auto
+            if got == force and force >= xted.CLASS_TINY:
+                k = force - xted.CLASS_TINY
+                assert max(t[0], t[1]) <= xted.TINY_SEG[k] and lds <= 2048 << k
+            if auto == NO_FORM:
+                assert got == NO_FORM

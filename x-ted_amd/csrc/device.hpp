@@ -409,4 +409,31 @@ XTED_HD inline int table_class(int a, int b, int kd_r, int kd_c, int leaves_c, b
   return row_class(wi, ci);
 }
 
+// The class of a table of class cls while class force is forced: force where
+// the table is neither the leaf kernel's nor without a form and fits it,
+// whatever the rule chose (a row-scan class takes tables of up to
+// kMaxOnChipCols columns), else cls.
+template <class Own>
+XTED_HD inline int forced_class(int force, int cls, int a, int b, int kd_r, int kd_c, int leaves_c,
+                                const ClassRule& rule, const Own& own, int64_t* need) {
+  const int cols = a <= b ? b : a;
+  const int slots = kd_r > 1 ? kd_r : 1;
+  if (cls < 1 || cls == kClassXL) return cls;
+  int64_t n = 0;
+  bool fits = false;
+  if (force >= kFirstXLClass && force < kFirstXLClass + kNumXLForms) {
+    const int k = force - kFirstXLClass;
+    fits = xl_form(slots, kd_c, leaves_c, k, rule.lds_max, own, &n) == k;
+  } else if (is_tiny(force)) {
+    n = scan_lds_need(slots, leaves_c, 0, 1);
+    fits = cols <= tiny_seg(force - kClassTiny) && n <= tiny_max_lds(force - kClassTiny);
+  } else if (force >= 1 && force <= kNumRowClasses) {
+    const int w = 1 << (force - 1) / 5, c = 1 << (force - 1) % 5;
+    n = scan_lds_need(slots, leaves_c, kd_c, w);
+    fits = cols <= 64 * w * c && cols <= kMaxOnChipCols && n <= rule.lds_max;
+  }
+  if (fits) *need = n;
+  return fits ? force : cls;
+}
+
 }  // namespace xted

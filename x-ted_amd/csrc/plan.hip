@@ -41,9 +41,6 @@ __device__ __forceinline__ void classify(const PlanArgs& A, const TreeMeta& tx,
   const int32_t kdx = A.pool.skd[kx], kdy = A.pool.skd[ly];
   const int32_t level = kdx + kdy + loff;
   const ClassRule& rule = A.tail_level[level] ? A.rule_tail : A.rule;
-  // One slot row per nesting level of the row keyroot (at least one: the
-  // kernels read slot 0 unconditionally).
-  const int32_t slots = max(a <= b ? kdx : kdy, 1);
   const int32_t leaves_c = a <= b ? A.pool.sleaf[ly] : A.pool.sleaf[kx];
   int64_t need = 0;
   // With the leaf kernel off, single-row tables take the row-scan forms.
@@ -61,39 +58,9 @@ __device__ __forceinline__ void classify(const PlanArgs& A, const TreeMeta& tx,
   };
   int cls = table_class(a, b, a <= b ? kdx : kdy, a <= b ? kdy : kdx, leaves_c, leaf_form, rule,
                         level_cells, own, &need);
-  // A forced column-blocked form takes every multi-row table it can hold.
-  if (A.force_class >= kFirstXLClass && A.force_class < kFirstXLClass + kNumXLForms && cls >= 1 &&
-      cls != kClassXL) {
-    const int k = A.force_class - kFirstXLClass;
-    const int32_t kd_c = a <= b ? kdy : kdx;
-    int64_t n = 0;
-    if (xl_form(slots, kd_c, leaves_c, k, A.rule.lds_max, own, &n) == k) {
-      cls = A.force_class;
-      need = n;
-    }
-  }
-  // A forced row-scan form (or tiny form) takes every on-chip table it can
-  // hold.
-  if (is_tiny(A.force_class) && cls >= 1 && (cls <= kNumRowClasses || is_tiny(cls))) {
-    const int k = A.force_class - kClassTiny;
-    const int cols = a <= b ? b : a;
-    const int64_t row_need = scan_lds_need(slots, leaves_c, 0, 1);
-    if (cols <= tiny_seg(k) && row_need <= tiny_max_lds(k)) {
-      cls = A.force_class;
-      need = row_need;
-    }
-  }
-  if (A.force_class >= 1 && A.force_class <= kNumRowClasses && cls >= 1 &&
-      (cls <= kNumRowClasses || is_tiny(cls) || is_shared(cls))) {
-    const int wi = (A.force_class - 1) / 5, ci = (A.force_class - 1) % 5;
-    const int cols = a <= b ? b : a;
-    const int64_t row_need = scan_lds_need(slots, leaves_c, a <= b ? kdy : kdx, 1 << wi);
-    if ((cls < kClassXL || is_tiny(cls) || is_shared(cls)) && cols <= 64 * (1 << wi) * (1 << ci) &&
-        row_need <= A.rule.lds_max) {
-      cls = A.force_class;
-      need = row_need;
-    }
-  }
+  if (A.force_class >= 0)
+    cls = forced_class(A.force_class, cls, a, b, a <= b ? kdx : kdy, a <= b ? kdy : kdx, leaves_c,
+                       A.rule, own, &need);
   *bucket = bucket_of(level, cls, size_band(cls, a <= b ? a : b, need, A.bands, A.light_per_wave));
   *lds = (int)need;
   *i0 = (uint32_t)A.pool.skr[kx];
