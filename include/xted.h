@@ -168,9 +168,13 @@ int xted_all_pairs(xted_context* ctx, int32_t ntrees, const int32_t* sizes,
 /* ---- tuning and test hooks ------------------------------------------------------
  * Granularity cut-overs, the role of the fixed thresholds 15 / 18,750 /
  * 25,250,000 in X-TED_GPU/parallel_X_TED.cu:382. lds_per_wave: slot bytes
- * one wave may own before a table gets more waves; max_cpl (1, 2, 4, 8 or
- * 16, the default): columns per lane before a table gets more waves; tables
- * with at least wide_cols columns get at least min_waves waves. */
+ * one wave may own before a table gets more waves (no more than whose shares
+ * of the far values fit LDS); max_cpl (1, 2, 4, 8 or 16, the default): columns
+ * per lane before a table gets more waves; tables with at least wide_cols
+ * columns get at least min_waves waves. Two kinds of table are split by what
+ * else their level holds: tall ones in levels of little work take more waves
+ * or workgroups, and with max_cpl of 8 or more, wide ones of few rows in levels
+ * of much work are swept by one wave (not where min_waves asks for more). */
 int xted_set_tuning(xted_context* ctx, int32_t lds_per_wave, int32_t max_cpl,
                     int32_t min_waves, int32_t wide_cols);
 /* Forces every table that fits into class cls, a row-scan class (1..25; tables

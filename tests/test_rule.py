@@ -89,3 +89,53 @@ def test_forced_blocks_and_tiny_forms(shim):
                 assert max(t[0], t[1]) <= xted.TINY_SEG[k] and lds <= 2048 << k
             if auto == NO_FORM:
                 assert got == NO_FORM
+
+
+def waves_and_columns(cls, cols):
+    """Waves of a table of class cls and the columns a lane of them holds."""
+    if 1 <= cls <= 25:
+        waves, cpl = 1 << (cls - 1) // 5, 1 << (cls - 1) % 5
+        return waves, cpl
+    if xted.CLASS_SHARED <= cls < xted.CLASS_SWEEP:
+        return 4 << (cls - xted.CLASS_SHARED), 8
+    if FIRST_XL <= cls < FIRST_XL + 6:
+        k = cls - FIRST_XL
+        blocks = -(-cols // xted.XL_BW[k])
+        return (8, 8, 8, 4, 1, 1)[k] * blocks, (8, 4, 2, 2, 4, 2)[k]
+    return 1, 1
+
+
+@pytest.mark.parametrize("max_cpl", [1, 2, 4, 8, 16])
+@pytest.mark.parametrize("min_waves,wide_cols", [(1, 1 << 30), (2, 600), (3, 300), (16, 1025)])
+def test_settings_hold_for_every_class(shim, max_cpl, min_waves, wide_cols):
+    """Tables of at least wide_cols columns get at least min_waves waves, and
+    every table as many as max_cpl columns a lane take (16 at most)."""
+    seen = set()
+    for t in tables(3, 6000):
+        cols = max(t[0], t[1])
+        cls, _ = classify(shim, t, (10 * 1024, max_cpl, min_waves, wide_cols, 0))
+        seen.add(cls)
+        if cls == NO_FORM or xted.CLASS_TINY <= cls < xted.CLASS_SHARED:
+            continue
+        on_chip = cls <= 25 or cls >= xted.CLASS_SHARED
+        waves, _ = waves_and_columns(cls, cols)
+        # (Column blocks are also where tables go that fit nothing else.)
+        if cols >= wide_cols and (on_chip or cls == FIRST_XL + 2):
+            assert waves >= min_waves, (t, cls)
+        if cls != xted.CLASS_SWEEP and on_chip:
+            assert waves >= min(16, -(-cols // (64 * max_cpl))), (t, cls)
+        if cls == xted.CLASS_SWEEP:
+            assert max_cpl >= 8
+    assert {xted.CLASS_SHARED + k for k in range(3)} & seen
+    assert max_cpl < 8 or min_waves > 1 or xted.CLASS_SWEEP in seen
+
+
+def test_every_table_that_fits_lds_has_a_form(shim):
+    """Under any settings: a table of up to 8192 columns whose slot rows fit
+    one workgroup is taken."""
+    for max_cpl, min_waves in ((16, 1), (8, 1), (8, 16), (16, 7)):
+        for t in tables(4, 6000):
+            if max(t[0], t[1]) <= 8192 and shim.scan_need(max(t[2], 1), t[4], t[3], 1) <= LDS_MAX:
+                for tail in (0, 1):
+                    cls, need = classify(shim, t, (10 * 1024, max_cpl, min_waves, 600, tail))
+                    assert cls != NO_FORM and need <= LDS_MAX + 10 * 1024, t

@@ -150,7 +150,8 @@ constexpr int kNumClasses = kClassSweep + 1;  // 40
 XTED_HD inline bool is_tiny(int cls) { return cls >= kClassTiny && cls < kClassShared; }
 XTED_HD inline bool is_shared(int cls) { return cls >= kClassShared && cls < kClassSweep; }
 // Shared-slot form k: 4, 8 or 16 waves of 8 columns per lane.
-XTED_HD inline int shared_cols(int k) { return 64 * 8 * (4 << k); }
+XTED_HD inline int shared_waves(int k) { return 4 << k; }
+XTED_HD inline int shared_cols(int k) { return 64 * 8 * shared_waves(k); }
 // Lanes per table (and most columns) of tiny form k.
 XTED_HD inline int tiny_seg(int k) { return 16 << k; }
 // Slot bytes of one table of tiny form k: 32 KiB per workgroup of 256 lanes.
@@ -364,20 +365,21 @@ XTED_HD inline int table_class(int a, int b, int kd_r, int kd_c, int leaves_c, b
     tall = cells <= rows * rule.tall2 ? 2 : cells <= rows * rule.tall4 ? 4 : 0;
     while (tall && wi < 4 && cols > 64 * tall * (1 << wi)) ++wi;
   }
-  if (!tall && wi > 0 && cols > 2 * kSweepCols && cells >= (int64_t)rows * cols * rule.sweep) {
+  // Waves a table gets at least, by its columns (a power of two).
+  const int wide = cols >= rule.wide_cols ? rule.min_waves : 1;
+  int least = 1;
+  while (least < kMaxRowWaves && (least < wide || cols > 64 * rule.max_cpl * least)) least *= 2;
+  if (wide <= 1 && rule.max_cpl >= kSweepCols / 64 && !tall && wi > 0 && cols > 2 * kSweepCols &&
+      cells >= (int64_t)rows * cols * rule.sweep) {
     const int64_t n = sweep_lds_need(slots, own(kSweepForm), kd_c, rows);
     if (n <= kSweepLds && n <= rule.lds_max) {
       *need = n;
       return kClassSweep;
     }
   }
-  if (cols >= rule.wide_cols) {
-    while (wi < 4 && (1 << wi) < rule.min_waves) ++wi;
-  }
-  // More waves hold more imports: no more than fit (up to 16 columns a lane).
-  while (wi > 0 && scan_lds_need(slots, leaves_c, kd_c, 1 << wi) > rule.lds_max &&
-         cols <= 64 * 16 * (1 << (wi - 1)))
-    --wi;
+  while (wi < 4 && (1 << wi) < least) ++wi;
+  // More waves hold more imports: no more than fit, down to the least.
+  while ((1 << wi) > least && scan_lds_need(slots, leaves_c, kd_c, 1 << wi) > rule.lds_max) --wi;
   const int first_tall = tall == 2 ? kTall2Form : tall == 4 ? kTall4Form : 0;
   const int first = rule.xl_first > first_tall ? rule.xl_first : first_tall;
   auto blocked = [&](int k) {
@@ -388,13 +390,13 @@ XTED_HD inline int table_class(int a, int b, int kd_r, int kd_c, int leaves_c, b
   // leaves them more columns per lane.
   if (tall && rule.blocks && rows > kTallBlockRows && rows > rule.xl_seq_rows &&
       (cols > xl_bw(first_tall) || cols > 64 * tall * (1 << wi))) {
-    const int cls = blocked(first);
-    if (cls != kClassXL) return cls;
+    const int cls = blocked(first), k = cls - kFirstXLClass;
+    if (cls != kClassXL && (cols + xl_bw(k) - 1) / xl_bw(k) * xl_waves(k) >= least) return cls;
   }
   *need = scan_lds_need(slots, leaves_c, kd_c, 1 << wi);
   if (*need > rule.lds_max && lds_need <= rule.lds_max) {
     for (int k = 0; k < kNumSharedForms; ++k) {
-      if (cols <= shared_cols(k)) {
+      if (cols <= shared_cols(k) && shared_waves(k) >= least) {
         *need = lds_need;
         return kClassShared + k;
       }
