@@ -32,6 +32,15 @@ int rule_class(const Rule* r, const Table* t, int force, long long* need) {
   return cls;
 }
 
+// A new context's settings: those of xted_set_tuning, then the tail rule's, the
+// level placement's, the size bands', the light LDS and the tiny forms'.
+void default_knobs(int* out) {
+  const ClassRule r = kDefaultRule;
+  const int v[] = {r.lds_per_wave,     r.max_cpl,         r.min_waves,   r.wide_cols, kDefaultTailPairs,
+                   kDefaultLevelAlign, kDefaultSizeBands, kLightPerWave, r.tiny};
+  for (int i = 0; i < 9; ++i) out[i] = v[i];
+}
+
 long long scan_need(int slots, int leaves_c, int kd_c, int w) {
   return scan_lds_need(slots, leaves_c, kd_c, w);
 }

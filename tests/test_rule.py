@@ -2,6 +2,7 @@
 table of given sides, nesting and leaves takes, and what a caller's settings
 promise about it."""
 import ctypes
+import inspect
 import itertools
 import os
 import random
@@ -9,6 +10,7 @@ import subprocess
 
 import pytest
 
+import autotune
 import xted
 from conftest import ROOT
 
@@ -139,3 +141,19 @@ def test_every_table_that_fits_lds_has_a_form(shim):
                 for tail in (0, 1):
                     cls, need = classify(shim, t, (10 * 1024, max_cpl, min_waves, 600, tail))
                     assert cls != NO_FORM and need <= LDS_MAX + 10 * 1024, t
+
+
+def test_python_defaults_are_a_new_contexts(shim):
+    """Context.set_tuning() restores a new context's rule, and the tuner's
+    baseline (also what load() gives without a stored rule) is that rule."""
+    out = (ctypes.c_int * 9)()
+    shim.default_knobs(out)
+    keys = ["lds_per_wave", "max_cpl", "min_waves", "wide_cols", "tail_pairs", "level_align",
+            "size_bands", "light_lds", "tiny_forms"]
+    knobs = dict(zip(keys, out))
+    assert autotune.DEFAULT == knobs
+    assert autotune.load("/nonexistent/tuning.json") == knobs
+    for method, names in (("set_tuning", keys[:4]), ("set_size_bands", ["size_bands"]),
+                          ("set_tiny_forms", ["tiny_forms"])):
+        params = list(inspect.signature(getattr(xted.Context, method)).parameters.values())[1:]
+        assert [p.default for p in params] == [knobs[k] for k in names], method

@@ -46,8 +46,9 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, HERE)
 import xted  # noqa: E402
 
-DEFAULT = {"lds_per_wave": 10 * 1024, "max_cpl": 8, "min_waves": 1, "wide_cols": 1 << 30,
-           "tail_pairs": 32, "level_align": 0, "size_bands": 1, "light_lds": 10 * 1024,
+# A new context's rule (kDefaultRule and the constants after it in csrc/device.hpp).
+DEFAULT = {"lds_per_wave": 10 * 1024, "max_cpl": 16, "min_waves": 1, "wide_cols": 1 << 30,
+           "tail_pairs": 32, "level_align": 1, "size_bands": 1, "light_lds": 10 * 1024,
            "tiny_forms": 1}
 # Seed stream of the tuning workload (bench.py times stream 3).
 SEED_TUNE = 1003

@@ -244,11 +244,7 @@ class Context {
   int poll(Group& g, bool wait, int32_t* dist);
 
   // Tuning / test hooks -----------------------------------------------------
-  // (Up to 16 columns per lane: the distance matrix of 96 trees of 100-1000
-  // nodes took 99.9 ms against 110.8 with 8, and 89.4 with level_align 1;
-  // under a cost model, whose 16-column form holds 204 VGPRs, 4096 pairs took
-  // 120 against 146, 1024 pairs 44 against 49.)
-  ClassRule rule{kLdsPerWave, 1, 1 << 30, kLdsMaxTable, 16, kXLSeqRows};
+  ClassRule rule = kDefaultRule;
   int32_t lds_limit = 0;  // device's dynamic LDS per workgroup for the slots
   int32_t force_class = -1;
   int32_t lane_enable = 1;
@@ -257,7 +253,7 @@ class Context {
   // Levels reached by at most this many pairs of a batch take the latency
   // rule (fewest waves, up to 16 columns per lane, LDS up to the device
   // limit); 0 turns it off.
-  int32_t tail_pairs = 32;
+  int32_t tail_pairs = kDefaultTailPairs;
   // A batch of at least batch_split_min pairs is cut into batch_groups groups
   // (pair i in group i mod batch_groups), each with its own plan and its own
   // stream: their levels run independently, so one group's level barriers
@@ -282,11 +278,11 @@ class Context {
   // few large tables of the deepest pairs. In ms with 0, 1, 2: the 96-tree
   // matrix 99.9, 89.3, 90; 128 pairs of 100-600 nodes 18.8, 17.2, 17.6; 1024
   // pairs under a cost model 54.0, 50.3, 49.4.
-  int32_t level_align = 1;
+  int32_t level_align = kDefaultLevelAlign;
   // 1: the tables of a launch start largest first (size bands); 2: and the
   // tables that need more slot storage than light_lds take launches of
   // their own; 0: plan order.
-  int32_t size_bands = 1;
+  int32_t size_bands = kDefaultSizeBands;
   // Mode 2: slot bytes per wave above which a row-scan table is heavy.
   int32_t light_per_wave = kLightPerWave;
   ClassProfile class_profile[kNumClasses];

@@ -361,7 +361,7 @@ class Context:
                                     _p(dist), ctypes.byref(st)))
         return dist, st
 
-    def set_tuning(self, lds_per_wave=10 * 1024, max_cpl=8, min_waves=1, wide_cols=1 << 30):
+    def set_tuning(self, lds_per_wave=10 * 1024, max_cpl=16, min_waves=1, wide_cols=1 << 30):
         _check(lib().xted_set_tuning(self._h, lds_per_wave, max_cpl, min_waves, wide_cols))
 
     def set_xl_rule(self, seq_rows):
