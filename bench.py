@@ -486,7 +486,7 @@ def main():
     xs, ys = ids[0::2].copy(), ids[1::2].copy()
     import autotune
     if args.autotune:
-        rule, _, _ = autotune.tune(ctx, xs, ys, log=log)
+        rule, _, _ = autotune.tune(ctx, xs, ys, log=log, start=autotune.DEFAULT)
     else:
         rule = autotune.load()
         if args.rule:

@@ -8,6 +8,7 @@ import os
 import random
 import subprocess
 
+import numpy as np
 import pytest
 
 import autotune
@@ -157,3 +158,32 @@ def test_python_defaults_are_a_new_contexts(shim):
                           ("set_tiny_forms", ["tiny_forms"])):
         params = list(inspect.signature(getattr(xted.Context, method)).parameters.values())[1:]
         assert [p.default for p in params] == [knobs[k] for k in names], method
+
+
+def test_tuner_starts_from_the_default(monkeypatch, tmp_path):
+    """The command's search has a new context's rule to beat."""
+    started = []
+
+    def fake_tune(ctx, xs, ys, **kw):
+        started.append(kw["start"])
+        return dict(kw["start"]), [], 0.0
+
+    class FakeContext:
+        def __init__(self, device):
+            pass
+
+        def __enter__(self):
+            return self
+
+        def __exit__(self, *exc):
+            pass
+
+        def pool_add(self, trees):
+            return np.arange(len(trees))
+
+    monkeypatch.setattr(autotune, "tune", fake_tune)
+    monkeypatch.setattr(autotune.xted, "Context", FakeContext)
+    monkeypatch.setattr("sys.argv", ["autotune", "--pairs", "2", "--out", str(tmp_path / "t.json")])
+    autotune.main()
+    assert started == [autotune.DEFAULT]
+    assert autotune.load(str(tmp_path / "t.json")) == autotune.DEFAULT

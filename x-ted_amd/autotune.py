@@ -25,10 +25,10 @@ on:
      winning.
 
 The workload is the 4096-pair uneven batch's generator on a seed stream of
-its own (not the one bench.py times). The rule starts as the default; a
+its own (not the one bench.py times). The rule starts as a new context's; a
 candidate replaces the current best only when every one of its steps is
 faster than the best rule's fastest step, so step-to-step noise cannot pick
-a rule. Every candidate must reproduce the default rule's distances
+a rule. Every candidate must reproduce the first rule's distances
 exactly, or the run stops.
 
     python x-ted_amd/autotune.py [--pairs N] [--out x-ted_amd/tuning.json]
@@ -50,6 +50,8 @@ import xted  # noqa: E402
 DEFAULT = {"lds_per_wave": 10 * 1024, "max_cpl": 16, "min_waves": 1, "wide_cols": 1 << 30,
            "tail_pairs": 32, "level_align": 1, "size_bands": 1, "light_lds": 10 * 1024,
            "tiny_forms": 1}
+# Where a search starts that names no rule: narrow lanes, every pair from level 0.
+START = dict(DEFAULT, max_cpl=8, level_align=0)
 # Seed stream of the tuning workload (bench.py times stream 3).
 SEED_TUNE = 1003
 SEED_CONFIRM = 1005  # second workload of the confirmation round
@@ -111,21 +113,22 @@ def steps(ctx, xs, ys, rule, reps):
 
 
 def tune(ctx, xs, ys, stages=STAGES, reps=3, log=print, confirm_top=CONFIRM_TOP, confirmed=None,
-         confirm_sets=()):
+         confirm_sets=(), start=None):
     """Returns (best_rule, results, spread): the staged search described in
-    the module docstring. results lists (rule, best step time); confirmed, if
+    the module docstring, from the rule start (START). results lists (rule, best step time); confirmed, if
     given, receives (rule, score) of the confirmation round, the score being
     the mean over (xs, ys) and the workloads of confirm_sets (pairs of id
     arrays) of each one's median step time."""
-    base_times, base_d = steps(ctx, xs, ys, DEFAULT, 6)
+    base = dict(START if start is None else start)
+    base_times, base_d = steps(ctx, xs, ys, base, 6)
     spread = max(base_times) - min(base_times)
     base_t = min(base_times)
-    results = [(dict(DEFAULT), base_t)]
-    log(f"default {DEFAULT}: {base_t * 1e3:.1f} ms, step-to-step spread {spread * 1e3:.2f} ms")
+    results = [(dict(base), base_t)]
+    log(f"start {base}: {base_t * 1e3:.1f} ms, step-to-step spread {spread * 1e3:.2f} ms")
     # The best rule's fastest step: a candidate wins only when its slowest
     # step beats it (every step of the candidate faster than every step of
     # the best), so neither rule's step-to-step noise can pick it.
-    best, best_t = dict(DEFAULT), base_t
+    best, best_t = dict(base), base_t
 
     def trial(rule):
         nonlocal best, best_t
@@ -148,22 +151,22 @@ def tune(ctx, xs, ys, stages=STAGES, reps=3, log=print, confirm_top=CONFIRM_TOP,
 
     for grid in stages:
         keys = list(grid)
-        start = dict(best)
+        around = dict(best)
         for vals in itertools.product(*(grid[k] for k in keys)):
-            trial(dict(start, **dict(zip(keys, vals))))
+            trial(dict(around, **dict(zip(keys, vals))))
     # Fine steps of slot bytes per wave around the coarse best.
-    start = dict(best)
+    around = dict(best)
     for k in range(-FINE_SPAN, FINE_SPAN + 1):
-        lds = start["lds_per_wave"] + k * FINE_STEP
+        lds = around["lds_per_wave"] + k * FINE_STEP
         if lds >= 2 * 1024:
-            trial(dict(start, lds_per_wave=lds))
+            trial(dict(around, lds_per_wave=lds))
     # Confirmation: the best rule and the fastest other candidates (by their
     # best step), re-timed in interleaved rounds; the lowest median step wins.
     ranked = [r for r, _ in sorted(results, key=lambda rt: rt[1]) if r != best]
     finalists = [best] + ranked[:max(0, confirm_top - 1)]
     sets = [(xs, ys, base_d)]
     for cx, cy in confirm_sets:
-        sets.append((cx, cy, steps(ctx, cx, cy, DEFAULT, 1)[1]))
+        sets.append((cx, cy, steps(ctx, cx, cy, base, 1)[1]))
     samples = [[[] for _ in sets] for _ in finalists]
     if len(finalists) > 1:
         for _ in range(CONFIRM_ROUNDS):
@@ -198,7 +201,7 @@ def main():
         ids = ctx.pool_add(trees)
         ids2 = ctx.pool_add(trees2)
         best, results, spread = tune(ctx, ids[0::2].copy(), ids[1::2].copy(),
-                                     confirmed=confirmed,
+                                     confirmed=confirmed, start=DEFAULT,
                                      confirm_sets=[(ids2[0::2].copy(), ids2[1::2].copy())])
     out = {"rule": best,
            "workload": f"batch{args.pairs}_uneven_n100-1000_deep50_shallow50_alphabet200 "
