@@ -350,8 +350,11 @@ __device__ __forceinline__ void scan_block(const DPArgs& A, const TaskDesc& dsc,
   constexpr bool kRing = W > 1 || kXL;                // edges are rings between waves
   constexpr bool kEdges = kRing || kMode == kSwept;
   static_assert(kMode != kSwept || W == 1);
-  // TD ring slots: a power of two dividing 64.
-  constexpr int S = C >= 16 || (W == 1 && C >= 8 && !kXL) || (kXL && kCost && C >= 8) ? 4 : 8;
+  // TD ring slots: a power of two dividing 64; 4 where 8 would leave too few
+  // waves, or spill: 16 waves have 128 registers each (with costs and 8 slots
+  // 34 of them spilled; 233,500 tables of a pair of 8000 and 250 nodes 7.8 ms,
+  // with 4 slots and none 6.6).
+  constexpr int S = C >= 16 || (C >= 8 && ((W == 1 && !kXL) || (kCost && (kXL || W == 16)))) ? 4 : 8;
   constexpr int PD = S - 1;                    // rows of TD prefetched
   constexpr int NW = C == 1 ? 1 : C / 2;       // words of one row: two 16-bit entries each
   constexpr int D = kXL ? xl_edge_rows(W) : kEdgeRows;
@@ -493,11 +496,11 @@ __device__ __forceinline__ void scan_block(const DPArgs& A, const TaskDesc& dsc,
     else return -e;
   };
   const int32_t T = kCost ? 0 : tlane;
-  // The columns' records are read 8 at a time and pinned, so that each is one
-  // 16-byte load in flight with the others (unpinned, the compiler splits them
-  // into loads of single fields in branches on lanes, each waiting for the one
-  // before).
-  constexpr int B = C < 8 ? C : 8;
+  // The columns' records are read 8 at a time (4 where 8 would spill) and
+  // pinned, so that each is one 16-byte load in flight with the others
+  // (unpinned, the compiler splits them into loads of single fields in branches
+  // on lanes, each waiting for the one before).
+  constexpr int B = C < 8 ? C : kXL && kCost ? 4 : 8;
 #pragma unroll
   for (int e0 = 0; e0 < C; e0 += B) {
     NodeRec cl[B], rl[kEdges ? B : 1];  // as a table column; (edges) as a row: kdep of c and c-1
