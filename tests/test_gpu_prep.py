@@ -49,3 +49,13 @@ def test_trees_at_the_lds_limit(gpu_ctx, shape, n):
     d, td, _ = gpu_ctx.ted(x, y)
     od, otd, _ = oracle.ted(x, y, threads=8)
     assert d == od and np.array_equal(td, otd)
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("n", [5484, 5485])
+def test_largest_tree_in_lds_and_the_next(gpu_ctx, shape, n):
+    """5484 nodes fill the 150 KiB of LDS that preparation may take."""
+    x, y = shaped("rrt", 12), shaped(shape, n)
+    d, td, _ = gpu_ctx.ted(x, y)
+    od, otd, _ = oracle.ted(x, y, threads=8)
+    assert d == od and np.array_equal(td, otd)

@@ -36,7 +36,8 @@ struct PrepArgs {
 };
 // Working arrays of n + 1 ints per tree, and the nodes of which they fit LDS.
 constexpr int kPrepArrays = 7;
-constexpr int kPrepLdsNodes = 150 * 1024 / (4 * kPrepArrays) - 1;  // 5485
+constexpr int kPrepLdsNodes = 150 * 1024 / (4 * kPrepArrays) - 1;
+static_assert(kPrepLdsNodes == 5484, "a tree of 5484 nodes takes 153,580 bytes");
 // maxn: the largest tree's nodes.
 void launch_tree_prep(const PrepArgs& a, int ntrees, int maxn, hipStream_t s);
 hipError_t prep_init_attributes();
