@@ -121,3 +121,49 @@ def test_forced_class_on_tall_tables(waves, cpl):
         ctx.force_class(cls, lane_enable=True)
         check(ctx, x, y)
         assert set(ctx.class_profile()) == {xted.CLASS_LANE, cls}
+
+
+def comb_and_star(comb_nodes, leaves):
+    """A root over a comb and that many leaves: nested as deep as the comb."""
+    parent, _ = comb(comb_nodes)
+    n = 1 + comb_nodes + leaves
+    out = np.zeros(n, np.int32)
+    out[0] = -1
+    out[1:1 + comb_nodes] = parent + 1
+    return out, (np.arange(n) * 5 % 4).astype(np.int32)
+
+
+@pytest.mark.parametrize("waves,rows,leaves", [(4, 100, 900), (8, 60, 2000), (16, 30, 4500)])
+@pytest.mark.parametrize("costs", [False, True])
+def test_every_shared_slot_form(waves, rows, leaves, costs):
+    """Columns nested 299 deep, above what column blocks hold, in trees of
+    1501, 2601 and 5101 nodes whose waves' imports do not fit LDS."""
+    model = cost_model(4, 33) if costs else None
+    x, y = comb(rows), comb_and_star(600, leaves)
+    with xted.Context(0) as ctx:
+        ctx.set_costs(model)
+        ctx.set_profile(True)
+        check(ctx, x, y, model)
+        assert f"shared_w{waves}_c8" in {xted.class_name(c) for c in ctx.class_profile()}
+        check(ctx, y, x, model)
+
+
+@pytest.mark.parametrize("waves,cpl", [(2, 8), (2, 16), (8, 2), (8, 8), (16, 8)])
+@pytest.mark.parametrize("costs", [False, True])
+def test_edges_of_wide_forms(waves, cpl, costs):
+    """Several active waves of 8 and 16 columns per lane, and 16 of them."""
+    block = 64 * cpl
+    full = block * waves
+    model = cost_model(6, 34) if costs else None
+    with xted.Context(0) as ctx:
+        ctx.set_costs(model)
+        ctx.force_class(row_class(waves, cpl), lane_enable=False)
+        ctx.set_profile(True)
+        kinds = (xted.GEN_RRT, xted.GEN_SHALLOW)
+        k = 0
+        for c in (block + 1, full - block, full - 1, full):
+            for r in (2, 9, 65):
+                x, y = tree(kinds[k % 2], r, 600 + 2 * k), tree(kinds[(k + 1) % 2], c, 601 + 2 * k)
+                check(ctx, x, y, model)
+                assert set(ctx.class_profile()) == {row_class(waves, cpl)}
+                k += 1
