@@ -133,6 +133,24 @@ def test_settings_hold_for_every_class(shim, max_cpl, min_waves, wide_cols):
     assert max_cpl < 8 or min_waves > 1 or xted.CLASS_SWEEP in seen
 
 
+def test_deep_tables_of_one_workgroup_stay_in_it(shim):
+    """Blocks of one wave take no table of up to 2048 columns that one
+    workgroup holds: their rows wait for each other longer than they save."""
+    one_wave = {FIRST_XL + 4, FIRST_XL + 5}
+    taken = {xted.CLASS_SHARED: 0, "on chip": 0}
+    for t in itertools.product((300, 500, 900), (350, 500, 1000, 1500, 2000, 2048), (20, 60, 100),
+                               (100, 150, 200, 250), (300, 450), (1 << 18, 1 << 22)):
+        if t[3] >= min(t[4], t[1] // 2) or t[4] > t[1] or t[0] > t[1] or t[2] >= t[0] // 2:
+            continue
+        if shim.scan_need(t[2], t[4], t[3], 1) > LDS_MAX:
+            continue
+        cls, _ = classify(shim, t, (10 * 1024, 16, 1, 1 << 30, 1))
+        assert cls not in one_wave, t
+        taken[xted.CLASS_SHARED] += cls == xted.CLASS_SHARED
+        taken["on chip"] += cls <= 25
+    assert all(taken.values())
+
+
 def test_every_table_that_fits_lds_has_a_form(shim):
     """Under any settings: a table of up to 8192 columns whose slot rows fit
     one workgroup is taken."""

@@ -398,11 +398,18 @@ XTED_HD inline int table_class(int a, int b, int kd_r, int kd_c, int leaves_c, b
     return form < 0 ? kClassXL : kFirstXLClass + form;
   };
   // Tall tables go in blocks where they are wider than one, and where LDS
-  // leaves them more columns per lane.
+  // leaves them more columns per lane; in blocks of one wave, the forms for
+  // deep trees, only above what 4 waves sharing their slot rows hold. (Pairs of
+  // trees nested about 250 deep, ms with such blocks for narrower tables too
+  // against one workgroup: 500 x 500 nodes 82 against 33, 1000 x 1000 150
+  // against 83, 2000 x 2000 321 against 217. One of 3000 x 3000 nodes, 190
+  // deep, above: 214 with blocks, 277 with 8 waves sharing slot rows.)
   if (tall && rule.blocks && rows > kTallBlockRows && rows > rule.xl_seq_rows &&
       (cols > xl_bw(first_tall) || cols > 64 * tall * (1 << wi))) {
     const int cls = blocked(first), k = cls - kFirstXLClass;
-    if (cls != kClassXL && (cols + xl_bw(k) - 1) / xl_bw(k) * xl_waves(k) >= least) return cls;
+    if (cls != kClassXL && (xl_waves(k) > 1 || cols > shared_cols(0)) &&
+        (cols + xl_bw(k) - 1) / xl_bw(k) * xl_waves(k) >= least)
+      return cls;
   }
   *need = scan_lds_need(slots, leaves_c, kd_c, 1 << wi);
   if (*need > rule.lds_max && lds_need <= rule.lds_max) {
