@@ -212,7 +212,9 @@ int xted_set_batch_groups(xted_context* ctx, int32_t groups, int32_t split_min);
 /* Where each pair's levels sit among the batch's levels: 0 starts every pair
  * at level 0, as the reference's single pair does
  * (X-TED_GPU/parallel_X_TED.cu:214-220); 1 (the default) ends every pair at
- * the batch's last level; 2 places it midway. A pair's own levels keep their order
+ * the batch's last level in batches of more than two pairs of enough cells, and
+ * is as 0 in the others, where that costs more launches than it saves; 2 places
+ * every pair midway. A pair's own levels keep their order
  * (level = depth_x + depth_y + offset), so results do not depend on it; the
  * offsets move the tables of shallow pairs into the levels whose time is set
  * by the few large tables of the deepest pairs. */

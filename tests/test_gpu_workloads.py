@@ -205,3 +205,29 @@ def test_serving_pool_10000_every_result():
     bad = np.flatnonzero(served != gold["dist"])
     assert len(bad) == 0, f"{len(bad)} served distances differ, first queries {bad[:8].tolist()}"
     assert (served[largest] == gold["dist"][largest]).all()
+
+
+def test_default_placement_adds_no_launches_where_pairs_are_small():
+    """Pairs end on one last level, with more launches, only in batches of
+    several pairs of enough cells (more of them where launches go one by one)."""
+    def launches(ctx, xs, ys, align):
+        if align is not None:
+            ctx.set_level_align(align)
+        d, _, st = ctx.batch(xs, ys)
+        return st.launches, d
+
+    kinds = (xted.GEN_DEEP, xted.GEN_SHALLOW)
+    for pairs, lo, hi, ends_together in ((2, 100, 600, False), (600, 10, 60, False),
+                                         (64, 50, 300, True)):
+        rng = np.random.default_rng(pairs)
+        trees = [xted.generate(kinds[i % 2], int(rng.integers(lo, hi + 1)), 20,
+                               xted.derive_seed(9606, i)) for i in range(2 * pairs)]
+        for graphs in (True, False):
+            with xted.Context(0) as ctx:
+                ctx.set_graphs(graphs)
+                ids = ctx.pool_add(trees)
+                xs, ys = ids[0::2].copy(), ids[1::2].copy()
+                default, d = launches(ctx, xs, ys, None)
+                from_zero, d0 = launches(ctx, xs, ys, 0)
+                assert np.array_equal(d, d0)
+                assert (default > from_zero) == (ends_together and graphs), (pairs, graphs)

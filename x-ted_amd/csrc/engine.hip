@@ -473,6 +473,21 @@ hipStream_t Context::lane_stream(int lane) const {
   return s[0];
 }
 
+// The placement of a batch's pairs among its levels (level_align). Ending all
+// pairs on the last level shortens the levels that the deepest pairs' large
+// tables hold up, and adds launches, a few us each (singly: one by one, without
+// a graph): it pays for more than two pairs of enough cells. ms with pairs from
+// level 0 / ending together, in a graph: 2 pairs of 100-1000 nodes 4.13 / 4.24,
+// 8 of them 6.02 / 4.61; 1000 pairs of 10-60 nodes (9e3 cells a pair) 0.35 /
+// 0.38, 8000 of 20-60 (1.2e4) 0.77 / 0.83, 100 of 20-150 (1e5) 0.70 / 0.62,
+// 512 of 50-300 (8e5) 2.65 / 1.90, 512 of 100-1000 (2e7) 20.4 / 17.0. One by one:
+// 100 of 20-150 1.05 / 1.20, 40 of 100-600 (5e6) 6.16 / 6.39, 8 of 100-1000
+// (1.7e7) 7.63 / 7.24, 16 of 1000-3000 (4e8) 80.9 / 77.8.
+int32_t Context::placement(int32_t npairs, int64_t cells, bool singly) const {
+  if (level_align != 1) return level_align;
+  return npairs > 2 && cells / npairs >= (singly ? 8000000 : 30000) ? 1 : 0;
+}
+
 int Context::plan(Group& g, int32_t npairs, const int32_t* xs, const int32_t* ys, int lane,
                   int64_t words_limit) {
   BatchStats& st = g.st;
@@ -553,10 +568,11 @@ int Context::plan(Group& g, int32_t npairs, const int32_t* xs, const int32_t* ys
   g.td_bytes = (int64_t)sizeof(td_t) * td_total;
   const int nb = nlevels * kNumClasses * kBands;
   g.loff.assign(npairs, 0);
-  if (level_align == 1 || level_align == 2) {
+  const int32_t align = placement(npairs, st.cells, !use_graphs);
+  if (align) {
     for (int32_t i = 0; i < npairs; ++i) {
       const int32_t spare = nlevels - (meta_[xs[i]].kdmax + meta_[ys[i]].kdmax + 1);
-      g.loff[i] = level_align == 1 ? spare : spare / 2;
+      g.loff[i] = align == 1 ? spare : spare / 2;
     }
   }
   // Levels that at most tail_pairs pairs reach use the latency rule.
@@ -583,7 +599,7 @@ int Context::plan(Group& g, int32_t npairs, const int32_t* xs, const int32_t* ys
   ST_TRY(g.dist.grow(sizeof(int32_t) * npairs, false, ps));
   ST_TRY(g.lines_d.grow(sizeof(int64_t) * (npairs + 1), false, ps));
   ST_TRY(g.leaf_d.grow((size_t)npairs, false, ps));
-  if (level_align) ST_TRY(g.loff_d.grow(sizeof(int32_t) * npairs, false, ps));
+  if (align) ST_TRY(g.loff_d.grow(sizeof(int32_t) * npairs, false, ps));
   HIP_TRY(hipMemcpyAsync(g.pairs.p, g.pm.data(), sizeof(PairMeta) * npairs,
                          hipMemcpyHostToDevice, ps));
   HIP_TRY(hipMemcpyAsync(g.blk.p, blk.data(), sizeof(int64_t) * (npairs + 1),
@@ -592,7 +608,7 @@ int Context::plan(Group& g, int32_t npairs, const int32_t* xs, const int32_t* ys
                          hipMemcpyHostToDevice, ps));
   HIP_TRY(hipMemcpyAsync(g.tail_lv.p, g.h_tail.data(), nlevels, hipMemcpyHostToDevice, ps));
   HIP_TRY(hipMemcpyAsync(g.leaf_d.p, leaf.data(), (size_t)npairs, hipMemcpyHostToDevice, ps));
-  if (level_align)
+  if (align)
     HIP_TRY(hipMemcpyAsync(g.loff_d.p, g.loff.data(), sizeof(int32_t) * npairs,
                            hipMemcpyHostToDevice, ps));
   for (hipEvent_t* e : {&g.ev_plan0, &g.ev_plan1, &g.ev_end})
@@ -617,7 +633,7 @@ int Context::plan(Group& g, int32_t npairs, const int32_t* xs, const int32_t* ys
   pa.pool = view();
   pa.pairs = g.pairs.as<PairMeta>();
   pa.blk_start = g.blk.as<int64_t>();
-  pa.level_off = level_align ? g.loff_d.as<int32_t>() : nullptr;
+  pa.level_off = align ? g.loff_d.as<int32_t>() : nullptr;
   pa.npairs = npairs;
   pa.nlevels = nlevels;
   pa.lchunk_tables = plan_chunk;

@@ -272,12 +272,10 @@ class Context {
   // launch with events.
   int32_t use_graphs = 1;
   // Where a pair's levels sit among the batch's: 0 = every pair starts at
-  // level 0, 1 = every pair ends at the batch's last level, 2 = midway. A
-  // pair's own levels keep their order, so each is a valid schedule; the
-  // choice moves shallow pairs' tables into levels whose time is set by the
-  // few large tables of the deepest pairs. In ms with 0, 1, 2: the 96-tree
-  // matrix 99.9, 89.3, 90; 128 pairs of 100-600 nodes 18.8, 17.2, 17.6; 1024
-  // pairs under a cost model 54.0, 50.3, 49.4.
+  // level 0, 1 = every pair ends at the batch's last level where that pays
+  // (placement), else as 0, 2 = midway. A pair's own levels keep their order, so
+  // each is a valid schedule; the choice moves shallow pairs' tables into levels
+  // whose time is set by the few large tables of the deepest pairs.
   int32_t level_align = kDefaultLevelAlign;
   // 1: the tables of a launch start largest first (size bands); 2: and the
   // tables that need more slot storage than light_lds take launches of
@@ -319,6 +317,7 @@ class Context {
   Group na_;                        // run_batch_noalloc's group, bound to na_arena_
   std::vector<void*> retired_;      // see retire_list()
   Arena na_arena_;                  // this device's fixed array (kNoAllocArray)
+  int32_t placement(int32_t npairs, int64_t cells, bool singly) const;
   int64_t noalloc_bytes(int32_t npairs, const int32_t* xs, const int32_t* ys, int32_t classes,
                         bool level_offsets) const;
   // Whether the leaf lines of pair (x, y) are written in closed form (the
