@@ -202,19 +202,24 @@ bool Server::tick(int lane) {
   if (L.active.empty()) return false;
   std::vector<Group*> gs;
   for (auto& a : L.active) gs.push_back(a.g.get());
-  // Streams 0 and 1 are the lanes' own. The heavy lane has stream 2 as well;
-  // the light lane has 2 and 3 while no heavy tick is in flight, and its own
-  // alone beside heavy ones: a tick joins all its streams and would wait for
-  // what a heavy tick has put on them, or on another stream of the same
-  // hardware queue (a process has 4, for the lanes' streams and the plan's).
+  // Streams 0 and 1 are the lanes' own. The heavy lane has stream 2 as well, and
+  // 3 while no light query is on the device; the light lane has 2 and 3 while no
+  // heavy tick is in flight, and its own alone beside heavy ones: a tick joins
+  // all its streams and would wait for what a heavy tick has put on them, or on
+  // another stream of the same hardware queue (a process has 4, for the lanes'
+  // streams and the plan's).
   // Latency of a light query beside a pair of 20,000 nodes, 8 of 5000, 120 of
-  // 2500, p50 ms: 1.1, 1.1, 1.1; with the second streams of both lanes lent to
+  // 2500, p50 ms: 1.3, 1.1, 1.1; with the second streams of both lanes lent to
   // the one that was alone 23, 17, 14, each lane keeping its own second one
   // 17, 9, 15. Bursts of 64 pairs of 50-5000 nodes, mean over six pools, ms:
-  // 135 to 140, 148 and 160; one stream a lane 228.
+  // 128, 148 and 160; with stream 3 left idle 136, always the heavy lane's 164,
+  // one stream a lane 228. p50 / p99 ms at 150 queries/s of the 10,000-tree
+  // pool: 4.9 / 403, lent to the one alone 5.4 / 403, 3 idle 4.3 / 480, always
+  // the heavy lane's 18 / 383.
   reap(lanes_[1]);
+  const bool light_idle = lanes_[0].active.empty();
   const bool heavy_idle = lanes_[1].active.empty() && lanes_[1].ticks.empty();
-  ctx_->lent_streams = lane == 1 ? 0x4u : heavy_idle ? 0xCu : 0u;
+  ctx_->lent_streams = lane == 1 ? (light_idle ? 0xCu : 0x4u) : heavy_idle ? 0xCu : 0u;
   const int st = ctx_->launch_levels(gs.data(), (int)gs.size(), nullptr, lane);
   ctx_->lent_streams = 0;
   hipEvent_t ev = nullptr;
