@@ -142,7 +142,7 @@ int xted_batch(xted_context* ctx, int32_t npairs, const int32_t* x_ids, const in
  * on each device it runs on until the process ends; the call makes no
  * hipMalloc / hipFree / pinned-host allocation and instantiates no graph
  * (its levels are launched one by one). Pairs whose buffers exceed the array
- * (8*m*n bytes of tables plus 72 bytes per planned keyroot-pair table, as in
+ * (4*m*n bytes of tables plus 72 bytes per planned keyroot-pair table, as in
  * xted_all_pairs) are refused with XTED_ERR_TOO_LARGE. Distances only. Calls
  * on one context are serialised; calls on different contexts of one device
  * share that device's array and must not overlap. */
@@ -154,10 +154,12 @@ int xted_batch_noalloc(xted_context* ctx, int32_t npairs, const int32_t* x_ids,
  * xted_pool_add). The reference's test() sizes a dimension x dimension
  * Distance matrix but fills only (0, 1) (X-TED_GPU/test_TED.cu:30-54). The
  * pairs run through the batched plan in chunks whose device bytes take at
- * most max_bytes of HBM (0: 16 GiB): a pair counts its TD and TD^T (8*m*n
+ * most max_bytes of HBM (0: 16 GiB): a pair counts its TD and TD^T (4*m*n
  * bytes) and its plan arrays (72 bytes per planned keyroot-pair table: the
  * tables of two non-leaf keyroots with unit costs, all K_x*K_y tables under
- * a cost model). With unit costs the matrix is
+ * a cost model). Tables that are split over several workgroups to be faster
+ * take more for what those hand each other, out of what the chunk's pairs leave
+ * of max_bytes; where that is too little they run in one workgroup each. With unit costs the matrix is
  * symmetric with a zero diagonal and only i < j is computed; under a cost
  * model every ordered pair, the diagonal included, is. The context's pool
  * is used as scratch (cleared first). stats sums the chunks. */
@@ -242,8 +244,8 @@ int xted_set_light_lds(xted_context* ctx, int32_t bytes_per_wave);
  * thread per cell anti-diagonal (X-TED_GPU/parallel_X_TED.cu:883-1131).
  * Results do not depend on it. A mask outside [0, 7]: XTED_ERR_INVALID_ARG. */
 int xted_set_tiny_forms(xted_context* ctx, int32_t mask);
-/* on = 1 (the default): the level launches of a batch without
- * column-blocked tables are captured once as a HIP graph and re-launched
+/* on = 1 (the default): the level launches of a batch are captured once as a
+ * HIP graph and re-launched
  * while a later batch plans to the same launches (same counts per level and
  * class, same buffers); 0 launches them one by one. Profiling launches them
  * one by one regardless. The reference launches every kernel directly
@@ -291,8 +293,11 @@ int xted_launch_profile(xted_context* ctx, int32_t i, int32_t* level, int32_t* c
 /* ---- continuous-batching server ---------------------------------------------------
  * No counterpart in the reference. A server thread drains submitted queries
  * over pool trees into device batches, admitting each by the HBM its TD and
- * TD^T tables (8*m*n bytes) and its plan arrays (72 bytes per planned
- * keyroot-pair table, as in xted_all_pairs) need against hbm_budget bytes. */
+ * TD^T tables (4*m*n bytes) and its plan arrays (72 bytes per planned
+ * keyroot-pair table) need against hbm_budget bytes; split tables take from
+ * what is left of it, as in xted_all_pairs. A pair whose smaller tree has at
+ * most 1024 nodes and whose tables have at most 96 levels never waits for the
+ * device work of larger ones. */
 typedef struct xted_server xted_server;
 typedef struct xted_result {
   uint64_t tag;         /* caller's tag from submit */

@@ -169,9 +169,14 @@ XTED_HD inline int xl_bw(int k) { return 64 * xl_waves(k) * xl_cpl(k); }  // 409
 // 256, 128, 64, 32 and 16 rows: 76.9, 75.1, 74.1, 73.7, 74.0.
 constexpr int32_t kXLSeqRows = 32;  // default of ClassRule::xl_seq_rows
 // A table that fits one workgroup goes in blocks for being tall only above
-// this: filling the pipeline of blocks takes about 16 rows and 3 us a block
-// (tables of up to 237 rows and 4999 columns, ms a pair: 12.8 in one
-// workgroup, 15.1 in blocks).
+// this: filling the pipeline of blocks takes about 16 rows and 3 us a block.
+// Device time in ms of deep pairs of 5000 columns with 100, 237, 300, 400, 600,
+// 1000, 2000 rows: in one workgroup 6.2, 12.4, 14.4, 17.7, 33.2, 58, 102; in
+// blocks from 33 rows on 9.4, 14.2, 15.8, 18.5, 25.9, 39, 75. Of 1500 columns,
+// two blocks: 2.0, 3.4, 3.8, 4.6, 7.2, 11.8, 23.4 and 2.3, 3.9, 4.2, 5.1, 8.0,
+// 12.8, 23.6. Pairs of wide trees and of random ones lie alike. The lines cross
+// at some 450 rows of 5000 columns and 2000 of 1500; with 256 no shape loses more
+// than 15%.
 constexpr int32_t kTallBlockRows = 256;
 constexpr int kFirstSeqXLForm = 2;
 // Far values a block takes from earlier blocks are indexed by the nesting
@@ -257,6 +262,11 @@ constexpr int32_t kTallCols = 256;
 constexpr int64_t kTall2Cells = 120000;
 constexpr int64_t kTall4Cells = 3000000;
 constexpr int kTallRows = 64;
+// A wide table that is at most this part of its level's cells is swept by one
+// wave: the 20,000-node pair took, with shares of 1/64, 1/256, 1/1024, 1/8192 and
+// no table swept, 91, 92, 88, 105 and 139 ms. Its edges and slot rows take at
+// most kSweepLds, so that 8 such waves share a compute unit (10, 20, 40 and 80
+// KiB: 66 ms each, and the matrix of 96 trees 92; few tables come near).
 constexpr int64_t kSweepShare = 1024;
 constexpr int kSweepLds = 20 * 1024;
 constexpr int kTall2Form = 2, kTall4Form = 1;

@@ -182,7 +182,7 @@ class Context {
   int64_t whole_tree_cost(const int32_t* labels, int32_t n, bool del) const;
   int32_t pool_size() const { return (int32_t)meta_.size(); }
   // Device bytes a batch holds for pair (x, y) of the pool: its TD and TD^T
-  // (8*m*n plus padding) and its plan arrays, a task word and a 64-byte
+  // (4*m*n plus padding) and its plan arrays, a task word and a 64-byte
   // descriptor per planned keyroot-pair table (tables of two non-leaf
   // keyroots with unit costs, every table under a cost model). Both ids
   // must be valid; the caller holds mutex().

@@ -327,13 +327,19 @@ __device__ __forceinline__ int64_t xl_words(const XLGeom& g) {
 // ---------------------------------------------------------------------------
 // Row scan with shared slot rows: one table per workgroup of W waves, kC = 8
 // columns per lane, for tables whose column keyroot is so deep that the
-// imports of several waves do not fit LDS (scan.hip). Every wave reads and
-// writes one set of slot rows and takes its scan carry from the totals of the
-// waves before it, with a barrier per row. Columns are counted from jmax:
-// t = jmax-1-j, lane l of wave w owning t in [w*512 + 8l, w*512 + 8l + 8).
+// imports of several waves do not fit LDS (scan.hip) and that are not split
+// over workgroups for being tall. Every wave reads and writes one set of slot
+// rows and takes its scan carry from the totals of the waves before it, with a
+// barrier per row. Columns are counted from jmax: t = jmax-1-j, lane l of wave w
+// owning t in [w*512 + 8l, w*512 + 8l + 8).
 // What bounds it: the barrier, at which all waves wait for the slowest one's
-// row (8 waves 0.5 us a row; a burst of 64 pairs of 500-5000 nodes with 21
-// such tables 129.8 ms, with them as column blocks 126.0).
+// row (8 waves 0.5 us a row). Against blocks of one wave, which is what such
+// tables would take instead: 4 waves are faster (the tall tables of 1025 to 2048
+// columns of a pair of 2000-node trees nested 250 deep, 217 ms against 321 with
+// blocks), 8 waves slower (2049 to 4096 columns, 3000-node trees nested 190
+// deep, 277 against 214; a burst of 64 pairs of 500-5000 nodes with 21 such
+// tables 129.8 against 126.0). Blocks need words in device memory, so short
+// tables, whose time is not their level's, keep to shared slot rows.
 // ---------------------------------------------------------------------------
 template <int W, bool kCost>
 __global__ __launch_bounds__(64 * W) void rowscan_kernel(DPArgs A) {

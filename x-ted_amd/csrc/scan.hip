@@ -94,8 +94,9 @@ __device__ __forceinline__ void lds_order() {
 // itself whether it is there. Carries are read a line (16 rows) at a time with
 // compare-exchanges against a value no word holds, which return the current
 // word; once a line is complete so are the imports of its rows, as a rule,
-// and these are read with plain loads, whose lines no XCD has read before. A
-// stale word all the same (its epoch is old) is read again atomically.
+// and these are read with plain loads. A stale word (levels share the memory,
+// so a line of an earlier launch may still be in an L2; its epoch is old) is
+// read again atomically.
 // Workgroups take (table, block) from a ticket counter in start order, so a
 // block only waits on blocks that are already running. Waits are bounded:
 // after kXLWaitTicks of the 100 MHz wall clock a wave raises the abort flag
